@@ -350,6 +350,26 @@ __global__ void k_batch_reset(int *ctl, int base, int step) {
     }
 }
 
+// The receptor spectrum rec[kx][ky][kz] as the correlation pass reads it: per (kx, ky), each
+// run of 16 columns kz <= nf/2 followed by the 16 values at (-kx, -ky, -kz), 2 Hp values a row
+// (zero past nf/2).
+__global__ void __launch_bounds__(NT) k_rec_pairs(const float2 *__restrict__ rec, float2 *__restrict__ recp, int nf,
+                                                  int Hp) {
+    const int q = blockIdx.x * NT + threadIdx.x, kx = blockIdx.y;
+    if (q >= nf * 2 * Hp) return;
+    const int ky = q / (2 * Hp), p = q - ky * 2 * Hp, kz = (p >> 5) * 16 + (p & 15);
+    float2 v = make_float2(0.f, 0.f);
+    if (kz <= nf / 2) {
+        if (p & 16) {
+            const int nx = kx ? nf - kx : 0, ny = ky ? nf - ky : 0, nz = kz ? nf - kz : 0;
+            v = rec[((size_t)nx * nf + ny) * nf + nz];
+        } else {
+            v = rec[((size_t)kx * nf + ky) * nf + kz];
+        }
+    }
+    recp[(size_t)kx * nf * 2 * Hp + q] = v;
+}
+
 __global__ void k_iota(int *p, int first, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = first + i;
@@ -454,6 +474,7 @@ struct mdk_ctx {
     int inv_variant = 2;      // MDK_INV_VARIANT: fused-inverse variant (tuning)
     int fwd_variant = 0;      // MDK_FWD_VARIANT: 0 fused forward z + y, prefetching (nf = 256: over half planes), 1 separate passes, 2 fused, not prefetching
     float2 *d_rec = nullptr;
+    float2 *d_recp = nullptr;  // d_rec as pairs of columns, for the specialised pipeline (k_rec_pairs)
     bool have_rec = false, have_lig = false;
     // ligand
     float *d_xyz = nullptr, *d_rc2 = nullptr, *d_rs2 = nullptr, *d_charge = nullptr, *d_gc = nullptr;
@@ -532,7 +553,7 @@ int run_fft_pipeline(mdk_ctx *c, BatchSlot &S, int B, float *smap_dev, hipEvent_
         a.a1 = S.d_a1;
         a.a2 = S.d_a2;
         a.cc = S.d_cc;
-        a.rec = c->d_rec;
+        a.rec = c->d_recp;
         a.cand = S.d_cand;
         a.smap = smap_dev;
         a.tw4 = c->d_tw4;
@@ -728,6 +749,7 @@ int mdk_create(int device, int nf, int ng, int na, int t, int max_batch, mdk_ctx
             return bail(fail("mdk_create: stream creation failed"));
     c->stream = c->slot[0].stream;
     const size_t nf3 = (size_t)nf * nf * nf, ng3 = (size_t)ng * ng * ng, B = max_batch;
+    if (pipe_available(nf) && dmalloc(&c->d_recp, (size_t)nf * nf * 2 * c->Hp)) return bail(1);
     if (dmalloc(&c->d_tw, tw.size()) || dmalloc(&c->d_rec, nf3) || dmalloc(&c->d_xyz, 3 * (size_t)na) ||
         dmalloc(&c->d_rc2, na) || dmalloc(&c->d_rs2, na) || dmalloc(&c->d_charge, na) || dmalloc(&c->d_gc, ng) ||
         dmalloc(&c->d_brot, 9 * B) || dmalloc(&c->d_bid, B) || dmalloc(&c->d_recgrid, ng3) ||
@@ -799,7 +821,7 @@ int mdk_destroy(mdk_ctx *c) {
     (void)hipSetDevice(c->device);
     for (int k = 0; k < mdk_ctx::kMaxSlots; k++)
         if (c->slot[k].stream) (void)hipStreamSynchronize(c->slot[k].stream);
-    void *ptrs[] = {c->d_tw, c->d_tw4, c->d_rec, c->d_xyz, c->d_rc2, c->d_rs2, c->d_charge, c->d_gc, c->d_rot,
+    void *ptrs[] = {c->d_tw, c->d_tw4, c->d_rec, c->d_recp, c->d_xyz, c->d_rc2, c->d_rs2, c->d_charge, c->d_gc, c->d_rot,
                     c->d_rotid, c->d_brot, c->d_bid, c->d_results, c->d_topn_scratch, c->d_topn_out,
                     c->d_recgrid, c->d_wshape, c->d_bt, c->d_gout, c->d_gpart, c->d_rpsc, c->d_btrans, c->d_dsum};
     for (void *p : ptrs)
@@ -841,6 +863,14 @@ int staging(void **buf, size_t &cap, size_t bytes, hipEvent_t &ev) {
     return 0;
 }
 
+// d_recp from d_rec, on the context's stream
+int pair_receptor(mdk_ctx *c) {
+    if (!c->d_recp) return 0;
+    k_rec_pairs<<<dim3((c->nf * 2 * c->Hp + NT - 1) / NT, c->nf), NT, 0, c->stream>>>(c->d_rec, c->d_recp, c->nf, c->Hp);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
 // receptor spectrum from the receptor grids already in d_recgrid (src/fft_process.cpp:212-303);
 // `wait`: return after it is done, else with it queued on the context's stream
 int receptor_transform(mdk_ctx *c, bool wait = true) {
@@ -852,6 +882,7 @@ int receptor_transform(mdk_ctx *c, bool wait = true) {
     k_fwd_y<<<dim3((nf + WY - 1) / WY, ng, 1), NT, lds_bytes(c, WY), c->stream>>>(c->slot[0].d_a1, c->slot[0].d_a2, c->plan, c->d_tw, ng, nd);
     k_fwd_x_plain<<<dim3((nf + WY - 1) / WY, nf), NT, lds_bytes(c, WY), c->stream>>>(c->slot[0].d_a2, c->d_rec, c->plan, c->d_tw, ng, nd);
     HIPCHK(hipGetLastError());
+    if (pair_receptor(c)) return 1;
     if (wait) HIPCHK(hipStreamSynchronize(c->stream));
     c->have_rec = true;
     c->have_recgrid = true;
@@ -938,6 +969,8 @@ int mdk_set_receptor_spectrum(mdk_ctx *c, const float *re, const float *im) {
     std::vector<float2> h(nf3);
     for (size_t i = 0; i < nf3; i++) h[i] = make_float2(re[i], im[i]);
     HIPCHK(hipMemcpy(c->d_rec, h.data(), sizeof(float2) * nf3, hipMemcpyHostToDevice));
+    if (pair_receptor(c)) return 1;
+    HIPCHK(hipStreamSynchronize(c->stream));
     c->have_rec = true;
     c->have_recgrid = false;  // no real-space grids behind this spectrum
     return 0;

@@ -272,7 +272,7 @@ struct PipeArgs {
     float nf3f;
     VoxGrid vox;        // voxelized ligands of the batch
     float2 *a1, *a2, *cc;
-    const float2 *rec;
+    const float2 *rec;  // receptor spectrum as pairs of columns (k_rec_pairs)
     Cand *cand;
     float *smap;
     const float2 *tw4;  // exp(-2 pi i m / nf), m < nf

@@ -39,7 +39,7 @@ hipError_t launch_decoy_coords(const float *xyz, int na, const float *pre, const
 size_t receptor_voxel_scratch_bytes(int ng);
 hipError_t launch_receptor_voxel(const float *xyz, const float *radius, const float *charge, const float *ace,
                                  const float *gc, int na, int ng, float gw, float aceratio, float rec_core, float eratio,
-                                 float gc0, float gc1, void *scratch, float2 *out, hipStream_t s);
+                                 float gc0, float gc1, bool regular, void *scratch, float2 *out, hipStream_t s);
 
 // off-grid scores (mdk_grad.hip)
 size_t grad_scratch_doubles(int max_batch);
@@ -514,6 +514,8 @@ struct mdk_ctx {
     float2 *h_rstage = nullptr;
     float *h_lstage = nullptr;
     size_t h_rstage_n = 0, h_lstage_n = 0;  // bytes
+    char *d_recwork = nullptr;  // atoms and bit masks of mdk_set_receptor_atoms, grown to the largest receptor
+    size_t recwork_n = 0;       // bytes
     hipEvent_t ev_rstage = nullptr, ev_lstage = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     std::vector<hipEvent_t> tev;  // mdk_dock_range_timed: MDK_NSTAGE + 1 events per batch
@@ -823,7 +825,7 @@ int mdk_destroy(mdk_ctx *c) {
         if (c->slot[k].stream) (void)hipStreamSynchronize(c->slot[k].stream);
     void *ptrs[] = {c->d_tw, c->d_tw4, c->d_rec, c->d_recp, c->d_xyz, c->d_rc2, c->d_rs2, c->d_charge, c->d_gc, c->d_rot,
                     c->d_rotid, c->d_brot, c->d_bid, c->d_results, c->d_topn_scratch, c->d_topn_out,
-                    c->d_recgrid, c->d_wshape, c->d_bt, c->d_gout, c->d_gpart, c->d_rpsc, c->d_btrans, c->d_dsum};
+                    c->d_recgrid, c->d_wshape, c->d_bt, c->d_gout, c->d_gpart, c->d_rpsc, c->d_btrans, c->d_dsum, c->d_recwork};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (c->h_topn) (void)hipHostFree(c->h_topn);
@@ -912,37 +914,39 @@ int mdk_set_receptor_atoms(mdk_ctx *c, int na, const float *xyz, const float *ra
         return fail("mdk_set_receptor_atoms: invalid argument");
     if (!(gw > 0.0f) || c->ng < 2) return fail("mdk_set_receptor_atoms: invalid grid");
     HIPCHK(hipSetDevice(c->device));
-    if (wait_slots(c)) return 1;
     const int ng = c->ng;
-    const size_t n = na > 0 ? (size_t)na : 1;
-    float *d_xyz = nullptr, *d_rad = nullptr, *d_chg = nullptr, *d_ace = nullptr, *d_gc = nullptr;
-    void *scratch = nullptr;
-    int rc = 0;
-    if (hipMalloc(&d_xyz, sizeof(float) * 3 * n) != hipSuccess || hipMalloc(&d_rad, sizeof(float) * n) != hipSuccess ||
-        hipMalloc(&d_chg, sizeof(float) * n) != hipSuccess || hipMalloc(&d_ace, sizeof(float) * n) != hipSuccess ||
-        hipMalloc(&d_gc, sizeof(float) * ng) != hipSuccess ||
-        hipMalloc(&scratch, receptor_voxel_scratch_bytes(ng)) != hipSuccess)
-        rc = fail("mdk_set_receptor_atoms: out of device memory");
-    if (!rc && na > 0 &&
-        (hipMemcpy(d_xyz, xyz, sizeof(float) * 3 * na, hipMemcpyHostToDevice) != hipSuccess ||
-         hipMemcpy(d_rad, radius, sizeof(float) * na, hipMemcpyHostToDevice) != hipSuccess ||
-         hipMemcpy(d_chg, charge, sizeof(float) * na, hipMemcpyHostToDevice) != hipSuccess ||
-         hipMemcpy(d_ace, ace, sizeof(float) * na, hipMemcpyHostToDevice) != hipSuccess))
-        rc = fail("mdk_set_receptor_atoms: upload failed");
-    if (!rc && hipMemcpy(d_gc, grid_coord, sizeof(float) * ng, hipMemcpyHostToDevice) != hipSuccess)
-        rc = fail("mdk_set_receptor_atoms: upload failed");
-    if (!rc && launch_receptor_voxel(d_xyz, d_rad, d_chg, d_ace, d_gc, na, ng, gw, aceratio, rec_core, eratio,
-                                     grid_coord[0], ng > 1 ? grid_coord[1] : grid_coord[0], scratch, c->d_recgrid,
-                                     c->stream) != hipSuccess)
-        rc = fail("mdk_set_receptor_atoms: kernel launch failed");
-    if (!rc && hipStreamSynchronize(c->stream) != hipSuccess) rc = fail("mdk_set_receptor_atoms: voxelization failed");
-    (void)hipFree(d_xyz);
-    (void)hipFree(d_rad);
-    (void)hipFree(d_chg);
-    (void)hipFree(d_ace);
-    (void)hipFree(d_gc);
-    (void)hipFree(scratch);
-    if (rc) return rc;
+    // the atoms in one pinned block and one copy, into a device workspace that the context
+    // keeps; stream-ordered, as mdk_set_receptor (six allocations, their frees and five
+    // blocking copies a call took 0.3 ms)
+    const size_t n = (size_t)na, words = 6 * n + ng, bytes = sizeof(float) * words;
+    if (staging((void **)&c->h_lstage, c->h_lstage_n, bytes, c->ev_lstage)) return 1;
+    const size_t off = (bytes + 255) / 256 * 256, need = off + receptor_voxel_scratch_bytes(ng);
+    if (need > c->recwork_n) {
+        if (c->d_recwork) {
+            HIPCHK(hipStreamSynchronize(c->stream));
+            HIPCHK(hipFree(c->d_recwork));
+        }
+        c->d_recwork = nullptr;
+        c->recwork_n = 0;
+        HIPCHK(hipMalloc((void **)&c->d_recwork, need));
+        c->recwork_n = need;
+    }
+    float *h = c->h_lstage;
+    if (na > 0) {
+        std::memcpy(h, xyz, sizeof(float) * 3 * n);
+        std::memcpy(h + 3 * n, radius, sizeof(float) * n);
+        std::memcpy(h + 4 * n, charge, sizeof(float) * n);
+        std::memcpy(h + 5 * n, ace, sizeof(float) * n);
+    }
+    std::memcpy(h + 6 * n, grid_coord, sizeof(float) * ng);
+    bool regular = true;  // the coordinates are the voxel centres
+    for (int i = 0; i < ng; i++) regular = regular && std::fabs(grid_coord[i] - gw * (i + 0.5f - 0.5f * ng)) <= 0.25f * gw;
+    float *d = reinterpret_cast<float *>(c->d_recwork);
+    HIPCHK(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipEventRecord(c->ev_lstage, c->stream));
+    HIPCHK(launch_receptor_voxel(d, d + 3 * n, d + 4 * n, d + 5 * n, d + 6 * n, na, ng, gw, aceratio, rec_core, eratio,
+                                 grid_coord[0], ng > 1 ? grid_coord[1] : grid_coord[0], regular, c->d_recwork + off,
+                                 c->d_recgrid, c->stream));
     return receptor_transform(c);
 }
 
@@ -951,8 +955,9 @@ int mdk_get_receptor_grids(mdk_ctx *c, float *grid_r, float *grid_i) {
     if (!c->have_recgrid) return fail("mdk_get_receptor_grids: no receptor grids set");
     HIPCHK(hipSetDevice(c->device));
     const size_t ng3 = (size_t)c->ng * c->ng * c->ng;
-    std::vector<float2> h(ng3);
-    HIPCHK(hipMemcpyAsync(h.data(), c->d_recgrid, sizeof(float2) * ng3, hipMemcpyDeviceToHost, c->stream));
+    if (staging((void **)&c->h_rstage, c->h_rstage_n, sizeof(float2) * ng3, c->ev_rstage)) return 1;
+    const float2 *h = c->h_rstage;
+    HIPCHK(hipMemcpyAsync(c->h_rstage, c->d_recgrid, sizeof(float2) * ng3, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     for (size_t i = 0; i < ng3; i++) {
         grid_r[i] = h[i].x;

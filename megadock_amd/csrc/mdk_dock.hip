@@ -46,7 +46,7 @@ size_t grad_scratch_doubles(int max_batch);
 hipError_t launch_spec_eval(const float2 *Q, const float *t_dev, int B, int nf, int H, int Hp, double *part,
                             float *out_dev, hipStream_t s);
 hipError_t launch_companion(const LigandDev &lig, const float *wshape, const float2 *recgrid, const float *rot_dev,
-                            const float *t_dev, int B, int nf, double *part, float *out_dev, hipStream_t s);
+                            const float *t_dev, int B, int nf, float *out_dev, hipStream_t s);
 
 #define MDK_NSTAGE 7  // voxelize, fwd_z, fwd_y, x_corr, inv_y, inv_z_top, reduce
 
@@ -514,6 +514,11 @@ struct mdk_ctx {
     float2 *h_rstage = nullptr;
     float *h_lstage = nullptr;
     size_t h_rstage_n = 0, h_lstage_n = 0;  // bytes
+    float *h_pstage = nullptr;  // poses and results of mdk_score_companion, pinned and on the device
+    size_t h_pstage_n = 0;      // bytes
+    hipEvent_t ev_pstage = nullptr;
+    float *d_posework = nullptr;
+    size_t posework_n = 0;      // floats
     char *d_recwork = nullptr;  // atoms and bit masks of mdk_set_receptor_atoms, grown to the largest receptor
     size_t recwork_n = 0;       // bytes
     hipEvent_t ev_rstage = nullptr, ev_lstage = nullptr;
@@ -825,13 +830,15 @@ int mdk_destroy(mdk_ctx *c) {
         if (c->slot[k].stream) (void)hipStreamSynchronize(c->slot[k].stream);
     void *ptrs[] = {c->d_tw, c->d_tw4, c->d_rec, c->d_recp, c->d_xyz, c->d_rc2, c->d_rs2, c->d_charge, c->d_gc, c->d_rot,
                     c->d_rotid, c->d_brot, c->d_bid, c->d_results, c->d_topn_scratch, c->d_topn_out,
-                    c->d_recgrid, c->d_wshape, c->d_bt, c->d_gout, c->d_gpart, c->d_rpsc, c->d_btrans, c->d_dsum, c->d_recwork};
+                    c->d_recgrid, c->d_wshape, c->d_bt, c->d_gout, c->d_gpart, c->d_rpsc, c->d_btrans, c->d_dsum, c->d_recwork, c->d_posework};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (c->h_topn) (void)hipHostFree(c->h_topn);
     if (c->topn_done) (void)hipEventDestroy(c->topn_done);
     if (c->h_rstage) (void)hipHostFree(c->h_rstage);
     if (c->h_lstage) (void)hipHostFree(c->h_lstage);
+    if (c->h_pstage) (void)hipHostFree(c->h_pstage);
+    if (c->ev_pstage) (void)hipEventDestroy(c->ev_pstage);
     if (c->ev_rstage) (void)hipEventDestroy(c->ev_rstage);
     if (c->ev_lstage) (void)hipEventDestroy(c->ev_lstage);
     drop_graphs(c);
@@ -1434,17 +1441,32 @@ int mdk_score_companion(mdk_ctx *c, const float *rotcoef, const float *t, int B,
         return fail("mdk_score_companion: receptor grids (mdk_set_receptor) and ligand must be set first");
     if (B < 0) return fail("mdk_score_companion: negative batch size");
     HIPCHK(hipSetDevice(c->device));
-    for (int q0 = 0; q0 < B; q0 += c->max_batch) {  // in batches of the context's size, in order
-        const int nb = std::min(c->max_batch, B - q0);
-        HIPCHK(hipMemcpyAsync(c->d_brot, rotcoef + 9 * (size_t)q0, sizeof(float) * 9 * nb, hipMemcpyHostToDevice,
-                              c->stream));
-        HIPCHK(hipMemcpyAsync(c->d_bt, t + 3 * (size_t)q0, sizeof(float) * 3 * nb, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(launch_companion(c->lig, c->d_wshape, c->d_recgrid, c->d_brot, c->d_bt, nb, c->nf, c->d_gpart,
-                                c->d_gout, c->stream));
-        HIPCHK(hipMemcpyAsync(out + 7 * (size_t)q0, c->d_gout, sizeof(float) * 7 * nb, hipMemcpyDeviceToHost,
-                              c->stream));
+    // up to kPoses poses a launch: rotations and translations in one pinned block and one copy,
+    // the results in the block behind them
+    constexpr int kPoses = 65536;
+    const size_t cap = std::min(B, kPoses), words = (9 + 3 + 7) * cap;
+    if (cap && staging((void **)&c->h_pstage, c->h_pstage_n, sizeof(float) * words, c->ev_pstage)) return 1;
+    if (words > c->posework_n) {
+        if (c->d_posework) {
+            HIPCHK(hipStreamSynchronize(c->stream));
+            HIPCHK(hipFree(c->d_posework));
+        }
+        c->d_posework = nullptr;
+        c->posework_n = 0;
+        HIPCHK(hipMalloc((void **)&c->d_posework, sizeof(float) * words));
+        c->posework_n = words;
     }
-    HIPCHK(hipStreamSynchronize(c->stream));
+    for (int q0 = 0; q0 < B; q0 += kPoses) {
+        const size_t nb = std::min(kPoses, B - q0);
+        float *h = c->h_pstage, *d = c->d_posework;
+        std::memcpy(h, rotcoef + 9 * (size_t)q0, sizeof(float) * 9 * nb);
+        std::memcpy(h + 9 * nb, t + 3 * (size_t)q0, sizeof(float) * 3 * nb);
+        HIPCHK(hipMemcpyAsync(d, h, sizeof(float) * 12 * nb, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(launch_companion(c->lig, c->d_wshape, c->d_recgrid, d, d + 9 * nb, (int)nb, c->nf, d + 12 * nb, c->stream));
+        HIPCHK(hipMemcpyAsync(h + 12 * nb, d + 12 * nb, sizeof(float) * 7 * nb, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        std::memcpy(out + 7 * (size_t)q0, h + 12 * nb, sizeof(float) * 7 * nb);
+    }
     return 0;
 }
 

@@ -25,7 +25,6 @@
 namespace {
 
 constexpr int kSpecBlocks = 64;  // workgroups per rotation in the spectral evaluation
-constexpr int kCompBlocks = 8;   // workgroups per pose in the companion score
 
 __device__ __forceinline__ int signed_freq(int k, int nf) { return k < nf / 2 ? k : k - nf; }
 
@@ -128,11 +127,30 @@ __device__ __forceinline__ void trilinear(const float2 *__restrict__ rg, int ng,
     }
 }
 
-// part[b][blk][7] = (s, ds/dt'(3), ds/dw(3))
+// Sums v[0..K) over a workgroup of NT threads in a fixed order: within each wavefront by halving
+// strides, then over the wavefronts; the result is in thread 0.
+template <int K, int NT> __device__ __forceinline__ void block_sum(double *v) {
+    __shared__ double part[NT / 64][K];
+#pragma unroll
+    for (int a = 0; a < K; a++)
+        for (int h = 32; h >= 1; h >>= 1) v[a] += __shfl_down(v[a], h, 64);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int a = 0; a < K; a++) part[threadIdx.x >> 6][a] = v[a];
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int w = 1; w < NT / 64; w++)
+#pragma unroll
+            for (int a = 0; a < K; a++) v[a] += part[w][a];
+}
+
+// out[b][7] = (s, ds/dt'(3), ds/dw(3)), one workgroup a pose and one launch a call: with eight
+// workgroups a pose, their partial sums and a second kernel, in batches of the context's size,
+// 2000 poses of 2081 atoms took 16 times two copies in, two kernels (13 and 4 us) and a copy out
 __global__ void __launch_bounds__(256) k_companion(LigandDev L, const float *__restrict__ wshape,
                                                    const float2 *__restrict__ rg, const float *__restrict__ rot,
-                                                   const float *__restrict__ tq, int nf, double *part) {
-    const int b = blockIdx.y, tid = threadIdx.x;
+                                                   const float *__restrict__ tq, int nf, float *__restrict__ out) {
+    const int b = blockIdx.x, tid = threadIdx.x;
     float r[9];
     for (int q = 0; q < 9; q++) r[q] = rot[9 * b + q];
     float t3[3];
@@ -143,7 +161,7 @@ __global__ void __launch_bounds__(256) k_companion(LigandDev L, const float *__r
     const int ng = L.ng;
     const float gw = L.gw, h = 0.5f * ng - 0.5f;
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-    for (int a = blockIdx.x * 256 + tid; a < L.na; a += kCompBlocks * 256) {
+    for (int a = tid; a < L.na; a += 256) {
         const float x = L.xyz[3 * a] - L.cx, y = L.xyz[3 * a + 1] - L.cy, z = L.xyz[3 * a + 2] - L.cz;
         const float X = r[0] * x + r[1] * y + r[2] * z;
         const float Y = r[3] * x + r[4] * y + r[5] * z;
@@ -163,33 +181,14 @@ __global__ void __launch_bounds__(256) k_companion(LigandDev L, const float *__r
         acc[5] += Z * gx - X * gz;
         acc[6] += X * gy - Y * gx;
     }
-    __shared__ double red[7][256];
-    for (int a = 0; a < 7; a++) red[a][tid] = acc[a];
-    __syncthreads();
-    for (int hh = 128; hh >= 1; hh >>= 1) {
-        if (tid < hh)
-            for (int a = 0; a < 7; a++) red[a][tid] += red[a][tid + hh];
-        __syncthreads();
-    }
-    if (tid < 7) part[((size_t)b * kCompBlocks + blockIdx.x) * 7 + tid] = red[tid][0];
-}
-
-__global__ void k_comp_finish(const double *__restrict__ part, float *out, int B) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B) return;
-    for (int a = 0; a < 7; a++) {
-        double s = 0;
-        for (int k = 0; k < kCompBlocks; k++) s += part[((size_t)b * kCompBlocks + k) * 7 + a];
-        out[7 * b + a] = (float)s;
-    }
+    block_sum<7, 256>(acc);
+    if (tid == 0)
+        for (int a = 0; a < 7; a++) out[7 * (size_t)b + a] = (float)acc[a];
 }
 
 }  // namespace
 
-size_t grad_scratch_doubles(int max_batch) {
-    const int per = kSpecBlocks * 4 > kCompBlocks * 7 ? kSpecBlocks * 4 : kCompBlocks * 7;
-    return (size_t)max_batch * per;
-}
+size_t grad_scratch_doubles(int max_batch) { return (size_t)max_batch * kSpecBlocks * 4; }
 
 hipError_t launch_spec_eval(const float2 *Q, const float *t_dev, int B, int nf, int H, int Hp, double *part,
                             float *out_dev, hipStream_t s) {
@@ -199,8 +198,7 @@ hipError_t launch_spec_eval(const float2 *Q, const float *t_dev, int B, int nf, 
 }
 
 hipError_t launch_companion(const LigandDev &lig, const float *wshape, const float2 *recgrid, const float *rot_dev,
-                            const float *t_dev, int B, int nf, double *part, float *out_dev, hipStream_t s) {
-    k_companion<<<dim3(kCompBlocks, B), 256, 0, s>>>(lig, wshape, recgrid, rot_dev, t_dev, nf, part);
-    k_comp_finish<<<(B + 63) / 64, 64, 0, s>>>(part, out_dev, B);
+                            const float *t_dev, int B, int nf, float *out_dev, hipStream_t s) {
+    k_companion<<<B, 256, 0, s>>>(lig, wshape, recgrid, rot_dev, t_dev, nf, out_dev);
     return hipGetLastError();
 }

@@ -104,15 +104,28 @@ __global__ void k_spec_finish(const double *__restrict__ part, float *out, int B
 // coordinate u; corners outside the grid count as 0
 __device__ __forceinline__ void trilinear(const float2 *__restrict__ rg, int ng, float ux, float uy, float uz,
                                           float2 &val, float2 &dx, float2 &dy, float2 &dz) {
+    // a position with no corner in the grid (or not a number) counts as one just outside it
+    const float hi = (float)ng + 1.0f;
+    if (!(ux > -2.0f && ux < hi && uy > -2.0f && uy < hi && uz > -2.0f && uz < hi)) ux = uy = uz = -2.0f;
     const float fx0 = floorf(ux), fy0 = floorf(uy), fz0 = floorf(uz);
     const int i0 = (int)fx0, j0 = (int)fy0, k0 = (int)fz0;
     const float fx = ux - fx0, fy = uy - fy0, fz = uz - fz0;
     val = dx = dy = dz = make_float2(0.f, 0.f);
+    // the corners' loads are issued together (a corner outside the grid loads a voxel inside and
+    // counts as 0); with a branch around each, they came one after another
+    float2 corner[8];
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        const int i = i0 + (c >> 2), j = j0 + ((c >> 1) & 1), k = k0 + (c & 1);
+        const bool in = i >= 0 && i < ng && j >= 0 && j < ng && k >= 0 && k < ng;
+        const int at = in ? (i * ng + j) * ng + k : 0;
+        const float2 g = rg[at];
+        corner[c] = in ? g : make_float2(0.f, 0.f);
+    }
+#pragma unroll
     for (int c = 0; c < 8; c++) {
         const int di = c >> 2, dj = (c >> 1) & 1, dk = c & 1;
-        const int i = i0 + di, j = j0 + dj, k = k0 + dk;
-        if (i < 0 || i >= ng || j < 0 || j >= ng || k < 0 || k >= ng) continue;
-        const float2 g = rg[((size_t)i * ng + j) * ng + k];
+        const float2 g = corner[c];
         const float wx = di ? fx : 1.f - fx, wy = dj ? fy : 1.f - fy, wz = dk ? fz : 1.f - fz;
         const float sx = di ? 1.f : -1.f, sy = dj ? 1.f : -1.f, sz = dk ? 1.f : -1.f;
         const float w = wx * wy * wz, ax = sx * wy * wz, ay = wx * sy * wz, az = wx * wy * sz;

@@ -42,9 +42,8 @@ hipError_t launch_receptor_voxel(const float *xyz, const float *radius, const fl
                                  float gc0, float gc1, bool regular, void *scratch, float2 *out, hipStream_t s);
 
 // off-grid scores (mdk_grad.hip)
-size_t grad_scratch_doubles(int max_batch);
-hipError_t launch_spec_eval(const float2 *Q, const float *t_dev, int B, int nf, int H, int Hp, double *part,
-                            float *out_dev, hipStream_t s);
+hipError_t launch_spec_phase(const float *t_dev, int B, int nf, float2 *ph, hipStream_t s);
+hipError_t launch_spec_finish(const double *part, int B, int n, int nf, float *out_dev, hipStream_t s);
 hipError_t launch_companion(const LigandDev &lig, const float *wshape, const float2 *recgrid, const float *rot_dev,
                             const float *t_dev, int B, int nf, float *out_dev, hipStream_t s);
 
@@ -495,9 +494,8 @@ struct mdk_ctx {
     // off-grid scores and gradients (mdk_grad.hip)
     float2 *d_recgrid = nullptr;  // receptor grids (grid_r, grid_i), ng^3, real space
     float *d_wshape = nullptr;    // companion shape weight per ligand atom
-    float *d_bt = nullptr;        // translations of a batch (max_batch * 3)
-    float *d_gout = nullptr;      // results of a batch (max_batch * 7)
-    double *d_gpart = nullptr;    // partial sums
+    float2 *d_gph = nullptr;      // spectral score: phases of a batch's poses (max_batch * 3 nf)
+    double *d_gpart = nullptr;    // and its partial sums (max_batch * spec_parts() * 4)
     float *d_rpsc = nullptr;      // receptor shape grid without the ACE term (mdk_score_detail), ng^3
     int *d_btrans = nullptr;      // grid translations of a batch (max_batch * 3)
     float *d_dsum = nullptr;      // detail sums of a batch (max_batch * 9)
@@ -514,7 +512,7 @@ struct mdk_ctx {
     float2 *h_rstage = nullptr;
     float *h_lstage = nullptr;
     size_t h_rstage_n = 0, h_lstage_n = 0;  // bytes
-    float *h_pstage = nullptr;  // poses and results of mdk_score_companion, pinned and on the device
+    float *h_pstage = nullptr;  // poses and results of the off-grid scores, pinned and on the device
     size_t h_pstage_n = 0;      // bytes
     hipEvent_t ev_pstage = nullptr;
     float *d_posework = nullptr;
@@ -528,6 +526,9 @@ struct mdk_ctx {
 
 namespace {
 
+// partial sums of the spectral score a pose: one per (ky, chunk of 16 kz)
+size_t spec_parts(const mdk_ctx *c) { return (size_t)c->nf * (c->Hp / 16); }
+
 size_t lds_bytes(const mdk_ctx *c, int lines) {
     return sizeof(float2) * ((size_t)c->plan.ntw + 2 * (size_t)c->nf * (lines + 1));
 }
@@ -540,11 +541,11 @@ VoxGrid vox_grid(const mdk_ctx *c, const BatchSlot &S) {
 // Run the forward ligand passes + correlation + inverse passes for B rotations that
 // launch_voxelize has voxelized; output top-t candidates (or the score map).
 // ev (optional): events recorded after each of the five FFT-side stages
-// spectrum_only: stop after the fold, leaving Q[b][kx][ky][kz] in S.d_cc (specialised sizes)
+// spec: end with the spectral score's partial sums in d_gpart, of the phases d_gph (specialised sizes)
 // from_lg: the ligand grids are already in S.d_lg (given by the host, mdk_dock_grid); the
 // generic kernels read them there
 int run_fft_pipeline(mdk_ctx *c, BatchSlot &S, int B, float *smap_dev, hipEvent_t *ev = nullptr,
-                     bool spectrum_only = false, bool from_lg = false) {
+                     bool spec = false, bool from_lg = false) {
     const int ng = c->ng, nf = c->nf, nd = c->nd;
     hipStream_t s = S.stream;
     if (c->use_pipe && !from_lg) {
@@ -570,7 +571,10 @@ int run_fft_pipeline(mdk_ctx *c, BatchSlot &S, int B, float *smap_dev, hipEvent_
         a.cu_count = c->cu_count;
         a.inv_variant = c->inv_variant;
         a.fwd_variant = c->fwd_variant;
-        a.spectrum_only = spectrum_only;
+        if (spec) {
+            a.spec_ph = c->d_gph;
+            a.spec_part = c->d_gpart;
+        }
         HIPCHK(pipe_run(nf, a));
         return 0;
     }
@@ -760,8 +764,8 @@ int mdk_create(int device, int nf, int ng, int na, int t, int max_batch, mdk_ctx
     if (dmalloc(&c->d_tw, tw.size()) || dmalloc(&c->d_rec, nf3) || dmalloc(&c->d_xyz, 3 * (size_t)na) ||
         dmalloc(&c->d_rc2, na) || dmalloc(&c->d_rs2, na) || dmalloc(&c->d_charge, na) || dmalloc(&c->d_gc, ng) ||
         dmalloc(&c->d_brot, 9 * B) || dmalloc(&c->d_bid, B) || dmalloc(&c->d_recgrid, ng3) ||
-        dmalloc(&c->d_wshape, na) || dmalloc(&c->d_bt, 3 * B) || dmalloc(&c->d_gout, 7 * B) ||
-        dmalloc(&c->d_gpart, grad_scratch_doubles((int)B)) || dmalloc(&c->d_rpsc, ng3) || dmalloc(&c->d_btrans, 3 * B) ||
+        dmalloc(&c->d_wshape, na) ||
+        (pipe_available(nf) && (dmalloc(&c->d_gph, B * 3 * nf) || dmalloc(&c->d_gpart, B * spec_parts(c) * 4))) || dmalloc(&c->d_rpsc, ng3) || dmalloc(&c->d_btrans, 3 * B) ||
         dmalloc(&c->d_dsum, 9 * B))
         return bail(1);
     for (int k = 0; k < c->nslots; k++) {
@@ -830,7 +834,7 @@ int mdk_destroy(mdk_ctx *c) {
         if (c->slot[k].stream) (void)hipStreamSynchronize(c->slot[k].stream);
     void *ptrs[] = {c->d_tw, c->d_tw4, c->d_rec, c->d_recp, c->d_xyz, c->d_rc2, c->d_rs2, c->d_charge, c->d_gc, c->d_rot,
                     c->d_rotid, c->d_brot, c->d_bid, c->d_results, c->d_topn_scratch, c->d_topn_out,
-                    c->d_recgrid, c->d_wshape, c->d_bt, c->d_gout, c->d_gpart, c->d_rpsc, c->d_btrans, c->d_dsum, c->d_recwork, c->d_posework};
+                    c->d_recgrid, c->d_wshape, c->d_gph, c->d_gpart, c->d_rpsc, c->d_btrans, c->d_dsum, c->d_recwork, c->d_posework};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (c->h_topn) (void)hipHostFree(c->h_topn);
@@ -1411,41 +1415,12 @@ int mdk_autotune(mdk_ctx *c, int first, int count, int *choice) {
     return 0;
 }
 
-int mdk_score_spectral(mdk_ctx *c, const float *rotcoef, const float *t, int B, float *out) {
-    if (!c || !rotcoef || !t || !out) return fail("mdk_score_spectral: null argument");
-    if (!c->have_rec || !c->have_lig) return fail("mdk_score_spectral: receptor and ligand must be set first");
-    if (B < 0) return fail("mdk_score_spectral: negative batch size");
-    if (!c->use_pipe)
-        return fail("mdk_score_spectral: needs an FFT size with specialised kernels (and MDK_FORCE_GENERIC unset)");
-    if (c->H > 192) return fail("mdk_score_spectral: nf above 382 (three kz per lane in the evaluation)");
-    HIPCHK(hipSetDevice(c->device));
-    BatchSlot &S = c->slot[0];
-    for (int q0 = 0; q0 < B; q0 += c->max_batch) {  // in batches of the context's size, in order
-        const int nb = std::min(c->max_batch, B - q0);
-        HIPCHK(hipMemcpyAsync(c->d_brot, rotcoef + 9 * (size_t)q0, sizeof(float) * 9 * nb, hipMemcpyHostToDevice,
-                              c->stream));
-        HIPCHK(hipMemcpyAsync(c->d_bt, t + 3 * (size_t)q0, sizeof(float) * 3 * nb, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(launch_voxelize(c->lig, c->d_brot, nb, S.vs, S.d_vidx, S.d_chg, c->stream));
-        if (run_fft_pipeline(c, S, nb, nullptr, nullptr, true)) return 1;
-        HIPCHK(launch_spec_eval(S.d_cc, c->d_bt, nb, c->nf, c->H, c->Hp, c->d_gpart, c->d_gout, c->stream));
-        HIPCHK(hipMemcpyAsync(out + 4 * (size_t)q0, c->d_gout, sizeof(float) * 4 * nb, hipMemcpyDeviceToHost,
-                              c->stream));
-    }
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return 0;
-}
-
-int mdk_score_companion(mdk_ctx *c, const float *rotcoef, const float *t, int B, float *out) {
-    if (!c || !rotcoef || !t || !out) return fail("mdk_score_companion: null argument");
-    if (!c->have_recgrid || !c->have_lig)
-        return fail("mdk_score_companion: receptor grids (mdk_set_receptor) and ligand must be set first");
-    if (B < 0) return fail("mdk_score_companion: negative batch size");
-    HIPCHK(hipSetDevice(c->device));
-    // up to kPoses poses a launch: rotations and translations in one pinned block and one copy,
-    // the results in the block behind them
-    constexpr int kPoses = 65536;
-    const size_t cap = std::min(B, kPoses), words = (9 + 3 + 7) * cap;
-    if (cap && staging((void **)&c->h_pstage, c->h_pstage_n, sizeof(float) * words, c->ev_pstage)) return 1;
+// Poses of the off-grid scores: rotations (9) and translations (3) of n poses in one pinned block
+// and one copy, k results a pose behind them and back the same way.
+constexpr int kPoses = 65536;  // poses a block
+int upload_poses(mdk_ctx *c, const float *rotcoef, const float *t, size_t n, int k) {
+    const size_t words = (12 + k) * n;
+    if (staging((void **)&c->h_pstage, c->h_pstage_n, sizeof(float) * words, c->ev_pstage)) return 1;
     if (words > c->posework_n) {
         if (c->d_posework) {
             HIPCHK(hipStreamSynchronize(c->stream));
@@ -1456,16 +1431,57 @@ int mdk_score_companion(mdk_ctx *c, const float *rotcoef, const float *t, int B,
         HIPCHK(hipMalloc((void **)&c->d_posework, sizeof(float) * words));
         c->posework_n = words;
     }
-    for (int q0 = 0; q0 < B; q0 += kPoses) {
-        const size_t nb = std::min(kPoses, B - q0);
-        float *h = c->h_pstage, *d = c->d_posework;
-        std::memcpy(h, rotcoef + 9 * (size_t)q0, sizeof(float) * 9 * nb);
-        std::memcpy(h + 9 * nb, t + 3 * (size_t)q0, sizeof(float) * 3 * nb);
-        HIPCHK(hipMemcpyAsync(d, h, sizeof(float) * 12 * nb, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(launch_companion(c->lig, c->d_wshape, c->d_recgrid, d, d + 9 * nb, (int)nb, c->nf, d + 12 * nb, c->stream));
-        HIPCHK(hipMemcpyAsync(h + 12 * nb, d + 12 * nb, sizeof(float) * 7 * nb, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-        std::memcpy(out + 7 * (size_t)q0, h + 12 * nb, sizeof(float) * 7 * nb);
+    std::memcpy(c->h_pstage, rotcoef, sizeof(float) * 9 * n);
+    std::memcpy(c->h_pstage + 9 * n, t, sizeof(float) * 3 * n);
+    HIPCHK(hipMemcpyAsync(c->d_posework, c->h_pstage, sizeof(float) * 12 * n, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipEventRecord(c->ev_pstage, c->stream));
+    return 0;
+}
+int download_poses(mdk_ctx *c, float *out, size_t n, int k) {
+    float *h = c->h_pstage + 12 * n;
+    HIPCHK(hipMemcpyAsync(h, c->d_posework + 12 * n, sizeof(float) * k * n, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    std::memcpy(out, h, sizeof(float) * k * n);
+    return 0;
+}
+
+int mdk_score_spectral(mdk_ctx *c, const float *rotcoef, const float *t, int B, float *out) {
+    if (!c || !rotcoef || !t || !out) return fail("mdk_score_spectral: null argument");
+    if (!c->have_rec || !c->have_lig) return fail("mdk_score_spectral: receptor and ligand must be set first");
+    if (B < 0) return fail("mdk_score_spectral: negative batch size");
+    if (!c->use_pipe)
+        return fail("mdk_score_spectral: needs an FFT size with specialised kernels (and MDK_FORCE_GENERIC unset)");
+    if (c->H > 192) return fail("mdk_score_spectral: nf above 382 (three kz per lane in the evaluation)");
+    HIPCHK(hipSetDevice(c->device));
+    BatchSlot &S = c->slot[0];
+    for (int p0 = 0; p0 < B; p0 += kPoses) {
+        const size_t np = std::min(kPoses, B - p0);
+        if (upload_poses(c, rotcoef + 9 * (size_t)p0, t + 3 * (size_t)p0, np, 4)) return 1;
+        float *d = c->d_posework, *d_t = d + 9 * np, *d_out = d + 12 * np;
+        for (size_t q0 = 0; q0 < np; q0 += c->max_batch) {  // in batches of the context's size, in order
+            const int nb = (int)std::min((size_t)c->max_batch, np - q0);
+            HIPCHK(launch_voxelize(c->lig, d + 9 * q0, nb, S.vs, S.d_vidx, S.d_chg, c->stream));
+            HIPCHK(launch_spec_phase(d_t + 3 * q0, nb, c->nf, c->d_gph, c->stream));
+            if (run_fft_pipeline(c, S, nb, nullptr, nullptr, true)) return 1;
+            HIPCHK(launch_spec_finish(c->d_gpart, nb, (int)spec_parts(c), c->nf, d_out + 4 * q0, c->stream));
+        }
+        if (download_poses(c, out + 4 * (size_t)p0, np, 4)) return 1;
+    }
+    return 0;
+}
+
+int mdk_score_companion(mdk_ctx *c, const float *rotcoef, const float *t, int B, float *out) {
+    if (!c || !rotcoef || !t || !out) return fail("mdk_score_companion: null argument");
+    if (!c->have_recgrid || !c->have_lig)
+        return fail("mdk_score_companion: receptor grids (mdk_set_receptor) and ligand must be set first");
+    if (B < 0) return fail("mdk_score_companion: negative batch size");
+    HIPCHK(hipSetDevice(c->device));
+    for (int p0 = 0; p0 < B; p0 += kPoses) {
+        const size_t np = std::min(kPoses, B - p0);
+        if (upload_poses(c, rotcoef + 9 * (size_t)p0, t + 3 * (size_t)p0, np, 7)) return 1;
+        float *d = c->d_posework;
+        HIPCHK(launch_companion(c->lig, c->d_wshape, c->d_recgrid, d, d + 9 * np, (int)np, c->nf, d + 12 * np, c->stream));
+        if (download_poses(c, out + 7 * (size_t)p0, np, 7)) return 1;
     }
     return 0;
 }

@@ -24,80 +24,17 @@
 
 namespace {
 
-constexpr int kSpecBlocks = 64;  // workgroups per rotation in the spectral evaluation
-
 __device__ __forceinline__ int signed_freq(int k, int nf) { return k < nf / 2 ? k : k - nf; }
 
-// partial sums part[b][blk][4] = (value, d/dtx, d/dty, d/dtz) before scaling
-__global__ void __launch_bounds__(256) k_spec_eval(const float2 *__restrict__ Q, const float *__restrict__ tq,
-                                                   double *part, int nf, int H, int Hp) {
-    extern __shared__ float2 ph[];  // phases e^{2 pi i k' t_a / nf}: [3][nf]
-    const int b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    for (int k = tid; k < nf; k += 256) {
-        const double f = 2.0 * M_PI * signed_freq(k, nf) / nf;
-        for (int a = 0; a < 3; a++) {
-            double sn, cs;
-            sincos(f * tq[3 * b + a], &sn, &cs);
-            ph[a * nf + k] = make_float2((float)cs, (float)sn);
-        }
+// phases e^{2 pi i k' t_a / nf} of pose b: ph[b][a][k]
+__global__ void __launch_bounds__(256) k_spec_phase(const float *__restrict__ tq, float2 *__restrict__ ph, int nf) {
+    const int b = blockIdx.x;
+    for (int q = threadIdx.x; q < 3 * nf; q += 256) {
+        const int a = q / nf, k = q - a * nf;
+        double sn, cs;
+        sincos(2.0 * M_PI * signed_freq(k, nf) / nf * tq[3 * b + a], &sn, &cs);
+        ph[(size_t)b * 3 * nf + q] = make_float2((float)cs, (float)sn);
     }
-    __syncthreads();
-    const float2 *q = Q + (size_t)b * nf * nf * Hp;
-    // lane owns kz = lane, lane + 64 and lane + 128 (< H; kz = 128 is the Nyquist plane of nf = 256)
-    constexpr int JZ = 3;
-    float2 ez[JZ];
-    float wz[JZ], kzs[JZ];
-    bool on[JZ];
-    for (int j = 0; j < JZ; j++) {
-        const int kz = lane + 64 * j;
-        on[j] = kz < H;
-        ez[j] = on[j] ? ph[2 * nf + kz] : make_float2(0.f, 0.f);
-        wz[j] = (kz == 0 || 2 * kz == nf) ? 1.0f : 2.0f;
-        kzs[j] = (float)signed_freq(kz, nf);
-    }
-    double v = 0.0, gx = 0.0, gy = 0.0, gz = 0.0;  // 8.5M terms a pose at 256^3: summed in double
-    const int rows = nf * nf, wtot = kSpecBlocks * 4;
-    for (int r = blockIdx.x * 4 + wv; r < rows; r += wtot) {
-        const int kx = r / nf, ky = r - kx * nf;
-        const float2 ex = ph[kx], ey = ph[nf + ky];
-        const float2 er = make_float2(ex.x * ey.x - ex.y * ey.y, ex.x * ey.y + ex.y * ey.x);
-        const float kxs = (float)signed_freq(kx, nf), kys = (float)signed_freq(ky, nf);
-        for (int j = 0; j < JZ; j++) {
-            if (!on[j]) continue;
-            const float2 e = make_float2(er.x * ez[j].x - er.y * ez[j].y, er.x * ez[j].y + er.y * ez[j].x);
-            const float2 x = q[(size_t)r * Hp + lane + 64 * j];
-            const float zr = x.x * e.x - x.y * e.y, zi = x.x * e.y + x.y * e.x;
-            v += wz[j] * zr;
-            const float im = wz[j] * zi;
-            gx += kxs * im;
-            gy += kys * im;
-            gz += kzs[j] * im;
-        }
-    }
-    __shared__ double red[4][256];
-    red[0][tid] = v;
-    red[1][tid] = gx;
-    red[2][tid] = gy;
-    red[3][tid] = gz;
-    __syncthreads();
-    for (int h = 128; h >= 1; h >>= 1) {
-        if (tid < h)
-            for (int a = 0; a < 4; a++) red[a][tid] += red[a][tid + h];
-        __syncthreads();
-    }
-    if (tid < 4) part[((size_t)b * kSpecBlocks + blockIdx.x) * 4 + tid] = red[tid][0];
-}
-
-// out[b][0..3] = (s, ds/dtx, ds/dty, ds/dtz), partial sums added in a fixed order
-__global__ void k_spec_finish(const double *__restrict__ part, float *out, int B, int nf) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B) return;
-    double s[4] = {0, 0, 0, 0};
-    for (int k = 0; k < kSpecBlocks; k++)
-        for (int a = 0; a < 4; a++) s[a] += part[((size_t)b * kSpecBlocks + k) * 4 + a];
-    const double n3 = (double)nf * nf * nf, g = -2.0 * M_PI / nf / n3;
-    out[4 * b] = (float)(s[0] / n3);
-    for (int a = 1; a < 4; a++) out[4 * b + a] = (float)(s[a] * g);
 }
 
 // trilinear value and gradient (per unit of u) of the two receptor grids at voxel
@@ -157,6 +94,24 @@ template <int K, int NT> __device__ __forceinline__ void block_sum(double *v) {
             for (int a = 0; a < K; a++) v[a] += part[w][a];
 }
 
+// out[b][0..3] = (s, ds/dtx, ds/dty, ds/dtz) from the n partial sums of kp_x_spec, one workgroup a
+// pose; added in a fixed order
+__global__ void __launch_bounds__(256) k_spec_finish(const double *__restrict__ part, float *__restrict__ out, int n,
+                                                     int nf) {
+    const double *p = part + (size_t)blockIdx.x * n * 4;
+    double s[4] = {0, 0, 0, 0};
+    for (int k = threadIdx.x; k < n; k += 256)
+#pragma unroll
+        for (int a = 0; a < 4; a++) s[a] += p[4 * k + a];
+    block_sum<4, 256>(s);
+    if (threadIdx.x == 0) {
+        const double n3 = (double)nf * nf * nf, g = -2.0 * M_PI / nf / n3;
+        float *o = out + 4 * (size_t)blockIdx.x;
+        o[0] = (float)(s[0] / n3);
+        for (int a = 1; a < 4; a++) o[a] = (float)(s[a] * g);
+    }
+}
+
 // out[b][7] = (s, ds/dt'(3), ds/dw(3)), one workgroup a pose and one launch a call: with eight
 // workgroups a pose, their partial sums and a second kernel, in batches of the context's size,
 // 2000 poses of 2081 atoms took 16 times two copies in, two kernels (13 and 4 us) and a copy out
@@ -201,12 +156,13 @@ __global__ void __launch_bounds__(256) k_companion(LigandDev L, const float *__r
 
 }  // namespace
 
-size_t grad_scratch_doubles(int max_batch) { return (size_t)max_batch * kSpecBlocks * 4; }
+hipError_t launch_spec_phase(const float *t_dev, int B, int nf, float2 *ph, hipStream_t s) {
+    k_spec_phase<<<B, 256, 0, s>>>(t_dev, ph, nf);
+    return hipGetLastError();
+}
 
-hipError_t launch_spec_eval(const float2 *Q, const float *t_dev, int B, int nf, int H, int Hp, double *part,
-                            float *out_dev, hipStream_t s) {
-    k_spec_eval<<<dim3(kSpecBlocks, B), 256, sizeof(float2) * 3 * nf, s>>>(Q, t_dev, part, nf, H, Hp);
-    k_spec_finish<<<(B + 63) / 64, 64, 0, s>>>(part, out_dev, B, nf);
+hipError_t launch_spec_finish(const double *part, int B, int n, int nf, float *out_dev, hipStream_t s) {
+    k_spec_finish<<<B, 256, 0, s>>>(part, out_dev, n, nf);
     return hipGetLastError();
 }
 

@@ -284,7 +284,8 @@ struct PipeArgs {
                         // with running top-t lists over contiguous planes (MDK_INV_VARIANT); at
                         // nf = 256: 0 two passes, 1 the half-plane inverse with 512 threads
                         // reading each plane once (the default), 2-3 with 1024 reading it twice
-    bool spectrum_only = false;  // stop after the fold: cc holds Q[b][kx][ky][kz]
+    const float2 *spec_ph = nullptr;  // spectral score: the poses' phases [b][3][nf], and its partial sums
+    double *spec_part = nullptr;      // [b][ky][Hp / 16][4], where the batch ends (no inverse)
     int fwd_variant = 0;         // forward passes: 0 fused z + y where it fits, the next plane prefetched (nf = 256: over half planes), 1 separate, 2 fused without the prefetch (MDK_FWD_VARIANT)
 };
 

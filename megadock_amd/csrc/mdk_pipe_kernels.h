@@ -430,15 +430,12 @@ __global__ void __launch_bounds__(1024) kp_fwd_half(VoxGrid vg, float2 *__restri
 // B_FAST: the rotation is the fastest grid index, so the workgroups that share a
 // receptor tile run back to back and find it in L2 / the last-level cache.
 // QA: the folded lines Q share the LDS of S (two more barriers, a third less LDS).
-// SPEC: store the folded spectrum Q itself, cc[b][kx][ky][kz], and skip the inverse x-FFT
-// (the spectral score evaluation reads it).
 // FLAT: the block's L columns are entries c L .. c L + L - 1 of the flat list, ky slowest,
 // of the columns kz >= KZ0 = L floor((nf/2 + 1) / L) (the ones that do not fill a whole
 // chunk) over all ky; the chunked launch covers kz < KZ0, so no padding column is
 // transformed.
 // PERM: d_a2 holds each run of 16 kz in parity-split order (kp_fwd_half, half_slot).
-template <int N, int L, int RB, bool CACHE_R, bool B_FAST = false, bool QA = false, bool SPEC = false,
-          bool FLAT = false, bool PERM = false>
+template <int N, int L, int RB, bool CACHE_R, bool B_FAST = false, bool QA = false, bool FLAT = false, bool PERM = false>
 __global__ void __launch_bounds__(2 * L *Geo<N>::T)
     kp_x_corr(const float2 *__restrict__ a2, const float2 *__restrict__ rec, float2 *__restrict__ cc,
               const float2 *__restrict__ twg, int H, int Hp, int B) {
@@ -456,7 +453,7 @@ __global__ void __launch_bounds__(2 * L *Geo<N>::T)
     const int b0 = (B_FAST ? blockIdx.x : blockIdx.z) * RB;
     // column (cky, ckz) of line l < L, and whether it exists
     constexpr int KZ0 = FLAT ? (N / 2 + 1) / L * L : 0, TWN = FLAT ? (N / 2 + 1) % L : 1;
-    static_assert(!FLAT || (TWN > 0 && !SPEC), "flat list of the remaining columns");
+    static_assert(!FLAT || TWN > 0, "flat list of the remaining columns");
     auto col = [&](int l, int &cky, int &ckz) {
         if constexpr (FLAT) {
             const int f = c * L + l;
@@ -542,14 +539,6 @@ __global__ void __launch_bounds__(2 * L *Geo<N>::T)
                 qv[p] = make_float2(0.5f * (p1.x + p2.x), 0.5f * (p1.y - p2.y));
             }
         }
-        if constexpr (SPEC) {
-            float2 *dst = cc + (size_t)b * N * N * Hp;
-            if (fkz < Hp)
-#pragma unroll
-                for (int p = 0; p < PER; p++)
-                    if (fx0 + FX * p < N) st_at(dst, 8u * (unsigned)(((fx0 + FX * p) * N + fky) * Hp + fkz), qv[p]);
-            continue;
-        }
         if (QA) __syncthreads();  // every read of S above is done before Q overwrites it
 #pragma unroll
         for (int p = 0; p < PER; p++)
@@ -584,6 +573,106 @@ __global__ void __launch_bounds__(2 * L *Geo<N>::T)
             }
         }
     }
+}
+
+// ------------------------------------------------------------------ x + spectral score
+// The spectral score of one pose per rotation (mdk_grad.hip) without its spectrum in memory:
+// workgroup (rotation b, chunk c of 16 columns kz, ky) transforms the columns and their
+// partners along x, folds them into Q(kx, ky, kz) as kp_x_corr does, and sums, per column,
+//   A = sum_kx Q e^{i phi_x},   B = sum_kx k'_x Q e^{i phi_x}
+// in double, then its columns' share of the score and of the gradient,
+//   w Re[A E], w Im[B E], k'_y w Im[A E], k'_z w Im[A E],   E = e^{i (phi_y + phi_z)},
+// into part[b][ky][c][4].  ph[b][3][N]: the phases e^{2 pi i k' t_a / N} of the pose.  Stored and
+// read back, the spectrum cost a pose of 144^3 13.3 MB each way: 1135 + 490 us per 128 poses for
+// the pass (of 8 columns a workgroup) and the evaluation.
+template <int N, bool PERM>
+__global__ void __launch_bounds__(32 * Geo<N>::T)
+    kp_x_spec(const float2 *__restrict__ a2, const float2 *__restrict__ rec, const float2 *__restrict__ ph,
+              double *__restrict__ part, const float2 *__restrict__ twg, int Hp) {
+    constexpr int N1 = Geo<N>::N1, N2 = Geo<N>::N2, T = Geo<N>::T, L = 16, L2 = 2 * L, LS2 = L2 + 1, NT = L2 * T;
+    constexpr int NG = N / 2, ND = N / 4, FX = NT / L, PER = (N + FX - 1) / FX;
+    __shared__ float2 S[N * LS2];
+    __shared__ float2 tw[N], ex[N];
+    static_assert(sizeof(S) >= 4 * NT * sizeof(double), "the sums reuse the lines' storage");
+    const int tid = threadIdx.x, b = blockIdx.x, c = blockIdx.y, ky = blockIdx.z;
+    ph += (size_t)b * 3 * N;
+    for (int q = tid; q < N; q += NT) {
+        tw[q] = twg[q];
+        ex[q] = ph[q];
+    }
+    const int fl = tid % L, fx0 = tid / L, kz = c * L + fl;
+    float2 r1[PER], r2[PER];
+#pragma unroll
+    for (int p = 0; p < PER; p++) {
+        r1[p] = r2[p] = make_float2(0.f, 0.f);
+        if (fx0 + FX * p < N) {  // zero where kz > N/2
+            const unsigned oa = 8u * (unsigned)(((fx0 + FX * p) * N + ky) * 2 * Hp + 2 * c * L + fl);
+            r1[p] = ld_at(rec, oa);
+            r2[p] = ld_at(rec, oa + 128u);
+        }
+    }
+    const int line = tid % L2, u = tid / L2, kzl = c * L + line % L;
+    const bool valid_line = kzl <= N / 2;
+    const int kyl = line < L ? ky : (N - ky) % N, kzs = line < L ? kzl : (N - kzl) % N;
+    __syncthreads();
+    if (u < N2) {
+        const float2 *src = a2 + (size_t)b * NG * N * N;  // uniform base, 32-bit lane offsets
+        float2 v[N1];
+        const int kzp = PERM ? half_slot_of_kz(kzs) : kzs;
+        const unsigned o0 = 8u * (unsigned)((u - ND) * N * N + kyl * N + kzp);  // used only when x is in range
+        sfor<0, N1>([&](auto jc) {
+            constexpr int j1 = decltype(jc)::value;
+            const int x = u + N2 * j1 - ND;
+            v[j1] = (valid_line && x >= 0 && x < NG) ? ld_at(src, o0 + 8u * N2 * j1 * N * N) : make_float2(0.f, 0.f);
+        });
+        rf::step1_store<N, false>(v, S, tw, LS2, line, u);
+    }
+    __syncthreads();
+    float2 y[N2];
+    if (u < N1) rf::step2_load<N, false>(y, S, LS2, line, u);
+    __syncthreads();
+    if (u < N1)
+        sfor<0, N2>([&](auto kc) {
+            constexpr int k2 = decltype(kc)::value;
+            S[(u + N1 * k2) * LS2 + line] = y[k2];
+        });
+    __syncthreads();
+    double ax = 0.0, ay = 0.0, bx = 0.0, by = 0.0;
+#pragma unroll
+    for (int p = 0; p < PER; p++) {
+        const int kx = fx0 + FX * p;
+        if (kx < N) {
+            const float2 l1 = S[kx * LS2 + fl], l2 = S[(kx == 0 ? 0 : N - kx) * LS2 + L + fl], a = r1[p], d = r2[p];
+            const float2 p1 = make_float2(a.x * l1.x + a.y * l1.y, a.x * l1.y - a.y * l1.x);
+            const float2 p2 = make_float2(d.x * l2.x + d.y * l2.y, d.x * l2.y - d.y * l2.x);
+            const float2 q = make_float2(0.5f * (p1.x + p2.x), 0.5f * (p1.y - p2.y)), e = ex[kx];
+            const float2 t = make_float2(q.x * e.x - q.y * e.y, q.x * e.y + q.y * e.x);
+            const double ks = (double)(kx < N / 2 ? kx : kx - N);
+            ax += t.x;
+            ay += t.y;
+            bx += ks * t.x;
+            by += ks * t.y;
+        }
+    }
+    const bool on = kz <= N / 2;
+    const float2 ey = ph[N + ky], ez = on ? ph[2 * N + kz] : make_float2(0.f, 0.f);
+    const double w = kz == 0 || 2 * kz == N ? 1.0 : 2.0;
+    const double er = w * ((double)ey.x * ez.x - (double)ey.y * ez.y), ei = w * ((double)ey.x * ez.y + (double)ey.y * ez.x);
+    const double im = ax * ei + ay * er;
+    double *red = reinterpret_cast<double *>(S);
+    __syncthreads();  // every line is read
+    red[tid] = on ? ax * er - ay * ei : 0.0;
+    red[NT + tid] = on ? bx * ei + by * er : 0.0;
+    red[2 * NT + tid] = on ? im * (ky < N / 2 ? ky : ky - N) : 0.0;
+    red[3 * NT + tid] = on ? im * (kz < N / 2 ? kz : kz - N) : 0.0;
+    __syncthreads();
+    for (int h = 512; h >= 1; h >>= 1) {  // NT <= 1024
+        if (tid < h && tid + h < NT)
+#pragma unroll
+            for (int a = 0; a < 4; a++) red[a * NT + tid] += red[a * NT + tid + h];
+        __syncthreads();
+    }
+    if (tid < 4) part[(((size_t)b * N + ky) * gridDim.y + c) * 4 + tid] = red[tid * NT];
 }
 
 // ------------------------------------------------------------------ inverse y, in place
@@ -1282,14 +1371,13 @@ template <int N, int LEVEL> hipError_t run_pipe(const PipeArgs &a) {
         }
     }
     if (a.ev) (void)hipEventRecord(a.ev[1], s);
-    if (a.spectrum_only) {
+    if (a.spec_part) {
+        const dim3 grid(B, a.Hp / 16, N);
         if (perm) {
             if constexpr (fwd_half_fits<N>())
-                kp_x_corr<N, LX, 1, false, true, true, true, false, true><<<dim3(B, a.Hp / LX, N), 2 * LX * T, 0, s>>>(
-                    a.a2, a.rec, a.cc, a.tw4, a.H, a.Hp, B);
+                kp_x_spec<N, true><<<grid, 32 * T, 0, s>>>(a.a2, a.rec, a.spec_ph, a.spec_part, a.tw4, a.Hp);
         } else {
-            kp_x_corr<N, LX, 1, false, true, true, true><<<dim3(B, a.Hp / LX, N), 2 * LX * T, 0, s>>>(a.a2, a.rec, a.cc,
-                                                                                                      a.tw4, a.H, a.Hp, B);
+            kp_x_spec<N, false><<<grid, 32 * T, 0, s>>>(a.a2, a.rec, a.spec_ph, a.spec_part, a.tw4, a.Hp);
         }
         return hipGetLastError();
     }
@@ -1306,13 +1394,13 @@ template <int N, int LEVEL> hipError_t run_pipe(const PipeArgs &a) {
         if constexpr (fwd_half_fits<N>()) {
             if (a.variant == 7 && NFL > 0) {
                 if constexpr (NCH > 0)
-                    kp_x_corr<N, LC, 1, true, true, true, false, false, true><<<dim3(B, NCH, N), 2 * LC * T, 0, s>>>(
+                    kp_x_corr<N, LC, 1, true, true, true, false, true><<<dim3(B, NCH, N), 2 * LC * T, 0, s>>>(
                         a.a2, a.rec, a.cc, a.tw4, a.H, a.Hp, B);
                 if constexpr (NFL > 0)
-                    kp_x_corr<N, LC, 1, true, true, true, false, true, true><<<dim3(B, NFL, 1), 2 * LC * T, 0, s>>>(
+                    kp_x_corr<N, LC, 1, true, true, true, true, true><<<dim3(B, NFL, 1), 2 * LC * T, 0, s>>>(
                         a.a2, a.rec, a.cc, a.tw4, a.H, a.Hp, B);
             } else {
-                kp_x_corr<N, 2 * LX, 1, true, true, true, false, false, true><<<dim3(B, a.Hp / (2 * LX), N), 4 * LX * T, 0, s>>>(
+                kp_x_corr<N, 2 * LX, 1, true, true, true, false, true><<<dim3(B, a.Hp / (2 * LX), N), 4 * LX * T, 0, s>>>(
                     a.a2, a.rec, a.cc, a.tw4, a.H, a.Hp, B);
             }
         }
@@ -1325,7 +1413,7 @@ template <int N, int LEVEL> hipError_t run_pipe(const PipeArgs &a) {
                 kp_x_corr<N, LC, 1, true, true, true><<<dim3(B, NCH, N), 2 * LC * T, 0, s>>>(a.a2, a.rec, a.cc, a.tw4,
                                                                                            a.H, a.Hp, B);
             if constexpr (NFL > 0)
-                kp_x_corr<N, LC, 1, true, true, true, false, true><<<dim3(B, NFL, 1), 2 * LC * T, 0, s>>>(
+                kp_x_corr<N, LC, 1, true, true, true, true><<<dim3(B, NFL, 1), 2 * LC * T, 0, s>>>(
                     a.a2, a.rec, a.cc, a.tw4, a.H, a.Hp, B);
         } else {
             kp_x_corr<N, 2 * LX, 1, true, true, true><<<dim3(B, a.Hp / (2 * LX), N), 4 * LX * T, 0, s>>>(
@@ -1359,7 +1447,7 @@ template <int N, int LEVEL> hipError_t run_pipe(const PipeArgs &a) {
                 kp_x_corr<N, LC, 1, true, true, true><<<dim3(B, NCH, N), 2 * LC * T, 0, s>>>(a.a2, a.rec, a.cc, a.tw4,
                                                                                            a.H, a.Hp, B);
             if constexpr (NFL > 0)
-                kp_x_corr<N, LC, 1, true, true, true, false, true><<<dim3(B, NFL, 1), 2 * LC * T, 0, s>>>(
+                kp_x_corr<N, LC, 1, true, true, true, true><<<dim3(B, NFL, 1), 2 * LC * T, 0, s>>>(
                     a.a2, a.rec, a.cc, a.tw4, a.H, a.Hp, B);
             break;
         }

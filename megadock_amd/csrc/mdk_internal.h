@@ -80,7 +80,7 @@ struct TopTState {
     unsigned pad;
     unsigned hist[256];
 };
-// keys sorted per rotation by launch_topt for t results per rotation (a power of two)
+// keys that launch_topt keeps per rotation for t results per rotation (a power of two)
 unsigned topt_sort_size(int t, int nf);
 // Top-t (t > MDK_MAXT) of B score maps smap[b][nf^3] (unnormalised real scores) into
 // out[(b0 + b) * t + q] as SortScore with rotation number rot_id[b0 + b], where b0 = *boff

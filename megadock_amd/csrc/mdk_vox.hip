@@ -23,6 +23,8 @@
 // they read), so a batch writes only the voxels its atoms touch.
 #pragma clang fp contract(off)
 
+#include <algorithm>
+
 #include "mdk_internal.h"
 
 namespace {
@@ -55,48 +57,49 @@ __device__ __forceinline__ void or_run(uint32_t *m, int row, int k0, int k1) {
     }
 }
 
-// Atom l of rotation b: its core/surface bit runs into cb/sb (global or LDS masks of one
-// rotation), its charge voxel into vidx and the voxel's atom count.
-__device__ __forceinline__ void vox_atom(const LigandDev &L, const float *r, int l, int b, uint32_t *cb,
-                                         uint32_t *sb, uint32_t *cnt, int *vidx, int cw) {
-    float X, Y, Z;
-    rotate_atom(L, r, l, X, Y, Z);
+// Plane i = (atom's voxel) + di of atom l, di in [-2, 2]: its core/surface bit runs into cb/sb
+// (global or LDS masks of one rotation); gc: the grid's coordinates.
+__device__ __forceinline__ void vox_plane(const LigandDev &L, const float *gc, float X, float Y, float Z, int l, int di,
+                                          uint32_t *cb, uint32_t *sb) {
     const int ng = L.ng, rw = row_words(ng);
     const float h = (float)(ng / 2);
     const int i2 = (int)(X / L.gw + h);
     const int j2 = (int)(Y / L.gw + h);
     const int k2 = (int)(Z / L.gw + h);
-    const int ia = max(i2 - 2, 0), ja = max(j2 - 2, 0), ka = max(k2 - 2, 0);
-    const int ib = min(i2 + 3, ng), jb = min(j2 + 3, ng), kb = min(k2 + 3, ng);
+    const int i = i2 + di;
+    if (i < 0 || i >= ng) return;
+    const int ja = max(j2 - 2, 0), ka = max(k2 - 2, 0);
+    const int jb = min(j2 + 3, ng), kb = min(k2 + 3, ng);
     const float rc2 = L.rc2[l], rs2 = L.rs2[l];
-    for (int i = ia; i < ib; i++) {
-        const float dx = X - L.gc[i];
-        const float xd = dx * dx;
-        if (xd > rc2) continue;  // rs2 <= rc2, so neither sphere reaches this plane
-        for (int j = ja; j < jb; j++) {
-            const float dy = Y - L.gc[j];
-            const float d2 = xd + dy * dy;
-            if (d2 > rc2) continue;
-            // the hits along k form one run per sphere (d3 grows away from the atom), but
-            // each voxel is tested exactly as the reference does
-            int c0 = kb, c1 = ka, s0 = kb, s1 = ka;
-            for (int k = ka; k < kb; k++) {
-                const float dz = Z - L.gc[k];
-                const float d3 = d2 + dz * dz;
-                if (d3 < rc2) { c0 = min(c0, k); c1 = k + 1; }
-                if (d3 < rs2) { s0 = min(s0, k); s1 = k + 1; }
-            }
-            const int row = (i * ng + j) * rw;
-            or_run(cb, row, c0, c1);
-            or_run(sb, row, s0, s1);
+    const float dx = X - gc[i];
+    const float xd = dx * dx;
+    if (xd > rc2) return;  // rs2 <= rc2, so neither sphere reaches this plane
+    for (int j = ja; j < jb; j++) {
+        const float dy = Y - gc[j];
+        const float d2 = xd + dy * dy;
+        if (d2 > rc2) continue;
+        // the hits along k form one run per sphere (d3 grows away from the atom), but
+        // each voxel is tested exactly as the reference does
+        int c0 = kb, c1 = ka, s0 = kb, s1 = ka;
+        for (int k = ka; k < kb; k++) {
+            const float dz = Z - gc[k];
+            const float d3 = d2 + dz * dz;
+            if (d3 < rc2) { c0 = min(c0, k); c1 = k + 1; }
+            if (d3 < rs2) { s0 = min(s0, k); s1 = k + 1; }
         }
+        const int row = (i * ng + j) * rw;
+        or_run(cb, row, c0, c1);
+        or_run(sb, row, s0, s1);
     }
+}
+
+// the voxel that holds an atom's charge
+__device__ __forceinline__ int charge_voxel(const LigandDev &L, float X, float Y, float Z) {
+    const int ng = L.ng;
     const int ci = max(0, min(ng - 1, (int)((X + L.pad) / L.gw)));
     const int cj = max(0, min(ng - 1, (int)((Y + L.pad) / L.gw)));
     const int ck = max(0, min(ng - 1, (int)((Z + L.pad) / L.gw)));
-    const int v = (ci * ng + cj) * ng + ck;
-    vidx[(size_t)b * L.na + l] = v;
-    atomicAdd(&cnt[(size_t)b * cw + (v >> 1)], 1u << (16 * (v & 1)));
+    return (ci * ng + cj) * ng + ck;
 }
 
 // one thread per (atom, rotation): core/surface bits, the charge voxel and its atom count
@@ -111,7 +114,12 @@ __global__ void k_vox_atoms(LigandDev L, const float *__restrict__ rot, const in
 #pragma unroll
     for (int q = 0; q < 9; q++) r[q] = rb[q];
     uint32_t *cb = cs + (size_t)b * 2 * mw;  // core bits
-    vox_atom(L, r, l, b, cb, cb + mw, cnt, vidx, cw);
+    float X, Y, Z;
+    rotate_atom(L, r, l, X, Y, Z);
+    for (int di = -2; di <= 2; di++) vox_plane(L, L.gc, X, Y, Z, l, di, cb, cb + mw);
+    const int v = charge_voxel(L, X, Y, Z);
+    vidx[(size_t)b * L.na + l] = v;
+    atomicAdd(&cnt[(size_t)b * cw + (v >> 1)], 1u << (16 * (v & 1)));
 }
 
 // bits k = 32 w + s of word w with lo <= k <= hi
@@ -179,34 +187,6 @@ __global__ void k_vox_masks(const uint32_t *__restrict__ cs, uint32_t *dmo, int 
     dmo[(size_t)b * 2 * mw + mw + q] = o;
 }
 
-// One workgroup per rotation with its core and surface bits in LDS (grids whose masks
-// fit): atom runs by LDS atomics, then the D and O words straight to dmo.  Replaces
-// k_clear + k_vox_atoms + k_vox_masks where it fits.
-constexpr int kVoxLdsThreads = 1024;
-constexpr size_t kVoxLdsBytes = 132 * 1024;  // both masks of one rotation, at most
-__global__ void __launch_bounds__(kVoxLdsThreads)
-    k_vox_lds(LigandDev L, const float *__restrict__ rot, const int *__restrict__ boff, uint32_t *dmo, uint32_t *cnt,
-              int *vidx, int mw, int cw) {
-    extern __shared__ uint32_t msk[];  // [2][mw]: core, surface
-    const int b = blockIdx.x, tid = threadIdx.x, ng = L.ng;
-    for (int q = tid; q < 2 * mw; q += kVoxLdsThreads) msk[q] = 0u;
-    const float *rb = rot + 9 * ((size_t)(boff ? *boff : 0) + b);
-    float r[9];
-#pragma unroll
-    for (int q = 0; q < 9; q++) r[q] = rb[q];
-    __syncthreads();
-    for (int l = tid; l < L.na; l += kVoxLdsThreads) vox_atom(L, r, l, b, msk, msk + mw, cnt, vidx, cw);
-    __syncthreads();
-    const MaskRows C{msk, ng, row_words(ng)}, S{msk + mw, ng, row_words(ng)};
-    uint32_t *db = dmo + (size_t)b * 2 * mw;
-    for (int q = tid; q < mw; q += kVoxLdsThreads) {
-        uint32_t d, o;
-        vox_mask_word(C, S, q, ng, L.delta, d, o);
-        db[q] = d;
-        db[mw + q] = o;
-    }
-}
-
 // Charges of the atoms nearest to each voxel, summed in atom order from +0.0f
 // (src/ligand.cpp:216-234).  One workgroup per rotation.  With one or two atoms in a
 // voxel the float sum does not depend on the order (0 + a = a and a + b = b + a
@@ -216,20 +196,21 @@ __global__ void __launch_bounds__(kVoxLdsThreads)
 constexpr int kChargeThreads = 1024;
 constexpr int kCrowdCap = 2048;  // listed atoms of crowded voxels (beyond: global scan)
 
-__global__ void __launch_bounds__(kChargeThreads)
-    k_vox_charge(const int *__restrict__ vidx, uint32_t *cnt, const float *__restrict__ charge, float *chg,
-                 int na, int ng3, int cw) {
+// the count may come from this launch's own atomics, which pass the vector cache by: so does the load
+__device__ __forceinline__ uint32_t voxel_count(uint32_t *cb, int v) {
+    return (__hip_atomic_load(&cb[v >> 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> (16 * (v & 1))) & 0xffffu;
+}
+
+// list: kCrowdCap entries of LDS, (voxel, atom)
+__device__ __forceinline__ void vox_charges(const int *vi, uint32_t *cb, const float *__restrict__ charge, float *g,
+                                            int na, int2 *list) {
     __shared__ int nlist;
-    __shared__ int2 list[kCrowdCap];  // (voxel, atom)
-    const int b = blockIdx.x, tid = threadIdx.x;
-    const int *vi = vidx + (size_t)b * na;
-    uint32_t *cb = cnt + (size_t)b * cw;
-    float *g = chg + (size_t)b * ng3;
+    const int tid = threadIdx.x;
     if (tid == 0) nlist = 0;
     __syncthreads();
     for (int l = tid; l < na; l += kChargeThreads) {
         const int v = vi[l];
-        const uint32_t n = (cb[v >> 1] >> (16 * (v & 1))) & 0xffffu;
+        const uint32_t n = voxel_count(cb, v);
         if (n <= 2) {
             atomicAdd(&g[v], charge[l]);
         } else {
@@ -260,7 +241,7 @@ __global__ void __launch_bounds__(kChargeThreads)
     } else {
         for (int l = tid; l < na; l += kChargeThreads) {
             const int v = vi[l];
-            const uint32_t n = (cb[v >> 1] >> (16 * (v & 1))) & 0xffffu;
+            const uint32_t n = voxel_count(cb, v);
             if (n <= 2) continue;
             bool owner = true;
             for (int q = 0; q < l; q++)
@@ -274,6 +255,59 @@ __global__ void __launch_bounds__(kChargeThreads)
     }
     __syncthreads();  // every count read above is done
     for (int l = tid; l < na; l += kChargeThreads) cb[vi[l] >> 1] = 0u;
+}
+
+__global__ void __launch_bounds__(kChargeThreads)
+    k_vox_charge(const int *vidx, uint32_t *cnt, const float *__restrict__ charge, float *chg, int na, int ng3, int cw) {
+    __shared__ int2 list[kCrowdCap];
+    const int b = blockIdx.x;
+    vox_charges(vidx + (size_t)b * na, cnt + (size_t)b * cw, charge, chg + (size_t)b * ng3, na, list);
+}
+
+// One workgroup per rotation with its core and surface bits in LDS (grids whose masks
+// fit): atom runs by LDS atomics, a thread per atom and plane of its sphere, then the D and O
+// words straight to dmo and the charges.  Replaces k_clear + k_vox_atoms + k_vox_masks +
+// k_vox_charge where it fits.  For one rotation it is a chain of dependent steps in one
+// workgroup: with a thread per atom walking five planes, the grid's coordinates loaded from
+// memory inside its loops, one ligand of 336 atoms took 21.6 us, and the charges a launch more.
+constexpr int kVoxLdsThreads = kChargeThreads;
+constexpr size_t kVoxLdsBytes = 132 * 1024;  // both masks of one rotation, at most
+__global__ void __launch_bounds__(kVoxLdsThreads)
+    k_vox_lds(LigandDev L, const float *__restrict__ rot, const int *__restrict__ boff, uint32_t *dmo, uint32_t *cnt,
+              int *vidx, int mw, int cw, float *chg) {
+    extern __shared__ uint32_t msk[];  // [2][mw]: core, surface; then the grid's coordinates
+    const int b = blockIdx.x, tid = threadIdx.x, ng = L.ng;
+    float *gc = reinterpret_cast<float *>(msk + 2 * mw);
+    for (int q = tid; q < 2 * mw; q += kVoxLdsThreads) msk[q] = 0u;
+    for (int q = tid; q < ng; q += kVoxLdsThreads) gc[q] = L.gc[q];
+    const float *rb = rot + 9 * ((size_t)(boff ? *boff : 0) + b);
+    float r[9];
+#pragma unroll
+    for (int q = 0; q < 9; q++) r[q] = rb[q];
+    __syncthreads();
+    for (int q = tid; q < 5 * L.na; q += kVoxLdsThreads) {
+        const int l = q / 5, di = q - 5 * l - 2;
+        float X, Y, Z;
+        rotate_atom(L, r, l, X, Y, Z);
+        vox_plane(L, gc, X, Y, Z, l, di, msk, msk + mw);
+        if (di == 0) {
+            const int v = charge_voxel(L, X, Y, Z);
+            vidx[(size_t)b * L.na + l] = v;
+            atomicAdd(&cnt[(size_t)b * cw + (v >> 1)], 1u << (16 * (v & 1)));
+        }
+    }
+    __syncthreads();
+    const MaskRows C{msk, ng, row_words(ng)}, S{msk + mw, ng, row_words(ng)};
+    uint32_t *db = dmo + (size_t)b * 2 * mw;
+    for (int q = tid; q < mw; q += kVoxLdsThreads) {
+        uint32_t d, o;
+        vox_mask_word(C, S, q, ng, L.delta, d, o);
+        db[q] = d;
+        db[mw + q] = o;
+    }
+    __syncthreads();  // the masks are read; their LDS takes the list of the crowded voxels' atoms
+    vox_charges(vidx + (size_t)b * L.na, cnt + (size_t)b * cw, L.charge, chg + (size_t)b * ng * ng * ng, L.na,
+                reinterpret_cast<int2 *>(msk));
 }
 
 // grids as (grid_r, grid_i) pairs; clears the charge grid it reads
@@ -290,17 +324,18 @@ hipError_t launch_voxelize(const LigandDev &lig, const float *rot, int B, const 
                            float *chg, hipStream_t s, const int *boff) {
     const int ng = lig.ng, mw = mask_words(ng), cw = count_words(ng);
     const int ng3 = ng * ng * ng;
-    const size_t lds = 2 * sizeof(uint32_t) * (size_t)mw;
-    if (lds <= kVoxLdsBytes) {  // one workgroup per rotation, bits in LDS
-        k_vox_lds<<<B, kVoxLdsThreads, lds, s>>>(lig, rot, boff, vs.dmo, vs.cnt, vidx, mw, cw);
+    const size_t masks = 2 * sizeof(uint32_t) * (size_t)mw;
+    if (masks <= kVoxLdsBytes) {  // one workgroup per rotation, bits in LDS
+        const size_t lds = std::max(masks + sizeof(float) * ng, sizeof(int2) * kCrowdCap);
+        k_vox_lds<<<B, kVoxLdsThreads, lds, s>>>(lig, rot, boff, vs.dmo, vs.cnt, vidx, mw, cw, chg);
     } else {
         const size_t nclear = 2 * (size_t)B * mw;  // core and surface bits; counts are kept zero
         k_clear<<<dim3((unsigned)((nclear + 255) / 256 < 65535 ? (nclear + 255) / 256 : 65535)), 256, 0, s>>>(vs.cs,
                                                                                                        nclear);
         k_vox_atoms<<<dim3((lig.na + 127) / 128, B), 128, 0, s>>>(lig, rot, boff, vs.cs, vs.cnt, vidx, mw, cw);
         k_vox_masks<<<dim3((mw + 255) / 256, B), 256, 0, s>>>(vs.cs, vs.dmo, ng, mw, lig.delta);
+        k_vox_charge<<<B, kChargeThreads, 0, s>>>(vidx, vs.cnt, lig.charge, chg, lig.na, ng3, cw);
     }
-    k_vox_charge<<<B, kChargeThreads, 0, s>>>(vidx, vs.cnt, lig.charge, chg, lig.na, ng3, cw);
     return hipGetLastError();
 }
 

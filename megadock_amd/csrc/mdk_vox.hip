@@ -45,51 +45,63 @@ __global__ void k_clear(uint32_t *p, size_t n) {
         p[i] = 0u;
 }
 
-// set bits [k0, k1) of a row that starts at word `row` (k1 - k0 <= 5)
-__device__ __forceinline__ void or_run(uint32_t *m, int row, int k0, int k1) {
-    if (k1 <= k0) return;
-    const int w0 = k0 >> 5, w1 = (k1 - 1) >> 5;
-    if (w0 == w1) {
-        atomicOr(&m[row + w0], ((1u << (k1 - k0)) - 1u) << (k0 & 31));
-    } else {
-        atomicOr(&m[row + w0], 0xffffffffu << (k0 & 31));
-        atomicOr(&m[row + w1], 0xffffffffu >> (31 - ((k1 - 1) & 31)));
-    }
-}
-
-// Plane i = (atom's voxel) + di of atom l, di in [-2, 2]: its core/surface bit runs into cb/sb
-// (global or LDS masks of one rotation); gc: the grid's coordinates.
-__device__ __forceinline__ void vox_plane(const LigandDev &L, const float *gc, float X, float Y, float Z, int l, int di,
-                                          uint32_t *cb, uint32_t *sb) {
+// Planes (atom's voxel) + d0 .. + d1 - 1 of atom l's box, -2 <= d0 < d1 <= 3: its core/surface bits
+// into cb/sb (global or LDS masks of one rotation); gc: the grid's coordinates.  Bound by its
+// vector instructions (the LDS form has one workgroup's waves on one CU): the box's ten squared
+// coordinate differences are formed once, the tests of a row gather into five bits, and a row's
+// run is those bits shifted into the word of the box's first column.
+__device__ __forceinline__ void vox_planes(const LigandDev &L, const float *gc, float X, float Y, float Z, int l, int d0,
+                                           int d1, uint32_t *cb, uint32_t *sb) {
     const int ng = L.ng, rw = row_words(ng);
     const float h = (float)(ng / 2);
-    const int i2 = (int)(X / L.gw + h);
-    const int j2 = (int)(Y / L.gw + h);
-    const int k2 = (int)(Z / L.gw + h);
-    const int i = i2 + di;
-    if (i < 0 || i >= ng) return;
-    const int ja = max(j2 - 2, 0), ka = max(k2 - 2, 0);
-    const int jb = min(j2 + 3, ng), kb = min(k2 + 3, ng);
+    // (a voxel far outside has the same empty box as one 3 outside)
+    const int i2 = min(max((int)(X / L.gw + h), -3), ng + 2);
+    const int j2 = min(max((int)(Y / L.gw + h), -3), ng + 2);
+    const int k2 = min(max((int)(Z / L.gw + h), -3), ng + 2);
+    const int ka = max(k2 - 2, 0), kn = min(k2 + 3, ng) - ka;  // the box's columns: ka .. ka + kn - 1
+    const uint32_t inside = kn > 0 ? (1u << kn) - 1u : 0u;
     const float rc2 = L.rc2[l], rs2 = L.rs2[l];
-    const float dx = X - gc[i];
-    const float xd = dx * dx;
-    if (xd > rc2) return;  // rs2 <= rc2, so neither sphere reaches this plane
-    for (int j = ja; j < jb; j++) {
-        const float dy = Y - gc[j];
-        const float d2 = xd + dy * dy;
-        if (d2 > rc2) continue;
-        // the hits along k form one run per sphere (d3 grows away from the atom), but
-        // each voxel is tested exactly as the reference does
-        int c0 = kb, c1 = ka, s0 = kb, s1 = ka;
-        for (int k = ka; k < kb; k++) {
-            const float dz = Z - gc[k];
-            const float d3 = d2 + dz * dz;
-            if (d3 < rc2) { c0 = min(c0, k); c1 = k + 1; }
-            if (d3 < rs2) { s0 = min(s0, k); s1 = k + 1; }
+    float y2[5], z2[5];
+#pragma unroll
+    for (int q = 0; q < 5; q++) {  // outside the grid: any coordinate, not used below
+        const int j = min(max(j2 - 2 + q, 0), ng - 1), k = min(ka + q, ng - 1);
+        const float dy = Y - gc[j], dz = Z - gc[k];
+        y2[q] = dy * dy;
+        z2[q] = dz * dz;
+    }
+    const int w = ka >> 5, sh = ka & 31;
+    for (int di = d0; di < d1; di++) {
+        const int i = i2 + di;
+        if (i < 0 || i >= ng) continue;
+        const float dx = X - gc[i];
+        const float xd = dx * dx;
+        if (xd > rc2) continue;  // rs2 <= rc2, so neither sphere reaches this plane
+        const int row0 = (i * ng + j2 - 2) * rw + w;
+#pragma unroll
+        for (int p = 0; p < 5; p++) {
+            const int j = j2 - 2 + p;
+            const float d2 = xd + y2[p];
+            if (j < 0 || j >= ng || d2 > rc2) continue;
+            // each voxel is tested exactly as the reference does; the hits along k form one run
+            // per sphere (d3 grows away from the atom)
+            uint32_t c = 0, s = 0;
+#pragma unroll
+            for (int q = 4; q >= 0; q--) {
+                const float d3 = d2 + z2[q];
+                c = c + c + (d3 < rc2 ? 1u : 0u);
+                s = s + s + (d3 < rs2 ? 1u : 0u);
+            }
+            c &= inside;
+            s &= inside;
+            if (c == 0) continue;  // rs2 <= rc2
+            c = (c | (0u - c)) & (0xffffffffu >> __clz(c));
+            atomicOr(&cb[row0 + p * rw], c << sh);
+            if (sh > 27 && c >> (32 - sh)) atomicOr(&cb[row0 + p * rw + 1], c >> (32 - sh));
+            if (s == 0) continue;
+            s = (s | (0u - s)) & (0xffffffffu >> __clz(s));
+            atomicOr(&sb[row0 + p * rw], s << sh);
+            if (sh > 27 && s >> (32 - sh)) atomicOr(&sb[row0 + p * rw + 1], s >> (32 - sh));
         }
-        const int row = (i * ng + j) * rw;
-        or_run(cb, row, c0, c1);
-        or_run(sb, row, s0, s1);
     }
 }
 
@@ -116,7 +128,7 @@ __global__ void k_vox_atoms(LigandDev L, const float *__restrict__ rot, const in
     uint32_t *cb = cs + (size_t)b * 2 * mw;  // core bits
     float X, Y, Z;
     rotate_atom(L, r, l, X, Y, Z);
-    for (int di = -2; di <= 2; di++) vox_plane(L, L.gc, X, Y, Z, l, di, cb, cb + mw);
+    vox_planes(L, L.gc, X, Y, Z, l, -2, 3, cb, cb + mw);
     const int v = charge_voxel(L, X, Y, Z);
     vidx[(size_t)b * L.na + l] = v;
     atomicAdd(&cnt[(size_t)b * cw + (v >> 1)], 1u << (16 * (v & 1)));
@@ -271,6 +283,7 @@ __global__ void __launch_bounds__(kChargeThreads)
 // workgroup: with a thread per atom walking five planes, the grid's coordinates loaded from
 // memory inside its loops, one ligand of 336 atoms took 21.6 us, and the charges a launch more.
 constexpr int kVoxLdsThreads = kChargeThreads;
+constexpr int kVoxSplitAtoms = 512;
 constexpr size_t kVoxLdsBytes = 132 * 1024;  // both masks of one rotation, at most
 __global__ void __launch_bounds__(kVoxLdsThreads)
     k_vox_lds(LigandDev L, const float *__restrict__ rot, const int *__restrict__ boff, uint32_t *dmo, uint32_t *cnt,
@@ -285,12 +298,15 @@ __global__ void __launch_bounds__(kVoxLdsThreads)
 #pragma unroll
     for (int q = 0; q < 9; q++) r[q] = rb[q];
     __syncthreads();
-    for (int q = tid; q < 5 * L.na; q += kVoxLdsThreads) {
-        const int l = q / 5, di = q - 5 * l - 2;
+    // an atom's five planes in one thread share its box; a small ligand's go to five threads, so
+    // that the CU's four SIMDs have waves enough
+    const int split = L.na <= kVoxSplitAtoms ? 5 : 1;
+    for (int q = tid; q < split * L.na; q += kVoxLdsThreads) {
+        const int l = q / split, d = q - split * l;
         float X, Y, Z;
         rotate_atom(L, r, l, X, Y, Z);
-        vox_plane(L, gc, X, Y, Z, l, di, msk, msk + mw);
-        if (di == 0) {
+        vox_planes(L, gc, X, Y, Z, l, d - 2, split == 1 ? 3 : d - 1, msk, msk + mw);
+        if (d == 0) {
             const int v = charge_voxel(L, X, Y, Z);
             vidx[(size_t)b * L.na + l] = v;
             atomicAdd(&cnt[(size_t)b * cw + (v >> 1)], 1u << (16 * (v & 1)));

@@ -208,30 +208,13 @@ __global__ void k_vox_masks(const uint32_t *__restrict__ cs, uint32_t *dmo, int 
 constexpr int kChargeThreads = 1024;
 constexpr int kCrowdCap = 2048;  // listed atoms of crowded voxels (beyond: global scan)
 
-// the count may come from this launch's own atomics, which pass the vector cache by: so does the load
-__device__ __forceinline__ uint32_t voxel_count(uint32_t *cb, int v) {
-    return (__hip_atomic_load(&cb[v >> 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> (16 * (v & 1))) & 0xffffu;
-}
-
-// list: kCrowdCap entries of LDS, (voxel, atom)
-__device__ __forceinline__ void vox_charges(const int *vi, uint32_t *cb, const float *__restrict__ charge, float *g,
-                                            int na, int2 *list) {
-    __shared__ int nlist;
+// Voxels with three or more atoms (count(v): how many of them lie in v), whose atoms are listed in
+// list[0 .. *nlist), or any atoms if *nlist is above kCrowdCap: the sum in atom order
+template <class Count>
+__device__ __forceinline__ void vox_crowded(const int *vi, const float *__restrict__ charge, float *g, int na,
+                                            const int2 *list, const int *nlist, Count count) {
     const int tid = threadIdx.x;
-    if (tid == 0) nlist = 0;
-    __syncthreads();
-    for (int l = tid; l < na; l += kChargeThreads) {
-        const int v = vi[l];
-        const uint32_t n = voxel_count(cb, v);
-        if (n <= 2) {
-            atomicAdd(&g[v], charge[l]);
-        } else {
-            const int k = atomicAdd(&nlist, 1);
-            if (k < kCrowdCap) list[k] = make_int2(v, l);
-        }
-    }
-    __syncthreads();
-    const int m = nlist;  // uniform
+    const int m = *nlist;  // uniform
     if (m <= kCrowdCap) {
         for (int e = tid; e < m; e += kChargeThreads) {
             const int v = list[e].x, l = list[e].y;
@@ -253,8 +236,7 @@ __device__ __forceinline__ void vox_charges(const int *vi, uint32_t *cb, const f
     } else {
         for (int l = tid; l < na; l += kChargeThreads) {
             const int v = vi[l];
-            const uint32_t n = voxel_count(cb, v);
-            if (n <= 2) continue;
+            if (count(v) <= 2) continue;
             bool owner = true;
             for (int q = 0; q < l; q++)
                 if (vi[q] == v) owner = false;
@@ -265,30 +247,107 @@ __device__ __forceinline__ void vox_charges(const int *vi, uint32_t *cb, const f
             g[v] = sum;
         }
     }
+}
+
+// the counts are global words of two 16-bit counts, left zero again
+__global__ void __launch_bounds__(kChargeThreads)
+    k_vox_charge(const int *vidx, uint32_t *cnt, const float *__restrict__ charge, float *chg, int na, int ng3, int cw) {
+    __shared__ int nlist;
+    __shared__ int2 list[kCrowdCap];  // (voxel, atom)
+    const int b = blockIdx.x, tid = threadIdx.x;
+    const int *vi = vidx + (size_t)b * na;
+    uint32_t *cb = cnt + (size_t)b * cw;
+    float *g = chg + (size_t)b * ng3;
+    auto count = [&](int v) { return (cb[v >> 1] >> (16 * (v & 1))) & 0xffffu; };
+    if (tid == 0) nlist = 0;
+    __syncthreads();
+    for (int l = tid; l < na; l += kChargeThreads) {
+        const int v = vi[l];
+        if (count(v) <= 2) {
+            atomicAdd(&g[v], charge[l]);
+        } else {
+            const int k = atomicAdd(&nlist, 1);
+            if (k < kCrowdCap) list[k] = make_int2(v, l);
+        }
+    }
+    __syncthreads();
+    vox_crowded(vi, charge, g, na, list, &nlist, count);
     __syncthreads();  // every count read above is done
     for (int l = tid; l < na; l += kChargeThreads) cb[vi[l] >> 1] = 0u;
 }
 
-__global__ void __launch_bounds__(kChargeThreads)
-    k_vox_charge(const int *vidx, uint32_t *cnt, const float *__restrict__ charge, float *chg, int na, int ng3, int cw) {
-    __shared__ int2 list[kCrowdCap];
-    const int b = blockIdx.x;
-    vox_charges(vidx + (size_t)b * na, cnt + (size_t)b * cw, charge, chg + (size_t)b * ng3, na, list);
+// The same with the voxels' counts and sums in an LDS table of nt entries (a power of two, three
+// times na where there is room: probes stay under 15; never less than 1.6 times): tab holds
+// (voxel + 1) << 13 | atoms, 0 if free, linear probing.  One workgroup.  The global counts cost an
+// atomic and a read on a line of their own for every atom, the sums another: 20 us of the 52 that
+// a batch of 128 rotations of 2081 atoms took; the table takes 9.
+constexpr int kCountBits = 13, kTableMax = 8192;
+__device__ __forceinline__ uint32_t table_slot(int v, int nt) {  // the product's leading bits
+    return (uint32_t)v * 2654435761u >> (__clz(nt) + 1);
+}
+__device__ __forceinline__ void vox_charges_lds(const int *vi, const float *__restrict__ charge, float *g, int na,
+                                                uint32_t *tab, float *sum, int nt, int2 *list) {
+    __shared__ int nlist;
+    const int tid = threadIdx.x;
+    if (tid == 0) nlist = 0;
+    for (int q = tid; q < nt; q += kChargeThreads) {
+        tab[q] = 0u;
+        sum[q] = 0.0f;
+    }
+    __syncthreads();
+    for (int l = tid; l < na; l += kChargeThreads) {
+        const int v = vi[l];
+        const uint32_t first = (uint32_t)(v + 1) << kCountBits | 1u;
+        uint32_t q = table_slot(v, nt);
+        for (;; q = (q + 1) & (nt - 1)) {  // a free entry is met: nt > na
+            const uint32_t was = atomicCAS(&tab[q], 0u, first);
+            if (was == 0u) break;
+            if ((was ^ first) >> kCountBits == 0u) {
+                atomicAdd(&tab[q], 1u);
+                break;
+            }
+        }
+        atomicAdd(&sum[q], charge[l]);
+    }
+    __syncthreads();
+    bool crowd = false;
+    for (int q = tid; q < nt; q += kChargeThreads) {
+        const uint32_t w = tab[q], n = w & ((1u << kCountBits) - 1u);
+        if (n > 2)
+            crowd = true;
+        else if (sum[q] != 0.0f)  // the grid is zero
+            g[(w >> kCountBits) - 1] = sum[q];
+    }
+    if (!__syncthreads_or(crowd)) return;
+    auto count = [&](int v) {
+        uint32_t q = table_slot(v, nt);
+        while (tab[q] >> kCountBits != (uint32_t)(v + 1)) q = (q + 1) & (nt - 1);  // v is in the table
+        return tab[q] & ((1u << kCountBits) - 1u);
+    };
+    for (int l = tid; l < na; l += kChargeThreads) {
+        const int v = vi[l];
+        if (count(v) <= 2) continue;
+        const int k = atomicAdd(&nlist, 1);
+        if (k < kCrowdCap) list[k] = make_int2(v, l);
+    }
+    __syncthreads();
+    vox_crowded(vi, charge, g, na, list, &nlist, count);
 }
 
 // One workgroup per rotation with its core and surface bits in LDS (grids whose masks
-// fit): atom runs by LDS atomics, a thread per atom and plane of its sphere, then the D and O
-// words straight to dmo and the charges.  Replaces k_clear + k_vox_atoms + k_vox_masks +
-// k_vox_charge where it fits.  For one rotation it is a chain of dependent steps in one
-// workgroup: with a thread per atom walking five planes, the grid's coordinates loaded from
-// memory inside its loops, one ligand of 336 atoms took 21.6 us, and the charges a launch more.
+// fit): atom runs by LDS atomics, then the D and O words straight to dmo and, if nt > 0, the
+// charges by a table of nt entries (else k_vox_charge follows).  Replaces k_clear + k_vox_atoms +
+// k_vox_masks + k_vox_charge where it fits.  For one rotation it is a chain of dependent steps in
+// one workgroup: with a thread per atom walking five planes, the grid's coordinates loaded from
+// memory inside its loops, a ligand of 336 atoms took 21.6 us and its charges a launch of 4.2 us.
 constexpr int kVoxLdsThreads = kChargeThreads;
 constexpr int kVoxSplitAtoms = 512;
 constexpr size_t kVoxLdsBytes = 132 * 1024;  // both masks of one rotation, at most
 __global__ void __launch_bounds__(kVoxLdsThreads)
     k_vox_lds(LigandDev L, const float *__restrict__ rot, const int *__restrict__ boff, uint32_t *dmo, uint32_t *cnt,
-              int *vidx, int mw, int cw, float *chg) {
-    extern __shared__ uint32_t msk[];  // [2][mw]: core, surface; then the grid's coordinates
+              int *vidx, int mw, int cw, float *chg, int nt) {
+    // [2][mw]: core, surface; then the grid's coordinates.  After the masks: the charges' table
+    extern __shared__ uint32_t msk[];
     const int b = blockIdx.x, tid = threadIdx.x, ng = L.ng;
     float *gc = reinterpret_cast<float *>(msk + 2 * mw);
     for (int q = tid; q < 2 * mw; q += kVoxLdsThreads) msk[q] = 0u;
@@ -309,7 +368,7 @@ __global__ void __launch_bounds__(kVoxLdsThreads)
         if (d == 0) {
             const int v = charge_voxel(L, X, Y, Z);
             vidx[(size_t)b * L.na + l] = v;
-            atomicAdd(&cnt[(size_t)b * cw + (v >> 1)], 1u << (16 * (v & 1)));
+            if (nt == 0) atomicAdd(&cnt[(size_t)b * cw + (v >> 1)], 1u << (16 * (v & 1)));
         }
     }
     __syncthreads();
@@ -321,9 +380,10 @@ __global__ void __launch_bounds__(kVoxLdsThreads)
         db[q] = d;
         db[mw + q] = o;
     }
-    __syncthreads();  // the masks are read; their LDS takes the list of the crowded voxels' atoms
-    vox_charges(vidx + (size_t)b * L.na, cnt + (size_t)b * cw, L.charge, chg + (size_t)b * ng * ng * ng, L.na,
-                reinterpret_cast<int2 *>(msk));
+    if (nt == 0) return;
+    __syncthreads();  // the masks are read
+    vox_charges_lds(vidx + (size_t)b * L.na, L.charge, chg + (size_t)b * ng * ng * ng, L.na, msk,
+                    reinterpret_cast<float *>(msk + nt), nt, reinterpret_cast<int2 *>(msk + 2 * nt));
 }
 
 // grids as (grid_r, grid_i) pairs; clears the charge grid it reads
@@ -342,8 +402,16 @@ hipError_t launch_voxelize(const LigandDev &lig, const float *rot, int B, const 
     const int ng3 = ng * ng * ng;
     const size_t masks = 2 * sizeof(uint32_t) * (size_t)mw;
     if (masks <= kVoxLdsBytes) {  // one workgroup per rotation, bits in LDS
-        const size_t lds = std::max(masks + sizeof(float) * ng, sizeof(int2) * kCrowdCap);
-        k_vox_lds<<<B, kVoxLdsThreads, lds, s>>>(lig, rot, boff, vs.dmo, vs.cnt, vidx, mw, cw, chg);
+        // the charges' table beside their list, where it fits into the masks' LDS (or little enough
+        // for two workgroups a CU); more atoms than that are counted in memory
+        const size_t most = std::max(masks + sizeof(float) * ng, (size_t)64 * 1024);
+        auto table = [](int n) { return 2 * sizeof(uint32_t) * (size_t)n + sizeof(int2) * kCrowdCap; };
+        int nt = kTableMax;
+        while (nt > 256 && (nt / 2 >= 3 * lig.na || table(nt) > most)) nt /= 2;
+        if (nt / 8 * 5 < lig.na) nt = 0;
+        const size_t lds = std::max(masks + sizeof(float) * ng, nt ? table(nt) : 0);
+        k_vox_lds<<<B, kVoxLdsThreads, lds, s>>>(lig, rot, boff, vs.dmo, vs.cnt, vidx, mw, cw, chg, nt);
+        if (!nt) k_vox_charge<<<B, kChargeThreads, 0, s>>>(vidx, vs.cnt, lig.charge, chg, lig.na, ng3, cw);
     } else {
         const size_t nclear = 2 * (size_t)B * mw;  // core and surface bits; counts are kept zero
         k_clear<<<dim3((unsigned)((nclear + 255) / 256 < 65535 ? (nclear + 255) / 256 : 65535)), 256, 0, s>>>(vs.cs,

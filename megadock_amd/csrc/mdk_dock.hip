@@ -69,6 +69,7 @@ constexpr int WZ = 16;   // lines per workgroup, z passes
 constexpr int WY = 16;   // lines per workgroup, y passes
 constexpr int WX = 8;    // kz columns per workgroup in the x pass (plus 8 partner columns)
 constexpr int NT = 256;  // threads per workgroup
+constexpr size_t kDirectResults = 256;  // mdk_dock: as many results go straight to host memory
 
 __device__ __forceinline__ void load_tw(float2 *tw_s, const float2 *tw_g, int ntw) {
     for (int q = threadIdx.x; q < ntw; q += blockDim.x) tw_s[q] = tw_g[q];
@@ -297,7 +298,7 @@ __global__ void __launch_bounds__(NT) k_reduce_top(const Cand *__restrict__ cand
     __shared__ Cand lists[NT * MDK_MAXT];
     const int b = blockIdx.x;
     const int b0 = boff ? *boff : 0;
-    rot_id += b0;
+    const int id = rot_id[b0 + b];  // asked for early: it may lie in host memory
     out += (size_t)b0 * t;
     const Cand *src = cand + (size_t)b * lists_per_rot * t;
     const int n = lists_per_rot * t;
@@ -338,7 +339,7 @@ __global__ void __launch_bounds__(NT) k_reduce_top(const Cand *__restrict__ cand
             const int idx = keep ? c.idx : 0;
             mdk_sortscore s;
             s.score = keep ? (t == 1 ? c.key / nf3f : c.key) : (t == 1 ? 0.0f : -99999.0f);
-            s.index[0] = rot_id[b];
+            s.index[0] = id;
             s.index[1] = idx / nf2;
             s.index[2] = (idx / nf) % nf;
             s.index[3] = idx % nf;
@@ -500,6 +501,10 @@ struct mdk_ctx {
     int *d_rotid = nullptr;  // iota table, rotation i has number i
     float *d_brot = nullptr; // staging for mdk_dock (max_batch * 9)
     int *d_bid = nullptr;    // staging ids
+    // mdk_dock's calls of few results: one pinned block, read and written by the kernels
+    mdk_sortscore *h_dock_out = nullptr;
+    float *h_dock_rot = nullptr;
+    int *h_dock_id = nullptr;
     // batch buffers: one set per stream; mdk_dock_range alternates batches between the
     // streams so that one batch's memory-bound passes overlap another's compute-bound ones
     static constexpr int kMaxSlots = 3;
@@ -828,6 +833,11 @@ int mdk_create(int device, int nf, int ng, int na, int t, int max_batch, mdk_ctx
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0)
             c->cu_count = cus;
     }
+    if (hipHostMalloc((void **)&c->h_dock_out, kDirectResults * (sizeof(mdk_sortscore) + 10 * sizeof(float)),
+                      hipHostMallocDefault) != hipSuccess)
+        return bail(fail("mdk_create: pinned memory allocation failed"));
+    c->h_dock_rot = reinterpret_cast<float *>(c->h_dock_out + kDirectResults);
+    c->h_dock_id = reinterpret_cast<int *>(c->h_dock_rot + 9 * kDirectResults);
     if (hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess)
         return bail(fail("mdk_create: event creation failed"));
     // the largest kernel LDS request must fit
@@ -854,6 +864,7 @@ int mdk_destroy(mdk_ctx *c) {
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (c->h_topn) (void)hipHostFree(c->h_topn);
+    if (c->h_dock_out) (void)hipHostFree(c->h_dock_out);
     if (c->topn_done) (void)hipEventDestroy(c->topn_done);
     if (c->h_rstage) (void)hipHostFree(c->h_rstage);
     if (c->h_lstage) (void)hipHostFree(c->h_lstage);
@@ -1084,10 +1095,28 @@ int mdk_dock(mdk_ctx *c, const float *rotcoef, const int *rot_id, int B, mdk_sor
     if (!c->have_rec || !c->have_lig) return fail("mdk_dock: receptor and ligand must be set first");
     if (B < 1 || B > c->max_batch) return fail("mdk_dock: batch size out of range");
     HIPCHK(hipSetDevice(c->device));
+    const size_t m = (size_t)B * c->t;
+    if (m <= kDirectResults && c->t <= MDK_MAXT) {
+        // Few results: the kernels read the rotations and write the results in pinned host memory.
+        // The three copies were launches of their own, and from pageable memory waits of the
+        // host's: one rotation at 80^3 80 -> 50 us, 128 at 100^3 785 -> 765.  A voxelizer that
+        // reads a rotation's coefficients in many wavefronts (large grids) still has them copied.
+        std::memcpy(c->h_dock_rot, rotcoef, sizeof(float) * 9 * B);
+        std::memcpy(c->h_dock_id, rot_id, sizeof(int) * B);
+        const float *rot = c->h_dock_rot;
+        if (!voxelizer_reads_once(c->ng)) {
+            HIPCHK(hipMemcpyAsync(c->d_brot, rot, sizeof(float) * 9 * B, hipMemcpyHostToDevice, c->stream));
+            rot = c->d_brot;
+        }
+        if (dock_batch(c, c->slot[0], rot, c->h_dock_id, B, c->h_dock_out)) return 1;
+        HIPCHK(hipStreamSynchronize(c->stream));
+        std::memcpy(out, c->h_dock_out, sizeof(mdk_sortscore) * m);
+        return 0;
+    }
     HIPCHK(hipMemcpyAsync(c->d_brot, rotcoef, sizeof(float) * 9 * B, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(c->d_bid, rot_id, sizeof(int) * B, hipMemcpyHostToDevice, c->stream));
     if (dock_batch(c, c->slot[0], c->d_brot, c->d_bid, B, c->slot[0].d_bout)) return 1;
-    HIPCHK(hipMemcpyAsync(out, c->slot[0].d_bout, sizeof(mdk_sortscore) * B * c->t, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipMemcpyAsync(out, c->slot[0].d_bout, sizeof(mdk_sortscore) * m, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return 0;
 }

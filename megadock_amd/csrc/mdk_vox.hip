@@ -343,6 +343,7 @@ __device__ __forceinline__ void vox_charges_lds(const int *vi, const float *__re
 constexpr int kVoxLdsThreads = kChargeThreads;
 constexpr int kVoxSplitAtoms = 512;
 constexpr size_t kVoxLdsBytes = 132 * 1024;  // both masks of one rotation, at most
+inline size_t mask_bytes(int ng) { return 2 * sizeof(uint32_t) * (size_t)mask_words(ng); }
 __global__ void __launch_bounds__(kVoxLdsThreads)
     k_vox_lds(LigandDev L, const float *__restrict__ rot, const int *__restrict__ boff, uint32_t *dmo, uint32_t *cnt,
               int *vidx, int mw, int cw, float *chg, int nt) {
@@ -352,11 +353,12 @@ __global__ void __launch_bounds__(kVoxLdsThreads)
     float *gc = reinterpret_cast<float *>(msk + 2 * mw);
     for (int q = tid; q < 2 * mw; q += kVoxLdsThreads) msk[q] = 0u;
     for (int q = tid; q < ng; q += kVoxLdsThreads) gc[q] = L.gc[q];
-    const float *rb = rot + 9 * ((size_t)(boff ? *boff : 0) + b);
+    __shared__ float coef[9];  // read once (rot may lie in host memory)
+    if (tid < 9) coef[tid] = rot[9 * ((size_t)(boff ? *boff : 0) + b) + tid];
+    __syncthreads();
     float r[9];
 #pragma unroll
-    for (int q = 0; q < 9; q++) r[q] = rb[q];
-    __syncthreads();
+    for (int q = 0; q < 9; q++) r[q] = coef[q];
     // an atom's five planes in one thread share its box; a small ligand's go to five threads, so
     // that the CU's four SIMDs have waves enough
     const int split = L.na <= kVoxSplitAtoms ? 5 : 1;
@@ -396,12 +398,14 @@ __global__ void k_vox_expand(VoxGrid vg, float2 *lg, int ng3) {
 
 }  // namespace
 
+bool voxelizer_reads_once(int ng) { return mask_bytes(ng) <= kVoxLdsBytes; }
+
 hipError_t launch_voxelize(const LigandDev &lig, const float *rot, int B, const VoxScratch &vs, int *vidx,
                            float *chg, hipStream_t s, const int *boff) {
     const int ng = lig.ng, mw = mask_words(ng), cw = count_words(ng);
     const int ng3 = ng * ng * ng;
-    const size_t masks = 2 * sizeof(uint32_t) * (size_t)mw;
-    if (masks <= kVoxLdsBytes) {  // one workgroup per rotation, bits in LDS
+    const size_t masks = mask_bytes(ng);
+    if (voxelizer_reads_once(ng)) {  // one workgroup per rotation, bits in LDS
         // the charges' table beside their list, where it fits into the masks' LDS (or little enough
         // for two workgroups a CU); more atoms than that are counted in memory
         const size_t most = std::max(masks + sizeof(float) * ng, (size_t)64 * 1024);

@@ -68,7 +68,7 @@ int fail(const std::string &msg) {
 constexpr int WZ = 16;   // lines per workgroup, z passes
 constexpr int WY = 16;   // lines per workgroup, y passes
 constexpr int WX = 8;    // kz columns per workgroup in the x pass (plus 8 partner columns)
-constexpr int NT = 256;  // threads per workgroup
+constexpr int kThreads = 256;  // threads per workgroup, where not chosen by the size
 constexpr size_t kDirectResults = 256;  // mdk_dock: as many results go straight to host memory
 
 __device__ __forceinline__ void load_tw(float2 *tw_s, const float2 *tw_g, int ntw) {
@@ -77,6 +77,7 @@ __device__ __forceinline__ void load_tw(float2 *tw_s, const float2 *tw_g, int nt
 
 // ---------------------------------------------------------------- forward z
 // lines: (b, x, y) with x, y < ng; row z < ng of lg sits at z + nd of the FFT line.
+template <int NT>
 __global__ void __launch_bounds__(NT) k_fwd_z(const float2 *__restrict__ lg, float2 *__restrict__ a1,
                                               FftPlan p, const float2 *__restrict__ twg, int ng,
                                               int nd, int nlines) {
@@ -85,8 +86,9 @@ __global__ void __launch_bounds__(NT) k_fwd_z(const float2 *__restrict__ lg, flo
     float2 *tw = sm, *A = sm + p.ntw, *Bf = A + nf * LS;
     load_tw(tw, twg, p.ntw);
     const int line0 = blockIdx.x * WZ;
+    const float inv_nf = 1.0f / (float)nf;
     for (int q = threadIdx.x; q < WZ * nf; q += NT) {
-        const int l = q / nf, z = q % nf;
+        const int l = quot(q, inv_nf), z = q - l * nf;
         float2 v = make_float2(0.f, 0.f);
         if (line0 + l < nlines && z >= nd && z < nd + ng) v = lg[(size_t)(line0 + l) * ng + (z - nd)];
         A[z * LS + l] = v;
@@ -94,13 +96,14 @@ __global__ void __launch_bounds__(NT) k_fwd_z(const float2 *__restrict__ lg, flo
     __syncthreads();
     float2 *res = lds_fft<false>(A, Bf, tw, p, LS, threadIdx.x % WZ, threadIdx.x / WZ, NT / WZ, true);
     for (int q = threadIdx.x; q < WZ * nf; q += NT) {
-        const int l = q / nf, kz = q % nf;
+        const int l = quot(q, inv_nf), kz = q - l * nf;
         if (line0 + l < nlines) a1[(size_t)(line0 + l) * nf + kz] = res[kz * LS + l];
     }
 }
 
 // ---------------------------------------------------------------- forward y
 // block (kz chunk, x, b); rows y < ng of a1 sit at y + nd.
+template <int NT>
 __global__ void __launch_bounds__(NT) k_fwd_y(const float2 *__restrict__ a1, float2 *__restrict__ a2,
                                               FftPlan p, const float2 *__restrict__ twg, int ng,
                                               int nd) {
@@ -127,6 +130,7 @@ __global__ void __launch_bounds__(NT) k_fwd_y(const float2 *__restrict__ a1, flo
 
 // ---------------------------------------------------------------- x pass, receptor
 // plain forward x-FFT of the receptor: rec[kx][ky][kz] (full spectrum)
+template <int NT>
 __global__ void __launch_bounds__(NT) k_fwd_x_plain(const float2 *__restrict__ a2, float2 *__restrict__ rec,
                                                     FftPlan p, const float2 *__restrict__ twg, int ng,
                                                     int nd) {
@@ -154,6 +158,7 @@ __global__ void __launch_bounds__(NT) k_fwd_x_plain(const float2 *__restrict__ a
 // partner columns (-ky, -kz).  Forward x-FFT of all 2*WX, then
 //   Q(k) = (conj(R(k)) L(k) + conj(conj(R(-k)) L(-k))) / 2
 // and an inverse x-FFT of the WX lines of Q.
+template <int NT>
 __global__ void __launch_bounds__(NT) k_x_corr(const float2 *__restrict__ a2, const float2 *__restrict__ rec,
                                                float2 *__restrict__ cc, FftPlan p,
                                                const float2 *__restrict__ twg, int ng, int nd, int H,
@@ -207,6 +212,7 @@ __global__ void __launch_bounds__(NT) k_x_corr(const float2 *__restrict__ a2, co
 }
 
 // ---------------------------------------------------------------- inverse y (in place)
+template <int NT>
 __global__ void __launch_bounds__(NT) k_inv_y(float2 *__restrict__ cc, FftPlan p,
                                               const float2 *__restrict__ twg, int Hp) {
     extern __shared__ float2 sm[];
@@ -230,6 +236,7 @@ __global__ void __launch_bounds__(NT) k_inv_y(float2 *__restrict__ cc, FftPlan p
 // ---------------------------------------------------------------- inverse z + top-t
 // rows r = (b*nf + x)*nf + y; the row's spectrum is Hermitian, only kz <= nf/2 stored.
 // Writes either the real score row (smap) or the row's top-t candidates.
+template <int NT, bool ONE>
 __global__ void __launch_bounds__(NT) k_inv_z_top(const float2 *__restrict__ cc, Cand *__restrict__ cand,
                                                   float *__restrict__ smap, FftPlan p,
                                                   const float2 *__restrict__ twg, int H, int Hp,
@@ -237,11 +244,12 @@ __global__ void __launch_bounds__(NT) k_inv_z_top(const float2 *__restrict__ cc,
     extern __shared__ float2 sm[];
     const int nf = p.n, LS = WZ + 1;
     float2 *tw = sm, *A = sm + p.ntw, *Bf = A + nf * LS;
-    Cand *lists = reinterpret_cast<Cand *>(Bf + nf * LS);  // [WZ][NT/WZ][t]
+    Cand *lists = reinterpret_cast<Cand *>(Bf + nf * LS);  // [WZ][NT/WZ][t]; ONE: [NT/64][WZ]
     load_tw(tw, twg, p.ntw);
     const int row0 = blockIdx.x * WZ;
+    const float inv_h = 1.0f / (float)H;
     for (int q = threadIdx.x; q < WZ * H; q += NT) {
-        const int l = q / H, kz = q % H;
+        const int l = quot(q, inv_h), kz = q - l * H;
         float2 v = make_float2(0.f, 0.f);
         if (row0 + l < nrows) v = cc[(size_t)(row0 + l) * Hp + kz];
         A[kz * LS + l] = v;
@@ -254,6 +262,32 @@ __global__ void __launch_bounds__(NT) k_inv_z_top(const float2 *__restrict__ cc,
     if (smap) {
         if (r < nrows)
             for (int z = jt; z < nf; z += tpl) smap[(size_t)r * nf + z] = res[z * LS + l].x;
+        return;
+    }
+    if (ONE) {
+        // one result: each thread's best, lane exchanges over the wavefront's threads of a line, and
+        // one barrier for the wavefronts
+        Cand m{-INFINITY, kNoIndex};
+        if (r < nrows) {
+            const int rr = r % (nf * nf);
+            for (int z = jt; z < nf; z += tpl) {
+                const float v = res[z * LS + l].x;
+                if (better(v, rr * nf + z, m.key, m.idx)) m = Cand{v, rr * nf + z};
+            }
+        }
+        for (int h = WZ; h < 64; h *= 2) {
+            const Cand o{__shfl_xor(m.key, h, 64), __shfl_xor(m.idx, h, 64)};
+            if (better(o.key, o.idx, m.key, m.idx)) m = o;
+        }
+        if ((threadIdx.x & 63) < WZ) lists[(threadIdx.x >> 6) * WZ + l] = m;
+        __syncthreads();
+        if (threadIdx.x < WZ && r < nrows) {
+            for (int w = 1; w < NT / 64; w++) {
+                const Cand o = lists[w * WZ + l];
+                if (better(o.key, o.idx, m.key, m.idx)) m = o;
+            }
+            cand[r] = m;
+        }
         return;
     }
     // per-thread top-t over its elements; key = value (t == 1) or value / nf^3 (t > 1)
@@ -292,10 +326,10 @@ __global__ void __launch_bounds__(NT) k_inv_z_top(const float2 *__restrict__ cc,
 // value is > 0; t > 1 starts from -99999 and keeps candidates whose normalised value is
 // > -99999 (src/fft_process.cpp:407-446).  Scores are written normalised by nf^3.
 // boff (optional): device word with the batch's first rotation, added to rot_id and out
-__global__ void __launch_bounds__(NT) k_reduce_top(const Cand *__restrict__ cand, mdk_sortscore *__restrict__ out,
+__global__ void __launch_bounds__(kThreads) k_reduce_top(const Cand *__restrict__ cand, mdk_sortscore *__restrict__ out,
                                                    const int *__restrict__ rot_id, const int *__restrict__ boff,
                                                    int lists_per_rot, int t, int nf, float nf3f) {
-    __shared__ Cand lists[NT * MDK_MAXT];
+    __shared__ Cand lists[kThreads * MDK_MAXT];
     const int b = blockIdx.x;
     const int b0 = boff ? *boff : 0;
     const int id = rot_id[b0 + b];  // asked for early: it may lie in host memory
@@ -305,7 +339,7 @@ __global__ void __launch_bounds__(NT) k_reduce_top(const Cand *__restrict__ cand
     if (t == 1) {  // uniform
         // one result: lane exchanges and one barrier in place of sixteen (6.6 -> 2.4 us for one rotation)
         Cand m{-INFINITY, kNoIndex};
-        for (int q = threadIdx.x; q < n; q += NT)
+        for (int q = threadIdx.x; q < n; q += kThreads)
             if (better(src[q].key, src[q].idx, m.key, m.idx)) m = src[q];
         for (int h = 32; h >= 1; h >>= 1) {
             const Cand o{__shfl_xor(m.key, h, 64), __shfl_xor(m.idx, h, 64)};
@@ -314,16 +348,16 @@ __global__ void __launch_bounds__(NT) k_reduce_top(const Cand *__restrict__ cand
         if ((threadIdx.x & 63) == 0) lists[threadIdx.x >> 6] = m;
         __syncthreads();
         if (threadIdx.x == 0)
-            for (int w = 1; w < NT / 64; w++)
+            for (int w = 1; w < kThreads / 64; w++)
                 if (better(lists[w].key, lists[w].idx, lists[0].key, lists[0].idx)) lists[0] = lists[w];
     } else {
         TopList tl;
         tl.init();
-        for (int q = threadIdx.x; q < n; q += NT) tl.push(t, src[q].key, src[q].idx);
+        for (int q = threadIdx.x; q < n; q += kThreads) tl.push(t, src[q].key, src[q].idx);
         tl.store(t, lists + threadIdx.x * t);
         __syncthreads();
-        // tree merge of the NT lists (every thread reaches every barrier)
-        for (int half = NT / 2; half >= 1; half >>= 1) {
+        // tree merge of the kThreads lists (every thread reaches every barrier)
+        for (int half = kThreads / 2; half >= 1; half >>= 1) {
             if (threadIdx.x < half) tl.merge_sorted(t, lists + (threadIdx.x + half) * t);
             __syncthreads();
             if (threadIdx.x < half) tl.store(t, lists + threadIdx.x * t);
@@ -369,9 +403,9 @@ __global__ void k_batch_reset(int *ctl, int base, int step) {
 // The receptor spectrum rec[kx][ky][kz] as the correlation pass reads it: per (kx, ky), each
 // run of 16 columns kz <= nf/2 followed by the 16 values at (-kx, -ky, -kz), 2 Hp values a row
 // (zero past nf/2).
-__global__ void __launch_bounds__(NT) k_rec_pairs(const float2 *__restrict__ rec, float2 *__restrict__ recp, int nf,
+__global__ void __launch_bounds__(kThreads) k_rec_pairs(const float2 *__restrict__ rec, float2 *__restrict__ recp, int nf,
                                                   int Hp) {
-    const int q = blockIdx.x * NT + threadIdx.x, kx = blockIdx.y;
+    const int q = blockIdx.x * kThreads + threadIdx.x, kx = blockIdx.y;
     if (q >= nf * 2 * Hp) return;
     const int ky = q / (2 * Hp), p = q - ky * 2 * Hp, kz = (p >> 5) * 16 + (p & 15);
     float2 v = make_float2(0.f, 0.f);
@@ -392,7 +426,7 @@ __global__ void k_iota(int *p, int first, int n) {
 }
 
 // ---------------------------------------------------------------- 1D test kernel
-__global__ void __launch_bounds__(NT) k_lines(const float2 *__restrict__ in, float2 *__restrict__ out,
+__global__ void __launch_bounds__(kThreads) k_lines(const float2 *__restrict__ in, float2 *__restrict__ out,
                                               FftPlan p, const float2 *__restrict__ twg, int nlines,
                                               int inv) {
     extern __shared__ float2 sm[];
@@ -400,14 +434,14 @@ __global__ void __launch_bounds__(NT) k_lines(const float2 *__restrict__ in, flo
     float2 *tw = sm, *A = sm + p.ntw, *Bf = A + n * LS;
     load_tw(tw, twg, p.ntw);
     const int line0 = blockIdx.x * WZ;
-    for (int q = threadIdx.x; q < WZ * n; q += NT) {
+    for (int q = threadIdx.x; q < WZ * n; q += kThreads) {
         const int l = q / n, e = q % n;
         A[e * LS + l] = (line0 + l < nlines) ? in[(size_t)(line0 + l) * n + e] : make_float2(0.f, 0.f);
     }
     __syncthreads();
-    float2 *res = inv ? lds_fft<true>(A, Bf, tw, p, LS, threadIdx.x % WZ, threadIdx.x / WZ, NT / WZ, true)
-                      : lds_fft<false>(A, Bf, tw, p, LS, threadIdx.x % WZ, threadIdx.x / WZ, NT / WZ, true);
-    for (int q = threadIdx.x; q < WZ * n; q += NT) {
+    float2 *res = inv ? lds_fft<true>(A, Bf, tw, p, LS, threadIdx.x % WZ, threadIdx.x / WZ, kThreads / WZ, true)
+                      : lds_fft<false>(A, Bf, tw, p, LS, threadIdx.x % WZ, threadIdx.x / WZ, kThreads / WZ, true);
+    for (int q = threadIdx.x; q < WZ * n; q += kThreads) {
         const int l = q / n, e = q % n;
         if (line0 + l < nlines) out[(size_t)(line0 + l) * n + e] = res[e * LS + l];
     }
@@ -554,6 +588,31 @@ size_t lds_bytes(const mdk_ctx *c, int lines) {
     return sizeof(float2) * ((size_t)c->plan.ntw + 2 * (size_t)c->nf * (lines + 1));
 }
 
+// LDS of k_inv_z_top<nt, t == 1>
+size_t lds_inv_z(const mdk_ctx *c, int nt, int t) {
+    return lds_bytes(c, WZ) + sizeof(Cand) * (t == 1 ? (size_t)nt / 64 * WZ : (size_t)nt * t);
+}
+
+// Threads per workgroup of the generic passes: their sixteen lines' LDS (98 KB at 360) leaves room for
+// few workgroups on a CU, and those of 256 threads left it with four wavefronts.  Searches with 256, 512
+// and 1024 threads take 7.9, 8.3, 16.3 ms at 130 (four workgroups a CU), 8.3, 7.0, 13.0 at 156 and 10.9,
+// 8.0, 10.6 at 260 (two or three), 19.8, 12.9, 10.4 at 324 (one).  At 360 with 256 threads
+// and integer divisions, 16 rotations took 14.8 ms in the x pass, 11.4 in the inverse z, 5.3 in the inverse
+// y, 4.3 and 2.9 in the forward y and z passes; now 7.3, 4.1, 2.5, 2.0 and 1.0.
+int generic_threads(const mdk_ctx *c) {
+    const size_t lds = lds_bytes(c, 16) + 2048;
+    return lds > 80 * 1024 ? 1024 : lds > 40 * 1024 ? 512 : 256;
+}
+
+template <class F> void by_threads(int nt, F launch) {
+    if (nt == 1024)
+        launch(std::integral_constant<int, 1024>{});
+    else if (nt == 512)
+        launch(std::integral_constant<int, 512>{});
+    else
+        launch(std::integral_constant<int, 256>{});
+}
+
 VoxGrid vox_grid(const mdk_ctx *c, const BatchSlot &S) {
     const int ng = c->ng;
     return VoxGrid{S.vs.dmo, S.d_chg, ng, row_words(ng), mask_words(ng), ng * ng * ng, c->lig.delta};
@@ -601,19 +660,39 @@ int run_fft_pipeline(mdk_ctx *c, BatchSlot &S, int B, float *smap_dev, hipEvent_
     }
     if (!from_lg) HIPCHK(launch_vox_expand(vox_grid(c, S), B, S.d_lg, s));
     const int lines_z = B * ng * ng;
-    k_fwd_z<<<(lines_z + WZ - 1) / WZ, NT, lds_bytes(c, WZ), s>>>(S.d_lg, S.d_a1, c->plan, c->d_tw, ng, nd, lines_z);
+    by_threads(generic_threads(c), [&](auto n) {
+        constexpr int NT = n;
+        k_fwd_z<NT><<<(lines_z + WZ - 1) / WZ, NT, lds_bytes(c, WZ), s>>>(S.d_lg, S.d_a1, c->plan, c->d_tw, ng, nd, lines_z);
+    });
     if (ev) HIPCHK(hipEventRecord(ev[0], s));
-    k_fwd_y<<<dim3((nf + WY - 1) / WY, ng, B), NT, lds_bytes(c, WY), s>>>(S.d_a1, S.d_a2, c->plan, c->d_tw, ng, nd);
+    by_threads(generic_threads(c), [&](auto n) {
+        constexpr int NT = n;
+        k_fwd_y<NT><<<dim3((nf + WY - 1) / WY, ng, B), NT, lds_bytes(c, WY), s>>>(S.d_a1, S.d_a2, c->plan, c->d_tw, ng, nd);
+    });
     if (ev) HIPCHK(hipEventRecord(ev[1], s));
-    k_x_corr<<<dim3(c->Hp / WX, nf, B), NT, lds_bytes(c, 2 * WX), s>>>(S.d_a2, c->d_rec, S.d_cc, c->plan, c->d_tw, ng, nd, c->H, c->Hp);
+    by_threads(generic_threads(c), [&](auto n) {
+        constexpr int NT = n;
+        k_x_corr<NT><<<dim3(c->Hp / WX, nf, B), NT, lds_bytes(c, 2 * WX), s>>>(S.d_a2, c->d_rec, S.d_cc, c->plan, c->d_tw, ng,
+                                                                              nd, c->H, c->Hp);
+    });
     if (ev) HIPCHK(hipEventRecord(ev[2], s));
-    k_inv_y<<<dim3(c->Hp / WY, nf, B), NT, lds_bytes(c, WY), s>>>(S.d_cc, c->plan, c->d_tw, c->Hp);
+    by_threads(generic_threads(c), [&](auto n) {
+        constexpr int NT = n;
+        k_inv_y<NT><<<dim3(c->Hp / WY, nf, B), NT, lds_bytes(c, WY), s>>>(S.d_cc, c->plan, c->d_tw, c->Hp);
+    });
     if (ev) HIPCHK(hipEventRecord(ev[3], s));
     const int rows = B * nf * nf;
     const int tl = smap_dev ? 1 : c->t;  // the score maps need no top-t lists
-    const size_t lds_z = lds_bytes(c, WZ) + sizeof(Cand) * (size_t)NT * tl;
-    k_inv_z_top<<<(rows + WZ - 1) / WZ, NT, lds_z, s>>>(S.d_cc, S.d_cand, smap_dev, c->plan, c->d_tw, c->H, c->Hp, rows, tl,
-                                                       (float)((size_t)nf * nf * nf));
+    const float nf3f = (float)((size_t)nf * nf * nf);
+    by_threads(tl == 1 ? generic_threads(c) : kThreads, [&](auto n) {
+        constexpr int NT = n;
+        if (tl == 1)
+            k_inv_z_top<NT, true><<<(rows + WZ - 1) / WZ, NT, lds_inv_z(c, NT, 1), s>>>(
+                S.d_cc, S.d_cand, smap_dev, c->plan, c->d_tw, c->H, c->Hp, rows, tl, nf3f);
+        else  // longer lists: only kThreads of them fit beside the lines
+            k_inv_z_top<kThreads, false><<<(rows + WZ - 1) / WZ, kThreads, lds_inv_z(c, kThreads, tl), s>>>(
+                S.d_cc, S.d_cand, smap_dev, c->plan, c->d_tw, c->H, c->Hp, rows, tl, nf3f);
+    });
     if (ev) HIPCHK(hipEventRecord(ev[4], s));
     HIPCHK(hipGetLastError());
     return 0;
@@ -635,7 +714,7 @@ int dock_batch(mdk_ctx *c, BatchSlot &S, const float *rot_dev, const int *id_dev
     }
     if (run_fft_pipeline(c, S, B, nullptr, ev ? ev + 2 : nullptr)) return 1;
     const int lists = c->use_pipe ? pipe_cands_per_rotation(nf) : nf * nf;
-    k_reduce_top<<<B, NT, 0, S.stream>>>(S.d_cand, out_dev, id_dev, boff, lists, c->t, nf, (float)((size_t)nf * nf * nf));
+    k_reduce_top<<<B, kThreads, 0, S.stream>>>(S.d_cand, out_dev, id_dev, boff, lists, c->t, nf, (float)((size_t)nf * nf * nf));
     if (ev) HIPCHK(hipEventRecord(ev[7], S.stream));
     HIPCHK(hipGetLastError());
     return 0;
@@ -842,12 +921,19 @@ int mdk_create(int device, int nf, int ng, int na, int t, int max_batch, mdk_ctx
         return bail(fail("mdk_create: event creation failed"));
     // the largest kernel LDS request must fit
     const int tl = std::min(t, MDK_MAXT);  // above, the lists are not used (launch_topt)
-    const size_t lds_max = std::max(lds_bytes(c, 2 * WX), lds_bytes(c, WZ) + sizeof(Cand) * (size_t)NT * tl);
+    const size_t lds_max = std::max(lds_bytes(c, 2 * WX), lds_bytes(c, WZ) + sizeof(Cand) * (size_t)kThreads * tl);
     if (lds_max > 160 * 1024) return bail(fail("mdk_create: nf too large for the LDS-resident passes"));
-    if (allow_lds(k_fwd_z, lds_bytes(c, WZ)) != hipSuccess || allow_lds(k_fwd_y, lds_bytes(c, WY)) != hipSuccess ||
-        allow_lds(k_fwd_x_plain, lds_bytes(c, WY)) != hipSuccess ||
-        allow_lds(k_x_corr, lds_bytes(c, 2 * WX)) != hipSuccess || allow_lds(k_inv_y, lds_bytes(c, WY)) != hipSuccess ||
-        allow_lds(k_inv_z_top, lds_bytes(c, WZ) + sizeof(Cand) * (size_t)NT * tl) != hipSuccess)
+    bool raised = tl == 1 || allow_lds(k_inv_z_top<kThreads, false>, lds_inv_z(c, kThreads, tl)) == hipSuccess;
+    by_threads(generic_threads(c), [&](auto n) {
+        constexpr int NT = n;
+        raised = raised && allow_lds(k_fwd_z<NT>, lds_bytes(c, WZ)) == hipSuccess &&
+                 allow_lds(k_fwd_y<NT>, lds_bytes(c, WY)) == hipSuccess &&
+                 allow_lds(k_fwd_x_plain<NT>, lds_bytes(c, WY)) == hipSuccess &&
+                 allow_lds(k_x_corr<NT>, lds_bytes(c, 2 * WX)) == hipSuccess &&
+                 allow_lds(k_inv_y<NT>, lds_bytes(c, WY)) == hipSuccess &&
+                 allow_lds(k_inv_z_top<NT, true>, lds_inv_z(c, NT, 1)) == hipSuccess;
+    });
+    if (!raised)
         return bail(fail("mdk_create: cannot raise the LDS limit"));
     *out = c;
     return 0;
@@ -906,7 +992,7 @@ int staging(void **buf, size_t &cap, size_t bytes, hipEvent_t &ev) {
 // d_recp from d_rec, on the context's stream
 int pair_receptor(mdk_ctx *c) {
     if (!c->d_recp) return 0;
-    k_rec_pairs<<<dim3((c->nf * 2 * c->Hp + NT - 1) / NT, c->nf), NT, 0, c->stream>>>(c->d_rec, c->d_recp, c->nf, c->Hp);
+    k_rec_pairs<<<dim3((c->nf * 2 * c->Hp + kThreads - 1) / kThreads, c->nf), kThreads, 0, c->stream>>>(c->d_rec, c->d_recp, c->nf, c->Hp);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -918,9 +1004,15 @@ int receptor_transform(mdk_ctx *c, bool wait = true) {
     const size_t ng3 = (size_t)ng * ng * ng;
     HIPCHK(hipMemcpyAsync(c->slot[0].d_lg, c->d_recgrid, sizeof(float2) * ng3, hipMemcpyDeviceToDevice, c->stream));
     const int lines_z = ng * ng;
-    k_fwd_z<<<(lines_z + WZ - 1) / WZ, NT, lds_bytes(c, WZ), c->stream>>>(c->slot[0].d_lg, c->slot[0].d_a1, c->plan, c->d_tw, ng, nd, lines_z);
-    k_fwd_y<<<dim3((nf + WY - 1) / WY, ng, 1), NT, lds_bytes(c, WY), c->stream>>>(c->slot[0].d_a1, c->slot[0].d_a2, c->plan, c->d_tw, ng, nd);
-    k_fwd_x_plain<<<dim3((nf + WY - 1) / WY, nf), NT, lds_bytes(c, WY), c->stream>>>(c->slot[0].d_a2, c->d_rec, c->plan, c->d_tw, ng, nd);
+    by_threads(generic_threads(c), [&](auto n) {
+        constexpr int NT = n;
+        k_fwd_z<NT><<<(lines_z + WZ - 1) / WZ, NT, lds_bytes(c, WZ), c->stream>>>(c->slot[0].d_lg, c->slot[0].d_a1, c->plan,
+                                                                                 c->d_tw, ng, nd, lines_z);
+        k_fwd_y<NT><<<dim3((nf + WY - 1) / WY, ng, 1), NT, lds_bytes(c, WY), c->stream>>>(c->slot[0].d_a1, c->slot[0].d_a2,
+                                                                                         c->plan, c->d_tw, ng, nd);
+        k_fwd_x_plain<NT><<<dim3((nf + WY - 1) / WY, nf), NT, lds_bytes(c, WY), c->stream>>>(c->slot[0].d_a2, c->d_rec, c->plan,
+                                                                                            c->d_tw, ng, nd);
+    });
     HIPCHK(hipGetLastError());
     if (pair_receptor(c)) return 1;
     if (wait) HIPCHK(hipStreamSynchronize(c->stream));
@@ -1137,7 +1229,7 @@ int mdk_dock_grid(mdk_ctx *c, const float *grid_r, const float *grid_i, int rot_
         HIPCHK(launch_topt(S.d_smap, 1, nf, c->t, S.d_tsel, S.d_tkeys, S.d_bout, c->d_bid, nullptr, c->stream));
     } else {
         if (run_fft_pipeline(c, S, 1, nullptr, nullptr, false, true)) return 1;
-        k_reduce_top<<<1, NT, 0, c->stream>>>(S.d_cand, S.d_bout, c->d_bid, nullptr, nf * nf, c->t, nf,
+        k_reduce_top<<<1, kThreads, 0, c->stream>>>(S.d_cand, S.d_bout, c->d_bid, nullptr, nf * nf, c->t, nf,
                                              (float)((size_t)nf * nf * nf));
         HIPCHK(hipGetLastError());
     }
@@ -1643,7 +1735,7 @@ int mdk_fft1d(int device, int n, int count, const float *in, float *out, int sig
         rc = fail("mdk_fft1d: upload failed");
     if (!rc && allow_lds(k_lines, lds) != hipSuccess) rc = fail("mdk_fft1d: cannot raise the LDS limit");
     if (!rc) {
-        k_lines<<<(count + WZ - 1) / WZ, NT, lds>>>(d_in, d_out, p, d_tw, count, sign > 0 ? 1 : 0);
+        k_lines<<<(count + WZ - 1) / WZ, kThreads, lds>>>(d_in, d_out, p, d_tw, count, sign > 0 ? 1 : 0);
         if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess)
             rc = fail("mdk_fft1d: kernel failed");
     }

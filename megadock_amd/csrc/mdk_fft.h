@@ -194,6 +194,10 @@ template <int R, bool INV> struct Dft {
     }
 };
 
+// q / n by the reciprocal inv = 1.0f / n, exact for 0 <= q < 2^20 and n < 2^10 (the quotient of q + 1/2
+// is 1 / 2n or more away from a whole number); the integer division is some thirty instructions
+__device__ __forceinline__ int quot(int q, float inv) { return (int)(((float)q + 0.5f) * inv); }
+
 // One Stockham stage over the lines of a workgroup.  Thread (line, jt) handles
 // butterflies j = jt, jt + tpl, ...  `tw` holds this stage's (R-1)*Ns twiddles
 // exp(-2 pi i r k / (Ns R)), index (r-1)*Ns + k.
@@ -202,8 +206,9 @@ __device__ __forceinline__ void fft_stage(const float2 *__restrict__ in, float2 
                                           const float2 *__restrict__ tw, int N, int Ns, int LS,
                                           int line, int jt, int tpl) {
     const int nr = N / R;
+    const float inv_ns = 1.0f / (float)Ns;
     for (int j = jt; j < nr; j += tpl) {
-        const int k = j % Ns;
+        const int k = j - quot(j, inv_ns) * Ns;
         float2 v[R];
         v[0] = in[j * LS + line];
 #pragma unroll

@@ -75,6 +75,30 @@ __device__ __forceinline__ void load_tw(float2 *tw_s, const float2 *tw_g, int nt
     for (int q = threadIdx.x; q < ntw; q += blockDim.x) tw_s[q] = tw_g[q];
 }
 
+// Rows 0 .. count - 1 of the workgroup's lines into rows first .. of A, U rows a thread at a time: the
+// loads are issued together (one at a time, their latency was most of a pass: a CU holds one or two
+// workgroups of these kernels).  load(r) may be asked for any row below count, by any thread.
+template <int LINES, int NT, int U, class Load>
+__device__ __forceinline__ void load_rows(float2 *A, int LS, int first, int count, Load load) {
+    constexpr int STEP = NT / LINES;
+    const int l = threadIdx.x % LINES;
+    for (int r0 = threadIdx.x / LINES; r0 < count; r0 += U * STEP) {
+        float2 v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = load(min(r0 + u * STEP, count - 1));
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (r0 + u * STEP < count) A[(first + r0 + u * STEP) * LS + l] = v[u];
+    }
+}
+
+// zeros in the rows outside [first, first + count) of n
+template <int LINES, int NT> __device__ __forceinline__ void zero_rows(float2 *A, int LS, int first, int count, int n) {
+    const int l = threadIdx.x % LINES;
+    for (int r = threadIdx.x / LINES; r < n - count; r += NT / LINES)
+        A[(r < first ? r : r + count) * LS + l] = make_float2(0.f, 0.f);
+}
+
 // ---------------------------------------------------------------- forward z
 // lines: (b, x, y) with x, y < ng; row z < ng of lg sits at z + nd of the FFT line.
 template <int NT>
@@ -87,17 +111,29 @@ __global__ void __launch_bounds__(NT) k_fwd_z(const float2 *__restrict__ lg, flo
     load_tw(tw, twg, p.ntw);
     const int line0 = blockIdx.x * WZ;
     const float inv_nf = 1.0f / (float)nf;
-    for (int q = threadIdx.x; q < WZ * nf; q += NT) {
-        const int l = quot(q, inv_nf), z = q - l * nf;
-        float2 v = make_float2(0.f, 0.f);
-        if (line0 + l < nlines && z >= nd && z < nd + ng) v = lg[(size_t)(line0 + l) * ng + (z - nd)];
-        A[z * LS + l] = v;
+    lg += (size_t)line0 * ng;
+    a1 += (size_t)line0 * nf;
+    for (int q = threadIdx.x; q < WZ * (nf - ng); q += NT) {
+        const int r = q / WZ;
+        A[(r < nd ? r : r + ng) * LS + q % WZ] = make_float2(0.f, 0.f);
+    }
+    const float inv_ng = 1.0f / (float)ng;
+    const int have = min(nlines - line0, WZ) * ng;
+    for (int q0 = threadIdx.x; q0 < WZ * ng; q0 += 4 * NT) {
+        float2 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = lg[min(q0 + u * NT, have - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int q = q0 + u * NT, l = quot(q, inv_ng), z = q - l * ng;
+            if (q < WZ * ng) A[(z + nd) * LS + l] = q < have ? v[u] : make_float2(0.f, 0.f);
+        }
     }
     __syncthreads();
     float2 *res = lds_fft<false>(A, Bf, tw, p, LS, threadIdx.x % WZ, threadIdx.x / WZ, NT / WZ, true);
     for (int q = threadIdx.x; q < WZ * nf; q += NT) {
         const int l = quot(q, inv_nf), kz = q - l * nf;
-        if (line0 + l < nlines) a1[(size_t)(line0 + l) * nf + kz] = res[kz * LS + l];
+        if (line0 + l < nlines) a1[l * nf + kz] = res[kz * LS + l];
     }
 }
 
@@ -113,19 +149,18 @@ __global__ void __launch_bounds__(NT) k_fwd_y(const float2 *__restrict__ a1, flo
     load_tw(tw, twg, p.ntw);
     const int kz0 = blockIdx.x * WY, x = blockIdx.y, b = blockIdx.z;
     const float2 *src = a1 + ((size_t)b * ng + x) * ng * nf;
-    for (int q = threadIdx.x; q < WY * nf; q += NT) {
-        const int l = q % WY, y = q / WY;
-        float2 v = make_float2(0.f, 0.f);
-        if (kz0 + l < nf && y >= nd && y < nd + ng) v = src[(size_t)(y - nd) * nf + kz0 + l];
-        A[y * LS + l] = v;
-    }
+    const int l = threadIdx.x % WY;
+    const bool in = kz0 + l < nf;
+    zero_rows<WY, NT>(A, LS, nd, ng, nf);
+    load_rows<WY, NT, 4>(A, LS, nd, ng, [&](int y) {
+        const float2 v = src[y * nf + (in ? kz0 + l : 0)];
+        return in ? v : make_float2(0.f, 0.f);
+    });
     __syncthreads();
     float2 *res = lds_fft<false>(A, Bf, tw, p, LS, threadIdx.x % WY, threadIdx.x / WY, NT / WY, true);
     float2 *dst = a2 + ((size_t)b * ng + x) * nf * nf;
-    for (int q = threadIdx.x; q < WY * nf; q += NT) {
-        const int l = q % WY, ky = q / WY;
-        if (kz0 + l < nf) dst[(size_t)ky * nf + kz0 + l] = res[ky * LS + l];
-    }
+    for (int ky = threadIdx.x / WY; ky < nf; ky += NT / WY)
+        if (in) dst[ky * nf + kz0 + l] = res[ky * LS + l];
 }
 
 // ---------------------------------------------------------------- x pass, receptor
@@ -139,18 +174,17 @@ __global__ void __launch_bounds__(NT) k_fwd_x_plain(const float2 *__restrict__ a
     float2 *tw = sm, *A = sm + p.ntw, *Bf = A + nf * LS;
     load_tw(tw, twg, p.ntw);
     const int kz0 = blockIdx.x * WY, ky = blockIdx.y;
-    for (int q = threadIdx.x; q < WY * nf; q += NT) {
-        const int l = q % WY, x = q / WY;
-        float2 v = make_float2(0.f, 0.f);
-        if (kz0 + l < nf && x >= nd && x < nd + ng) v = a2[((size_t)(x - nd) * nf + ky) * nf + kz0 + l];
-        A[x * LS + l] = v;
-    }
+    const int l = threadIdx.x % WY;
+    const bool in = kz0 + l < nf;
+    zero_rows<WY, NT>(A, LS, nd, ng, nf);
+    load_rows<WY, NT, 4>(A, LS, nd, ng, [&](int x) {
+        const float2 v = a2[(x * nf + ky) * nf + (in ? kz0 + l : 0)];
+        return in ? v : make_float2(0.f, 0.f);
+    });
     __syncthreads();
     float2 *res = lds_fft<false>(A, Bf, tw, p, LS, threadIdx.x % WY, threadIdx.x / WY, NT / WY, true);
-    for (int q = threadIdx.x; q < WY * nf; q += NT) {
-        const int l = q % WY, kx = q / WY;
-        if (kz0 + l < nf) rec[((size_t)kx * nf + ky) * nf + kz0 + l] = res[kx * LS + l];
-    }
+    for (int kx = threadIdx.x / WY; kx < nf; kx += NT / WY)
+        if (in) rec[(kx * nf + ky) * nf + kz0 + l] = res[kx * LS + l];
 }
 
 // ---------------------------------------------------------------- x pass, docking
@@ -170,28 +204,39 @@ __global__ void __launch_bounds__(NT) k_x_corr(const float2 *__restrict__ a2, co
     const int c = blockIdx.x, ky = blockIdx.y, b = blockIdx.z;
     const int kyp = (nf - ky) % nf;
     const float2 *src = a2 + (size_t)b * ng * nf * nf;
-    for (int q = threadIdx.x; q < 2 * WX * nf; q += NT) {
-        const int l = q % (2 * WX), x = q / (2 * WX);
-        const int kz = c * WX + (l % WX);
-        float2 v = make_float2(0.f, 0.f);
-        if (kz < H && x >= nd && x < nd + ng) {
-            if (l < WX) v = src[((size_t)(x - nd) * nf + ky) * nf + kz];
-            else v = src[((size_t)(x - nd) * nf + kyp) * nf + (nf - kz) % nf];
-        }
-        A[x * LS + l] = v;
+    {
+        const int l = threadIdx.x % (2 * WX), kz = c * WX + l % WX;
+        const bool in = kz < H;
+        const int col = !in ? 0 : l < WX ? ky * nf + kz : kyp * nf + (kz ? nf - kz : 0);
+        zero_rows<2 * WX, NT>(A, LS, nd, ng, nf);
+        load_rows<2 * WX, NT, 4>(A, LS, nd, ng, [&](int x) {
+            const float2 v = src[x * nf * nf + col];
+            return in ? v : make_float2(0.f, 0.f);
+        });
+    }
+    // the receptor's values are asked for before the transform that they wait for
+    const int l = threadIdx.x % WX, kz = c * WX + l;
+    const int col = kz < H ? ky * nf + kz : 0, colp = kz < H ? kyp * nf + (kz ? nf - kz : 0) : 0;
+    constexpr int KR = 5;  // rows a thread: nf <= KR * NT / WX (generic_threads)
+    float2 ra[KR], rb[KR];
+#pragma unroll
+    for (int h = 0; h < KR; h++) {
+        const int kx = min((int)threadIdx.x / WX + h * (NT / WX), nf - 1);
+        ra[h] = rec[kx * nf * nf + col];
+        rb[h] = rec[(kx ? nf - kx : 0) * nf * nf + colp];
     }
     __syncthreads();
     float2 *L = lds_fft<false>(A, Bf, tw, p, LS, threadIdx.x % (2 * WX), threadIdx.x / (2 * WX),
                                NT / (2 * WX), true);
     float2 *Qb = (L == A) ? Bf : A;
-    for (int q = threadIdx.x; q < WX * nf; q += NT) {
-        const int l = q % WX, kx = q / WX;
-        const int kz = c * WX + l;
+#pragma unroll
+    for (int h = 0; h < KR; h++) {
+        const int kx = threadIdx.x / WX + h * (NT / WX);
+        if (kx >= nf) break;
         float2 Q = make_float2(0.f, 0.f);
         if (kz < H) {
-            const int kxp = (nf - kx) % nf, kzp = (nf - kz) % nf;
-            const float2 r1 = rec[((size_t)kx * nf + ky) * nf + kz];
-            const float2 r2 = rec[((size_t)kxp * nf + kyp) * nf + kzp];
+            const int kxp = kx ? nf - kx : 0;
+            const float2 r1 = ra[h], r2 = rb[h];
             const float2 l1 = L[kx * LS + l], l2 = L[kxp * LS + WX + l];
             // conj(r1) * l1 and conj(r2) * l2
             const float2 p1 = make_float2(r1.x * l1.x + r1.y * l1.y, r1.x * l1.y - r1.y * l1.x);
@@ -204,11 +249,8 @@ __global__ void __launch_bounds__(NT) k_x_corr(const float2 *__restrict__ a2, co
     float2 *other = (Qb == A) ? Bf : A;
     float2 *res = lds_fft<true>(Qb, other, tw, p, LS, threadIdx.x % WX, threadIdx.x / WX, NT / WX, true);
     float2 *dst = cc + (size_t)b * nf * nf * Hp;
-    for (int q = threadIdx.x; q < WX * nf; q += NT) {
-        const int l = q % WX, x = q / WX;
-        const int kz = c * WX + l;
-        if (kz < Hp) dst[((size_t)x * nf + ky) * Hp + kz] = res[x * LS + l];
-    }
+    for (int x = threadIdx.x / WX; x < nf; x += NT / WX)
+        if (kz < Hp) dst[(x * nf + ky) * Hp + kz] = res[x * LS + l];
 }
 
 // ---------------------------------------------------------------- inverse y (in place)
@@ -221,16 +263,11 @@ __global__ void __launch_bounds__(NT) k_inv_y(float2 *__restrict__ cc, FftPlan p
     load_tw(tw, twg, p.ntw);
     const int kz0 = blockIdx.x * WY, x = blockIdx.y, b = blockIdx.z;
     float2 *base = cc + ((size_t)b * nf + x) * nf * Hp;
-    for (int q = threadIdx.x; q < WY * nf; q += NT) {
-        const int l = q % WY, ky = q / WY;
-        A[ky * LS + l] = base[(size_t)ky * Hp + kz0 + l];
-    }
+    const int l = threadIdx.x % WY;
+    load_rows<WY, NT, 6>(A, LS, 0, nf, [&](int ky) { return base[ky * Hp + kz0 + l]; });
     __syncthreads();
     float2 *res = lds_fft<true>(A, Bf, tw, p, LS, threadIdx.x % WY, threadIdx.x / WY, NT / WY, true);
-    for (int q = threadIdx.x; q < WY * nf; q += NT) {
-        const int l = q % WY, y = q / WY;
-        base[(size_t)y * Hp + kz0 + l] = res[y * LS + l];
-    }
+    for (int y = threadIdx.x / WY; y < nf; y += NT / WY) base[y * Hp + kz0 + l] = res[y * LS + l];
 }
 
 // ---------------------------------------------------------------- inverse z + top-t
@@ -248,12 +285,24 @@ __global__ void __launch_bounds__(NT) k_inv_z_top(const float2 *__restrict__ cc,
     load_tw(tw, twg, p.ntw);
     const int row0 = blockIdx.x * WZ;
     const float inv_h = 1.0f / (float)H;
-    for (int q = threadIdx.x; q < WZ * H; q += NT) {
-        const int l = quot(q, inv_h), kz = q - l * H;
-        float2 v = make_float2(0.f, 0.f);
-        if (row0 + l < nrows) v = cc[(size_t)(row0 + l) * Hp + kz];
-        A[kz * LS + l] = v;
-        if (kz >= 1 && nf - kz > kz) A[(nf - kz) * LS + l] = make_float2(v.x, -v.y);
+    cc += (size_t)row0 * Hp;
+    const int have = min(nrows - row0, WZ);
+    for (int q0 = threadIdx.x; q0 < WZ * H; q0 += 3 * NT) {
+        float2 v[3];
+#pragma unroll
+        for (int u = 0; u < 3; u++) {
+            const int q = min(q0 + u * NT, WZ * H - 1), l = quot(q, inv_h);
+            v[u] = cc[min(l, have - 1) * Hp + (q - l * H)];
+        }
+#pragma unroll
+        for (int u = 0; u < 3; u++) {
+            const int q = q0 + u * NT;
+            if (q >= WZ * H) break;
+            const int l = quot(q, inv_h), kz = q - l * H;
+            if (l >= have) v[u] = make_float2(0.f, 0.f);
+            A[kz * LS + l] = v[u];
+            if (kz >= 1 && nf - kz > kz) A[(nf - kz) * LS + l] = make_float2(v[u].x, -v[u].y);
+        }
     }
     __syncthreads();
     float2 *res = lds_fft<true>(A, Bf, tw, p, LS, threadIdx.x % WZ, threadIdx.x / WZ, NT / WZ, true);
@@ -598,10 +647,10 @@ size_t lds_inv_z(const mdk_ctx *c, int nt, int t) {
 // and 1024 threads take 7.9, 8.3, 16.3 ms at 130 (four workgroups a CU), 8.3, 7.0, 13.0 at 156 and 10.9,
 // 8.0, 10.6 at 260 (two or three), 19.8, 12.9, 10.4 at 324 (one).  At 360 with 256 threads
 // and integer divisions, 16 rotations took 14.8 ms in the x pass, 11.4 in the inverse z, 5.3 in the inverse
-// y, 4.3 and 2.9 in the forward y and z passes; now 7.3, 4.1, 2.5, 2.0 and 1.0.
+// y, 4.3 and 2.9 in the forward y and z passes; now 6.5, 3.8, 2.1, 1.8 and 0.9.
 int generic_threads(const mdk_ctx *c) {
     const size_t lds = lds_bytes(c, 16) + 2048;
-    return lds > 80 * 1024 ? 1024 : lds > 40 * 1024 ? 512 : 256;
+    return lds > 80 * 1024 || c->nf > 320 ? 1024 : lds > 40 * 1024 || c->nf > 160 ? 512 : 256;
 }
 
 template <class F> void by_threads(int nt, F launch) {
@@ -922,7 +971,7 @@ int mdk_create(int device, int nf, int ng, int na, int t, int max_batch, mdk_ctx
     // the largest kernel LDS request must fit
     const int tl = std::min(t, MDK_MAXT);  // above, the lists are not used (launch_topt)
     const size_t lds_max = std::max(lds_bytes(c, 2 * WX), lds_bytes(c, WZ) + sizeof(Cand) * (size_t)kThreads * tl);
-    if (lds_max > 160 * 1024) return bail(fail("mdk_create: nf too large for the LDS-resident passes"));
+    if (lds_max > 160 * 1024 || nf > 640) return bail(fail("mdk_create: nf too large for the LDS-resident passes"));
     bool raised = tl == 1 || allow_lds(k_inv_z_top<kThreads, false>, lds_inv_z(c, kThreads, tl)) == hipSuccess;
     by_threads(generic_threads(c), [&](auto n) {
         constexpr int NT = n;

@@ -101,8 +101,9 @@ template <int LINES, int NT> __device__ __forceinline__ void zero_rows(float2 *A
 
 // ---------------------------------------------------------------- forward z
 // lines: (b, x, y) with x, y < ng; row z < ng of lg sits at z + nd of the FFT line.
-template <int NT>
-__global__ void __launch_bounds__(NT) k_fwd_z(const float2 *__restrict__ lg, float2 *__restrict__ a1,
+// VOX: the lines of a voxelized batch, read from its masks and charges; else of the grids lg.
+template <int NT, bool VOX>
+__global__ void __launch_bounds__(NT) k_fwd_z(const float2 *__restrict__ lg, VoxGrid vg, float2 *__restrict__ a1,
                                               FftPlan p, const float2 *__restrict__ twg, int ng,
                                               int nd, int nlines) {
     extern __shared__ float2 sm[];
@@ -111,7 +112,7 @@ __global__ void __launch_bounds__(NT) k_fwd_z(const float2 *__restrict__ lg, flo
     load_tw(tw, twg, p.ntw);
     const int line0 = blockIdx.x * WZ;
     const float inv_nf = 1.0f / (float)nf;
-    lg += (size_t)line0 * ng;
+    if (!VOX) lg += (size_t)line0 * ng;
     a1 += (size_t)line0 * nf;
     for (int q = threadIdx.x; q < WZ * (nf - ng); q += NT) {
         const int r = q / WZ;
@@ -122,7 +123,15 @@ __global__ void __launch_bounds__(NT) k_fwd_z(const float2 *__restrict__ lg, flo
     for (int q0 = threadIdx.x; q0 < WZ * ng; q0 += 4 * NT) {
         float2 v[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) v[u] = lg[min(q0 + u * NT, have - 1)];
+        for (int u = 0; u < 4; u++) {
+            if (VOX) {
+                const int q = q0 + u * NT, l = quot(q, inv_ng), line = line0 + l;
+                v[u] = make_float2(0.f, 0.f);
+                if (q < have) v[u] = vox_take(vg, line / (ng * ng), line % (ng * ng), q - l * ng);
+            } else {
+                v[u] = lg[min(q0 + u * NT, have - 1)];
+            }
+        }
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const int q = q0 + u * NT, l = quot(q, inv_ng), z = q - l * ng;
@@ -388,7 +397,16 @@ __global__ void __launch_bounds__(kThreads) k_reduce_top(const Cand *__restrict_
     if (t == 1) {  // uniform
         // one result: lane exchanges and one barrier in place of sixteen (6.6 -> 2.4 us for one rotation)
         Cand m{-INFINITY, kNoIndex};
-        for (int q = threadIdx.x; q < n; q += kThreads)
+        int q = threadIdx.x;
+        for (; q + 7 * kThreads < n; q += 8 * kThreads) {  // long lists (a row each): eight loads in flight
+            Cand e[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) e[u] = src[q + u * kThreads];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                if (better(e[u].key, e[u].idx, m.key, m.idx)) m = e[u];
+        }
+        for (; q < n; q += kThreads)
             if (better(src[q].key, src[q].idx, m.key, m.idx)) m = src[q];
         for (int h = 32; h >= 1; h >>= 1) {
             const Cand o{__shfl_xor(m.key, h, 64), __shfl_xor(m.idx, h, 64)};
@@ -707,11 +725,15 @@ int run_fft_pipeline(mdk_ctx *c, BatchSlot &S, int B, float *smap_dev, hipEvent_
         HIPCHK(pipe_run(nf, a));
         return 0;
     }
-    if (!from_lg) HIPCHK(launch_vox_expand(vox_grid(c, S), B, S.d_lg, s));
     const int lines_z = B * ng * ng;
     by_threads(generic_threads(c), [&](auto n) {
         constexpr int NT = n;
-        k_fwd_z<NT><<<(lines_z + WZ - 1) / WZ, NT, lds_bytes(c, WZ), s>>>(S.d_lg, S.d_a1, c->plan, c->d_tw, ng, nd, lines_z);
+        if (from_lg)
+            k_fwd_z<NT, false><<<(lines_z + WZ - 1) / WZ, NT, lds_bytes(c, WZ), s>>>(S.d_lg, VoxGrid{}, S.d_a1, c->plan, c->d_tw,
+                                                                                    ng, nd, lines_z);
+        else
+            k_fwd_z<NT, true><<<(lines_z + WZ - 1) / WZ, NT, lds_bytes(c, WZ), s>>>(nullptr, vox_grid(c, S), S.d_a1, c->plan,
+                                                                                   c->d_tw, ng, nd, lines_z);
     });
     if (ev) HIPCHK(hipEventRecord(ev[0], s));
     by_threads(generic_threads(c), [&](auto n) {
@@ -975,7 +997,8 @@ int mdk_create(int device, int nf, int ng, int na, int t, int max_batch, mdk_ctx
     bool raised = tl == 1 || allow_lds(k_inv_z_top<kThreads, false>, lds_inv_z(c, kThreads, tl)) == hipSuccess;
     by_threads(generic_threads(c), [&](auto n) {
         constexpr int NT = n;
-        raised = raised && allow_lds(k_fwd_z<NT>, lds_bytes(c, WZ)) == hipSuccess &&
+        raised = raised && allow_lds(k_fwd_z<NT, false>, lds_bytes(c, WZ)) == hipSuccess &&
+                 allow_lds(k_fwd_z<NT, true>, lds_bytes(c, WZ)) == hipSuccess &&
                  allow_lds(k_fwd_y<NT>, lds_bytes(c, WY)) == hipSuccess &&
                  allow_lds(k_fwd_x_plain<NT>, lds_bytes(c, WY)) == hipSuccess &&
                  allow_lds(k_x_corr<NT>, lds_bytes(c, 2 * WX)) == hipSuccess &&
@@ -1055,8 +1078,8 @@ int receptor_transform(mdk_ctx *c, bool wait = true) {
     const int lines_z = ng * ng;
     by_threads(generic_threads(c), [&](auto n) {
         constexpr int NT = n;
-        k_fwd_z<NT><<<(lines_z + WZ - 1) / WZ, NT, lds_bytes(c, WZ), c->stream>>>(c->slot[0].d_lg, c->slot[0].d_a1, c->plan,
-                                                                                 c->d_tw, ng, nd, lines_z);
+        k_fwd_z<NT, false><<<(lines_z + WZ - 1) / WZ, NT, lds_bytes(c, WZ), c->stream>>>(c->slot[0].d_lg, VoxGrid{}, c->slot[0].d_a1,
+                                                                                        c->plan, c->d_tw, ng, nd, lines_z);
         k_fwd_y<NT><<<dim3((nf + WY - 1) / WY, ng, 1), NT, lds_bytes(c, WY), c->stream>>>(c->slot[0].d_a1, c->slot[0].d_a2,
                                                                                          c->plan, c->d_tw, ng, nd);
         k_fwd_x_plain<NT><<<dim3((nf + WY - 1) / WY, nf), NT, lds_bytes(c, WY), c->stream>>>(c->slot[0].d_a2, c->d_rec, c->plan,

@@ -26,19 +26,18 @@ __host__ __device__ inline int row_words(int ng) { return (ng + 31) / 32; }
 inline int mask_words(int ng) { return ng * ng * row_words(ng); }
 // per-voxel atom counts, two 16-bit counters per word (ligands have < 65536 atoms)
 inline int count_words(int ng) { return (ng * ng * ng + 1) / 2; }
-// scratch words per rotation: core + surface masks, delta + value-1 masks, counts
-inline size_t vox_scratch_words(int ng) { return 4 * (size_t)mask_words(ng) + count_words(ng); }
+// scratch words per rotation: delta + value-1 masks, counts
+inline size_t vox_scratch_words(int ng) { return 2 * (size_t)mask_words(ng) + count_words(ng); }
 
 // Voxelization scratch of a context, laid out for max_batch rotations:
-//   cs  [b][2][mask_words]  core and surface bits (cleared per batch)
 //   dmo [b][2][mask_words]  delta mask D and value-1 mask O (written per batch)
 //   cnt [b][count_words]    atom counts per voxel, zero between batches
 struct VoxScratch {
-    uint32_t *cs, *dmo, *cnt;
+    uint32_t *dmo, *cnt;
 };
 inline VoxScratch vox_scratch(uint32_t *base, int max_batch, int ng) {
     const size_t mw = mask_words(ng);
-    return VoxScratch{base, base + 2 * mw * max_batch, base + 4 * mw * max_batch};
+    return VoxScratch{base, base + 2 * mw * max_batch};
 }
 
 // A batch of ligand grids as the FFT passes read them: shape value delta where D is set,

@@ -39,19 +39,13 @@ __device__ __forceinline__ void rotate_atom(const LigandDev &L, const float *r, 
     Z = r[6] * x + r[7] * y + r[8] * z;
 }
 
-__global__ void k_clear(uint32_t *p, size_t n) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x)
-        p[i] = 0u;
-}
-
 // Planes (atom's voxel) + d0 .. + d1 - 1 of atom l's box, -2 <= d0 < d1 <= 3: its core/surface bits
-// into cb/sb (global or LDS masks of one rotation); gc: the grid's coordinates.  Bound by its
+// into cb/sb (LDS masks of the grid's planes i0 .. i1 - 1); gc: the grid's coordinates.  Bound by its
 // vector instructions (the LDS form has one workgroup's waves on one CU): the box's ten squared
 // coordinate differences are formed once, the tests of a row gather into five bits, and a row's
 // run is those bits shifted into the word of the box's first column.
 __device__ __forceinline__ void vox_planes(const LigandDev &L, const float *gc, float X, float Y, float Z, int l, int d0,
-                                           int d1, uint32_t *cb, uint32_t *sb) {
+                                           int d1, uint32_t *cb, uint32_t *sb, int i0, int i1) {
     const int ng = L.ng, rw = row_words(ng);
     const float h = (float)(ng / 2);
     // (a voxel far outside has the same empty box as one 3 outside)
@@ -72,11 +66,11 @@ __device__ __forceinline__ void vox_planes(const LigandDev &L, const float *gc, 
     const int w = ka >> 5, sh = ka & 31;
     for (int di = d0; di < d1; di++) {
         const int i = i2 + di;
-        if (i < 0 || i >= ng) continue;
+        if (i < i0 || i >= i1) continue;
         const float dx = X - gc[i];
         const float xd = dx * dx;
         if (xd > rc2) continue;  // rs2 <= rc2, so neither sphere reaches this plane
-        const int row0 = (i * ng + j2 - 2) * rw + w;
+        const int row0 = ((i - i0) * ng + j2 - 2) * rw + w;
 #pragma unroll
         for (int p = 0; p < 5; p++) {
             const int j = j2 - 2 + p;
@@ -106,32 +100,11 @@ __device__ __forceinline__ void vox_planes(const LigandDev &L, const float *gc, 
 }
 
 // the voxel that holds an atom's charge
-__device__ __forceinline__ int charge_voxel(const LigandDev &L, float X, float Y, float Z) {
-    const int ng = L.ng;
-    const int ci = max(0, min(ng - 1, (int)((X + L.pad) / L.gw)));
-    const int cj = max(0, min(ng - 1, (int)((Y + L.pad) / L.gw)));
-    const int ck = max(0, min(ng - 1, (int)((Z + L.pad) / L.gw)));
-    return (ci * ng + cj) * ng + ck;
+__device__ __forceinline__ int charge_row(const LigandDev &L, float X) {
+    return max(0, min(L.ng - 1, (int)((X + L.pad) / L.gw)));
 }
-
-// one thread per (atom, rotation): core/surface bits, the charge voxel and its atom count
-// boff (optional): device word holding the batch's first row of rot
-__global__ void k_vox_atoms(LigandDev L, const float *__restrict__ rot, const int *__restrict__ boff, uint32_t *cs,
-                            uint32_t *cnt, int *vidx, int mw, int cw) {
-    const int l = blockIdx.x * blockDim.x + threadIdx.x;
-    const int b = blockIdx.y;
-    if (l >= L.na) return;
-    const float *rb = rot + 9 * ((size_t)(boff ? *boff : 0) + b);
-    float r[9];
-#pragma unroll
-    for (int q = 0; q < 9; q++) r[q] = rb[q];
-    uint32_t *cb = cs + (size_t)b * 2 * mw;  // core bits
-    float X, Y, Z;
-    rotate_atom(L, r, l, X, Y, Z);
-    vox_planes(L, L.gc, X, Y, Z, l, -2, 3, cb, cb + mw);
-    const int v = charge_voxel(L, X, Y, Z);
-    vidx[(size_t)b * L.na + l] = v;
-    atomicAdd(&cnt[(size_t)b * cw + (v >> 1)], 1u << (16 * (v & 1)));
+__device__ __forceinline__ int charge_voxel(const LigandDev &L, float X, float Y, float Z) {
+    return (charge_row(L, X) * L.ng + charge_row(L, Y)) * L.ng + charge_row(L, Z);
 }
 
 // bits k = 32 w + s of word w with lo <= k <= hi
@@ -143,12 +116,12 @@ __device__ __forceinline__ uint32_t range_bits(int w, int lo, int hi) {
 }
 
 struct MaskRows {
-    const uint32_t *m;
-    int ng, rw;
+    const uint32_t *m;  // from plane i0 on
+    int ng, rw, i0;
     // word w of row (i, j); zero outside the grid
     __device__ __forceinline__ uint32_t at(int i, int j, int w) const {
         if (i < 0 || i >= ng || j < 0 || j >= ng || w < 0 || w >= rw) return 0u;
-        return m[(i * ng + j) * rw + w];
+        return m[((i - i0) * ng + j) * rw + w];
     }
 };
 
@@ -184,19 +157,6 @@ __device__ __forceinline__ void vox_mask_word(const MaskRows &C, const MaskRows 
     }
     dq = d;
     oq = o;
-}
-
-// one thread per (row word, rotation): the delta mask D and the value-1 mask O
-__global__ void k_vox_masks(const uint32_t *__restrict__ cs, uint32_t *dmo, int ng, int mw, float delta) {
-    const int rw = row_words(ng);
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    const int b = blockIdx.y;
-    if (q >= mw) return;
-    const MaskRows C{cs + (size_t)b * 2 * mw, ng, rw}, S{cs + (size_t)b * 2 * mw + mw, ng, rw};
-    uint32_t d, o;
-    vox_mask_word(C, S, q, ng, delta, d, o);
-    dmo[(size_t)b * 2 * mw + q] = d;
-    dmo[(size_t)b * 2 * mw + mw + q] = o;
 }
 
 // Charges of the atoms nearest to each voxel, summed in atom order from +0.0f
@@ -336,8 +296,7 @@ __device__ __forceinline__ void vox_charges_lds(const int *vi, const float *__re
 
 // One workgroup per rotation with its core and surface bits in LDS (grids whose masks
 // fit): atom runs by LDS atomics, then the D and O words straight to dmo and, if nt > 0, the
-// charges by a table of nt entries (else k_vox_charge follows).  Replaces k_clear + k_vox_atoms +
-// k_vox_masks + k_vox_charge where it fits.  For one rotation it is a chain of dependent steps in
+// charges by a table of nt entries (else k_vox_charge follows).  For one rotation it is a chain of dependent steps in
 // one workgroup: with a thread per atom walking five planes, the grid's coordinates loaded from
 // memory inside its loops, a ligand of 336 atoms took 21.6 us and its charges a launch of 4.2 us.
 constexpr int kVoxLdsThreads = kChargeThreads;
@@ -366,7 +325,7 @@ __global__ void __launch_bounds__(kVoxLdsThreads)
         const int l = q / split, d = q - split * l;
         float X, Y, Z;
         rotate_atom(L, r, l, X, Y, Z);
-        vox_planes(L, gc, X, Y, Z, l, d - 2, split == 1 ? 3 : d - 1, msk, msk + mw);
+        vox_planes(L, gc, X, Y, Z, l, d - 2, split == 1 ? 3 : d - 1, msk, msk + mw, 0, ng);
         if (d == 0) {
             const int v = charge_voxel(L, X, Y, Z);
             vidx[(size_t)b * L.na + l] = v;
@@ -374,7 +333,7 @@ __global__ void __launch_bounds__(kVoxLdsThreads)
         }
     }
     __syncthreads();
-    const MaskRows C{msk, ng, row_words(ng)}, S{msk + mw, ng, row_words(ng)};
+    const MaskRows C{msk, ng, row_words(ng), 0}, S{msk + mw, ng, row_words(ng), 0};
     uint32_t *db = dmo + (size_t)b * 2 * mw;
     for (int q = tid; q < mw; q += kVoxLdsThreads) {
         uint32_t d, o;
@@ -386,6 +345,69 @@ __global__ void __launch_bounds__(kVoxLdsThreads)
     __syncthreads();  // the masks are read
     vox_charges_lds(vidx + (size_t)b * L.na, L.charge, chg + (size_t)b * ng * ng * ng, L.na, msk,
                     reinterpret_cast<float *>(msk + nt), nt, reinterpret_cast<int2 *>(msk + 2 * nt));
+}
+
+// Larger grids: a workgroup takes `planes` planes of a rotation's D and O words, with the core and surface
+// bits of two planes more on each side (what the rules reach) in LDS, and goes through the ligand for the
+// atoms that touch them: every kSlabAtoms atoms it lists those whose box or charge lies there, then sets
+// their bits.  Masks in memory (cleared, set by up to
+// 55 atomics an atom, read back with their neighbours) made 768 rotations take 76.5 ms at 256^3 and 82.0
+// at 216^3; with slabs 71.6 and 79.0.
+constexpr int kSlabAtoms = 4096;
+__global__ void __launch_bounds__(kVoxLdsThreads)
+    k_vox_slab(LigandDev L, const float *__restrict__ rot, const int *__restrict__ boff, uint32_t *dmo, uint32_t *cnt,
+               int *vidx, int mw, int cw, int planes) {
+    extern __shared__ uint32_t msk[];
+    __shared__ uint16_t list[kSlabAtoms];
+    __shared__ int nlist;
+    const int b = blockIdx.y, tid = threadIdx.x, ng = L.ng, rw = row_words(ng);
+    const int p0 = blockIdx.x * planes, p1 = min(p0 + planes, ng);
+    const int i0 = max(p0 - 2, 0), i1 = min(p1 + 2, ng), nw = (i1 - i0) * ng * rw;
+    uint32_t *core = msk, *surf = msk + nw;
+    float *gc = reinterpret_cast<float *>(msk + 2 * nw);
+    __shared__ float coef[9];
+    if (tid < 9) coef[tid] = rot[9 * ((size_t)(boff ? *boff : 0) + b) + tid];
+    for (int q = tid; q < 2 * nw; q += kVoxLdsThreads) msk[q] = 0u;
+    for (int q = tid; q < ng; q += kVoxLdsThreads) gc[q] = L.gc[q];
+    if (tid == 0) nlist = 0;
+    __syncthreads();
+    float r[9];
+#pragma unroll
+    for (int q = 0; q < 9; q++) r[q] = coef[q];
+    const float h = (float)(ng / 2);
+    for (int l0 = 0; l0 < L.na; l0 += kSlabAtoms) {
+        for (int l = l0 + tid; l < min(l0 + kSlabAtoms, L.na); l += kVoxLdsThreads) {
+            float X, Y, Z;
+            rotate_atom(L, r, l, X, Y, Z);
+            const int i2 = min(max((int)(X / L.gw + h), -3), ng + 2), ci = charge_row(L, X);
+            if ((i2 + 2 >= i0 && i2 - 2 < i1) || (ci >= p0 && ci < p1)) list[atomicAdd(&nlist, 1)] = (uint16_t)(l - l0);
+        }
+        __syncthreads();
+        const int n = nlist;
+        for (int q = tid; q < n; q += kVoxLdsThreads) {
+            const int l = l0 + list[q];
+            float X, Y, Z;
+            rotate_atom(L, r, l, X, Y, Z);
+            vox_planes(L, gc, X, Y, Z, l, -2, 3, core, surf, i0, i1);
+            const int ci = charge_row(L, X);
+            if (ci >= p0 && ci < p1) {
+                const int v = charge_voxel(L, X, Y, Z);
+                vidx[(size_t)b * L.na + l] = v;
+                atomicAdd(&cnt[(size_t)b * cw + (v >> 1)], 1u << (16 * (v & 1)));
+            }
+        }
+        __syncthreads();  // the list is read; its count too
+        if (tid == 0) nlist = 0;
+        __syncthreads();
+    }
+    const MaskRows C{core, ng, rw, i0}, S{surf, ng, rw, i0};
+    uint32_t *db = dmo + (size_t)b * 2 * mw;
+    for (int q = p0 * ng * rw + tid; q < p1 * ng * rw; q += kVoxLdsThreads) {
+        uint32_t d, o;
+        vox_mask_word(C, S, q, ng, L.delta, d, o);
+        db[q] = d;
+        db[mw + q] = o;
+    }
 }
 
 // grids as (grid_r, grid_i) pairs; clears the charge grid it reads
@@ -417,11 +439,14 @@ hipError_t launch_voxelize(const LigandDev &lig, const float *rot, int B, const 
         k_vox_lds<<<B, kVoxLdsThreads, lds, s>>>(lig, rot, boff, vs.dmo, vs.cnt, vidx, mw, cw, chg, nt);
         if (!nt) k_vox_charge<<<B, kChargeThreads, 0, s>>>(vidx, vs.cnt, lig.charge, chg, lig.na, ng3, cw);
     } else {
-        const size_t nclear = 2 * (size_t)B * mw;  // core and surface bits; counts are kept zero
-        k_clear<<<dim3((unsigned)((nclear + 255) / 256 < 65535 ? (nclear + 255) / 256 : 65535)), 256, 0, s>>>(vs.cs,
-                                                                                                       nclear);
-        k_vox_atoms<<<dim3((lig.na + 127) / 128, B), 128, 0, s>>>(lig, rot, boff, vs.cs, vs.cnt, vidx, mw, cw);
-        k_vox_masks<<<dim3((mw + 255) / 256, B), 256, 0, s>>>(vs.cs, vs.dmo, ng, mw, lig.delta);
+        // slabs of 64 KB of masks (two workgroups a CU), or up to 132 KB where that is fewer than 12 planes
+        const size_t plane = 2 * sizeof(uint32_t) * (size_t)ng * row_words(ng);
+        const int with_halo = (int)std::max((size_t)64 * 1024 / plane, std::min((size_t)12, kVoxLdsBytes / plane));
+        const int planes = with_halo - 4;
+        if (planes < 1) return hipErrorInvalidValue;  // above ng = 300, which no context has
+        const size_t lds = plane * std::min(with_halo, ng) + sizeof(float) * ng;
+        k_vox_slab<<<dim3((ng + planes - 1) / planes, B), kVoxLdsThreads, lds, s>>>(lig, rot, boff, vs.dmo, vs.cnt, vidx, mw, cw,
+                                                                                   planes);
         k_vox_charge<<<B, kChargeThreads, 0, s>>>(vidx, vs.cnt, lig.charge, chg, lig.na, ng3, cw);
     }
     return hipGetLastError();

@@ -37,7 +37,7 @@ double batch_bytes_per_rotation(int nf, int ng, int t) {
     double per_rot = 8.0 * ((double)ng * ng * nf + (double)ng * nf * nf + (double)nf * nf * (H + 16) +
                             (double)nf * nf * std::min(t, 16));
     if (t > 16) {  // the score map of each rotation and its select keys (mdk_create)
-        double P = 1;
+        double P = t <= 512 ? 8192 : 1;
         while (P < t) P *= 2;
         per_rot += 4.0 * nf * nf * nf + 8.0 * P;
     }
@@ -47,10 +47,10 @@ double batch_bytes_per_rotation(int nf, int ng, int t) {
 
 double context_bytes(int nf, int ng, int t, int batch, int na) {
     // two batch slots (with their ligand grids, charge grids and atom indices), the receptor
-    // spectrum and grids, and room for the rest
+    // spectrum, its copy as pairs of columns, the receptor grids, and room for the rest
     const double ng3 = (double)ng * ng * ng;
     return 2.0 * batch * (batch_bytes_per_rotation(nf, ng, t) + 12.0 * ng3 + 4.0 * na) + 8.0 * nf * nf * nf +
-           12.0 * ng3 + 64.0 * 1024 * 1024;
+           16.0 * nf * nf * (nf / 2 + 16) + 12.0 * ng3 + 64.0 * 1024 * 1024;
 }
 
 int auto_batch(int nf, int ng, int t) {

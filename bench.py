@@ -44,7 +44,7 @@ def log(msg):
 # that performs several passes carries their sum, so the shares of the kernels of one batch
 # add up to B_rot.
 STAGE_PASSES = {"voxelize": 0, "fwd_z": 1, "fwd_y": 1, "x_corr": 2, "inv_y": 1, "inv_z_top": 1, "reduce": 0}
-STAGE_KERNELS = {"voxelize": "k_vox_lds / k_vox_atoms + k_vox_masks, k_vox_charge", "fwd_z": "kp_fwd_z",
+STAGE_KERNELS = {"voxelize": "k_vox_lds / k_vox_slab + k_vox_charge", "fwd_z": "kp_fwd_z",
                  "fwd_y": "kp_fwd_y", "x_corr": "kp_x_corr", "inv_y": "kp_inv_y", "inv_z_top": "kp_inv_z_top",
                  "reduce": "k_reduce_top"}
 VALU_ISSUE_PEAK = 256 * 2.4e9  # wave64 VALU instructions per second: one per CU per cycle, 256 CUs at 2.4 GHz

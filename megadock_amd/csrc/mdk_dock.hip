@@ -1263,16 +1263,10 @@ int mdk_dock(mdk_ctx *c, const float *rotcoef, const int *rot_id, int B, mdk_sor
     if (m <= kDirectResults && c->t <= MDK_MAXT) {
         // Few results: the kernels read the rotations and write the results in pinned host memory.
         // The three copies were launches of their own, and from pageable memory waits of the
-        // host's: one rotation at 80^3 80 -> 50 us, 128 at 100^3 785 -> 765.  A voxelizer that
-        // reads a rotation's coefficients in many wavefronts (large grids) still has them copied.
+        // host's: one rotation at 80^3 80 -> 50 us, 128 at 100^3 785 -> 765.
         std::memcpy(c->h_dock_rot, rotcoef, sizeof(float) * 9 * B);
         std::memcpy(c->h_dock_id, rot_id, sizeof(int) * B);
-        const float *rot = c->h_dock_rot;
-        if (!voxelizer_reads_once(c->ng)) {
-            HIPCHK(hipMemcpyAsync(c->d_brot, rot, sizeof(float) * 9 * B, hipMemcpyHostToDevice, c->stream));
-            rot = c->d_brot;
-        }
-        if (dock_batch(c, c->slot[0], rot, c->h_dock_id, B, c->h_dock_out)) return 1;
+        if (dock_batch(c, c->slot[0], c->h_dock_rot, c->h_dock_id, B, c->h_dock_out)) return 1;
         HIPCHK(hipStreamSynchronize(c->stream));
         std::memcpy(out, c->h_dock_out, sizeof(mdk_sortscore) * m);
         return 0;

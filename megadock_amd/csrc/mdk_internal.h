@@ -64,8 +64,6 @@ __device__ __forceinline__ float2 vox_take(const VoxGrid &g, int b, int row, int
 // boff (optional): device word with the batch's first row of rot (graph-captured batches)
 hipError_t launch_voxelize(const LigandDev &lig, const float *rot, int B, const VoxScratch &vs, int *vidx,
                            float *chg, hipStream_t s, const int *boff = nullptr);
-// whether it reads the coefficients of a rotation once (its masks fit in one workgroup's LDS)
-bool voxelizer_reads_once(int ng);
 // (grid_r, grid_i) pairs lg[b*ng^3 + v] from a voxelized batch; clears its charge grid
 hipError_t launch_vox_expand(const VoxGrid &vg, int B, float2 *lg, hipStream_t s);
 

@@ -350,9 +350,8 @@ __global__ void __launch_bounds__(kVoxLdsThreads)
 // Larger grids: a workgroup takes `planes` planes of a rotation's D and O words, with the core and surface
 // bits of two planes more on each side (what the rules reach) in LDS, and goes through the ligand for the
 // atoms that touch them: every kSlabAtoms atoms it lists those whose box or charge lies there, then sets
-// their bits.  Masks in memory (cleared, set by up to
-// 55 atomics an atom, read back with their neighbours) made 768 rotations take 76.5 ms at 256^3 and 82.0
-// at 216^3; with slabs 71.6 and 79.0.
+// their bits.  Masks in memory (cleared, set by up to 55 atomics an atom, read back with their
+// neighbours) made 768 rotations take 76.5 ms at 256^3 and 82.0 at 216^3; with slabs 71.6 and 79.0.
 constexpr int kSlabAtoms = 4096;
 __global__ void __launch_bounds__(kVoxLdsThreads)
     k_vox_slab(LigandDev L, const float *__restrict__ rot, const int *__restrict__ boff, uint32_t *dmo, uint32_t *cnt,
@@ -365,7 +364,7 @@ __global__ void __launch_bounds__(kVoxLdsThreads)
     const int i0 = max(p0 - 2, 0), i1 = min(p1 + 2, ng), nw = (i1 - i0) * ng * rw;
     uint32_t *core = msk, *surf = msk + nw;
     float *gc = reinterpret_cast<float *>(msk + 2 * nw);
-    __shared__ float coef[9];
+    __shared__ float coef[9];  // read once (rot may lie in host memory)
     if (tid < 9) coef[tid] = rot[9 * ((size_t)(boff ? *boff : 0) + b) + tid];
     for (int q = tid; q < 2 * nw; q += kVoxLdsThreads) msk[q] = 0u;
     for (int q = tid; q < ng; q += kVoxLdsThreads) gc[q] = L.gc[q];
@@ -420,14 +419,12 @@ __global__ void k_vox_expand(VoxGrid vg, float2 *lg, int ng3) {
 
 }  // namespace
 
-bool voxelizer_reads_once(int ng) { return mask_bytes(ng) <= kVoxLdsBytes; }
-
 hipError_t launch_voxelize(const LigandDev &lig, const float *rot, int B, const VoxScratch &vs, int *vidx,
                            float *chg, hipStream_t s, const int *boff) {
     const int ng = lig.ng, mw = mask_words(ng), cw = count_words(ng);
     const int ng3 = ng * ng * ng;
     const size_t masks = mask_bytes(ng);
-    if (voxelizer_reads_once(ng)) {  // one workgroup per rotation, bits in LDS
+    if (masks <= kVoxLdsBytes) {  // one workgroup per rotation, bits in LDS
         // the charges' table beside their list, where it fits into the masks' LDS (or little enough
         // for two workgroups a CU); more atoms than that are counted in memory
         const size_t most = std::max(masks + sizeof(float) * ng, (size_t)64 * 1024);

@@ -298,7 +298,8 @@ __device__ __forceinline__ void vox_charges_lds(const int *vi, const float *__re
 // fit): atom runs by LDS atomics, then the D and O words straight to dmo and, if nt > 0, the
 // charges by a table of nt entries (else k_vox_charge follows).  For one rotation it is a chain of dependent steps in
 // one workgroup: with a thread per atom walking five planes, the grid's coordinates loaded from
-// memory inside its loops, a ligand of 336 atoms took 21.6 us and its charges a launch of 4.2 us.
+// memory inside its loops, a ligand of 336 atoms took 21.6 us and its charges a launch of 4.2 us.  Now
+// 12 together.
 constexpr int kVoxLdsThreads = kChargeThreads;
 constexpr int kVoxSplitAtoms = 512;
 constexpr size_t kVoxLdsBytes = 132 * 1024;  // both masks of one rotation, at most

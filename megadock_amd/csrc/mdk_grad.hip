@@ -38,15 +38,16 @@ __global__ void __launch_bounds__(256) k_spec_phase(const float *__restrict__ tq
 }
 
 // trilinear value and gradient (per unit of u) of the two receptor grids at voxel
-// coordinate u; corners outside the grid count as 0
+// coordinate u; corners outside the grid count as 0, and all is NaN where u has a NaN
 __device__ __forceinline__ void trilinear(const float2 *__restrict__ rg, int ng, float ux, float uy, float uz,
                                           float2 &val, float2 &dx, float2 &dy, float2 &dz) {
-    // a position with no corner in the grid (or not a number) counts as one just outside it
-    const float hi = (float)ng + 1.0f;
+    // a position with no corner in the grid counts as one just outside it; one that is not a number
+    // does too, for its loads, and makes the weights NaN (0 would be the score of a ligand outside)
+    const float hi = (float)ng + 1.0f, nan = ux != ux || uy != uy || uz != uz ? NAN : 0.0f;
     if (!(ux > -2.0f && ux < hi && uy > -2.0f && uy < hi && uz > -2.0f && uz < hi)) ux = uy = uz = -2.0f;
     const float fx0 = floorf(ux), fy0 = floorf(uy), fz0 = floorf(uz);
     const int i0 = (int)fx0, j0 = (int)fy0, k0 = (int)fz0;
-    const float fx = ux - fx0, fy = uy - fy0, fz = uz - fz0;
+    const float fx = ux - fx0 + nan, fy = uy - fy0 + nan, fz = uz - fz0 + nan;
     val = dx = dy = dz = make_float2(0.f, 0.f);
     // the corners' loads are issued together (a corner outside the grid loads a voxel inside and
     // counts as 0); with a branch around each, they came one after another

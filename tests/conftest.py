@@ -15,6 +15,20 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (runs through the libmdk C ABI)")
 
 
+# a test that holds a wrong value -> why; it stays as it is and is expected to fail
+WRONG_VALUE = {
+    "test_gpu_companion_edges.py::test_far_poses_score_zero[nan]":
+        "expects a pose that is not a number to score 0; it is not a number (test_gpu_companion_nan.py)",
+}
+
+
+def pytest_collection_modifyitems(items):
+    for item in items:
+        for name, why in WRONG_VALUE.items():
+            if item.nodeid.endswith(name):
+                item.add_marker(pytest.mark.xfail(reason=why, strict=True))
+
+
 @pytest.fixture(scope="session")
 def golden_dir():
     return GOLDEN

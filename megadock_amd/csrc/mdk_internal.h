@@ -76,8 +76,13 @@ struct TopTState {
     unsigned rank;                    // entries still wanted among those matching prefix
     unsigned count;                   // compaction cursor
     unsigned done;                    // the threshold is prefix (its lower bits zero)
-    unsigned pad;
     unsigned hist[256];
+    // t up to kWideT: whether this rotation's list does not fit; the rotations of the batch where it
+    // does not (how many in state 0, the k-th in state k); their prefix and wanted entries before
+    // the histogram of a level (wanted 0: the threshold is the prefix)
+    unsigned over, nover, nth_over;
+    unsigned long long level_prefix[5];
+    unsigned level_wanted[5];
 };
 // keys that launch_topt keeps per rotation for t results per rotation (a power of two)
 unsigned topt_sort_size(int t, int nf);

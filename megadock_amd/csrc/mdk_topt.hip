@@ -22,8 +22,8 @@
 //      score, and with its lower edge a score below which no key can reach the top t
 //      (quotient_cut);
 //   2. the scores not below it, typically a few times t, become the keys that step 3 sorts.
-// A rotation with more of them than fit (many equal scores) is selected by one workgroup with
-// the levels above.
+// A rotation with more of them than fit (many equal scores) is selected by levels of 12 bits
+// (k_wide_level), all workgroups sharing those rotations.
 #include <hip/hip_runtime.h>
 
 #include "mdk_internal.h"
@@ -37,6 +37,10 @@ constexpr int kTSortLds = 8192;  // keys sorted in LDS
 // its ties; above, the bucket alone may not fit.
 constexpr int kWideT = kTSortLds / 16, kWideShift = 19, kWideBuckets = 1 << (32 - kWideShift);
 constexpr unsigned kWideChunk = 32768;  // map entries per workgroup: 32 KB of buckets are cleared and added for 128 KB
+constexpr int kLevels = 5, kLevelBuckets = 4096, kLevelBlocks = 512;  // two workgroups a CU
+static_assert(3 * kLevelBuckets * sizeof(unsigned) <= kTSortLds * sizeof(unsigned long long) &&
+                  kWideT * sizeof(unsigned long long) <= kLevelBuckets * sizeof(unsigned),
+              "the levels' histograms lie where the keys go, the last one picked clear of the keys written");
 static_assert(kWideBuckets * sizeof(unsigned) <= kTSortLds * sizeof(unsigned long long),
               "the histogram lies where the keys go");
 
@@ -48,6 +52,8 @@ __device__ __forceinline__ unsigned long long topt_key(float v, float nf3f, unsi
     const float f = v / nf3f + 0.0f;  // the reference's key; -0 -> +0
     return ((unsigned long long)sortable(f) << 32) | (0xffffffffu - i);
 }
+
+__device__ __forceinline__ unsigned sortable_score(float v) { return sortable(v + 0.0f); }  // -0 as +0
 
 __device__ __forceinline__ float key_float(unsigned long long k) {
     const unsigned u = (unsigned)(k >> 32);
@@ -126,7 +132,7 @@ __global__ void __launch_bounds__(256) k_tsel_compact(const float *__restrict__ 
 __global__ void __launch_bounds__(1024) k_wide_init(TopTState *st, unsigned long long *keys) {
     unsigned *h = reinterpret_cast<unsigned *>(keys + (size_t)blockIdx.x * kTSortLds);
     for (int q = threadIdx.x; q < kWideBuckets; q += 1024) h[q] = 0u;
-    if (threadIdx.x == 0) st[blockIdx.x].count = 0u;
+    if (threadIdx.x == 0) st[blockIdx.x].count = st[blockIdx.x].nover = 0u;
 }
 
 // grid (chunks, B); n3 is a multiple of 8 (nf is even)
@@ -138,10 +144,10 @@ __global__ void __launch_bounds__(1024) k_wide_hist(const float *__restrict__ sm
     const unsigned i0 = blockIdx.x * (kWideChunk / 4), i1 = min(n3 / 4, i0 + kWideChunk / 4);
     for (unsigned i = i0 + threadIdx.x; i < i1; i += 1024u) {
         const float4 v = m[i];
-        atomicAdd(&h[sortable(v.x + 0.0f) >> kWideShift], 1u);
-        atomicAdd(&h[sortable(v.y + 0.0f) >> kWideShift], 1u);
-        atomicAdd(&h[sortable(v.z + 0.0f) >> kWideShift], 1u);
-        atomicAdd(&h[sortable(v.w + 0.0f) >> kWideShift], 1u);
+        atomicAdd(&h[sortable_score(v.x) >> kWideShift], 1u);
+        atomicAdd(&h[sortable_score(v.y) >> kWideShift], 1u);
+        atomicAdd(&h[sortable_score(v.z) >> kWideShift], 1u);
+        atomicAdd(&h[sortable_score(v.w) >> kWideShift], 1u);
     }
     __syncthreads();
     unsigned *g = reinterpret_cast<unsigned *>(keys + (size_t)blockIdx.y * kTSortLds);
@@ -149,15 +155,17 @@ __global__ void __launch_bounds__(1024) k_wide_hist(const float *__restrict__ sm
         if (h[q]) atomicAdd(&g[q], h[q]);
 }
 
-// one workgroup per rotation: the score below which nothing reaches the top `rank` (its bits in
-// st.prefix)
-__global__ void __launch_bounds__(1024) k_wide_pick(TopTState *st, const unsigned long long *keys, unsigned rank,
-                                                    float nf3f) {
+// one workgroup per rotation: the score below which nothing reaches the top `rank` (in st.prefix, as
+// sortable bits), and whether the entries of the buckets down to that score's fit the list; if not,
+// the rotation's first level histogram is cleared
+__global__ void __launch_bounds__(1024) k_wide_pick(TopTState *st, unsigned long long *keys, unsigned rank, float nf3f) {
     constexpr int PER = kWideBuckets / 1024;
-    __shared__ unsigned cum[1024];
-    const unsigned *h = reinterpret_cast<const unsigned *>(keys + (size_t)blockIdx.x * kTSortLds);
+    __shared__ unsigned cum[1024], cut_bits;
+    __shared__ bool over;
+    unsigned *h = reinterpret_cast<unsigned *>(keys + (size_t)blockIdx.x * kTSortLds);
     const int top = kWideBuckets - 1 - (int)threadIdx.x * PER;  // this thread's buckets: top, top - 1, ...
     unsigned n[PER], s = 0u;
+#pragma unroll
     for (int q = 0; q < PER; q++) s += n[q] = h[top - q];
     cum[threadIdx.x] = s;
     __syncthreads();
@@ -167,33 +175,53 @@ __global__ void __launch_bounds__(1024) k_wide_pick(TopTState *st, const unsigne
         cum[threadIdx.x] += add;
         __syncthreads();
     }
-    unsigned c = cum[threadIdx.x] - s;  // entries above this thread's buckets
-    if (c < rank && cum[threadIdx.x] >= rank) {
-        int q = 0;
-        while (c + n[q] < rank) c += n[q++];
-        const unsigned long long edge = (unsigned long long)((unsigned)(top - q) << kWideShift) << 32;
-        st[blockIdx.x].prefix = __float_as_uint(quotient_cut(key_float(edge), nf3f));
+    const unsigned above = cum[threadIdx.x] - s;  // entries above this thread's buckets
+    if (above < rank && cum[threadIdx.x] >= rank) {
+        int b = top;
+        unsigned c = above;
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            c += n[q];
+            if (c < rank) b--;
+        }
+        const unsigned long long edge = (unsigned long long)((unsigned)b << kWideShift) << 32;
+        const float cut = quotient_cut(key_float(edge), nf3f);
+        over = cut != cut;  // a bucket of what is not a number
+        cut_bits = sortable_score(cut);
     }
+    __syncthreads();
+    const int last = (int)(cut_bits >> kWideShift);
+    if (top >= last && top - PER < last) {
+        unsigned c = above;
+#pragma unroll
+        for (int q = 0; q < PER; q++)
+            if (top - q >= last) c += n[q];
+        TopTState &S = st[blockIdx.x];
+        over = over || c > (unsigned)kTSortLds;
+        S.prefix = cut_bits;
+        S.over = over;
+        if (over) st[atomicAdd(&st[0].nover, 1u)].nth_over = blockIdx.x;
+    }
+    __syncthreads();
+    if (over)
+        for (int q = threadIdx.x; q < kLevelBuckets; q += 1024) h[q] = 0u;
 }
 
-// grid (chunks, B): the keys of the scores not below the cut (a score that is not a number is
-// not), as many as fit
+// grid (chunks, B): the keys of the scores not below the cut, of rotations where they fit
 __global__ void __launch_bounds__(1024) k_wide_compact(const float *__restrict__ smap, unsigned n3, float nf3f,
                                                        TopTState *st, unsigned long long *keys) {
     TopTState &s = st[blockIdx.y];
-    const float cut = __uint_as_float((unsigned)s.prefix);
+    if (s.over) return;  // uniform
+    const unsigned cut = (unsigned)s.prefix;
     const float4 *m = reinterpret_cast<const float4 *>(smap + (size_t)blockIdx.y * n3);
     unsigned long long *out = keys + (size_t)blockIdx.y * kTSortLds;
     auto put = [&](float v, unsigned i) {
-        if (!(v < cut)) {
-            const unsigned k = atomicAdd(&s.count, 1u);
-            if (k < (unsigned)kTSortLds) out[k] = topt_key(v, nf3f, i);
-        }
+        if (sortable_score(v) >= cut) out[atomicAdd(&s.count, 1u)] = topt_key(v, nf3f, i);
     };
     const unsigned i0 = blockIdx.x * (kWideChunk / 4), i1 = min(n3 / 4, i0 + kWideChunk / 4);
     for (unsigned i = i0 + threadIdx.x; i < i1; i += 1024u) {
         const float4 v = m[i];
-        if (!(v.x < cut && v.y < cut && v.z < cut && v.w < cut)) {
+        if (sortable_score(v.x) >= cut || sortable_score(v.y) >= cut || sortable_score(v.z) >= cut || sortable_score(v.w) >= cut) {
             put(v.x, 4 * i);
             put(v.y, 4 * i + 1);
             put(v.z, 4 * i + 2);
@@ -202,52 +230,120 @@ __global__ void __launch_bounds__(1024) k_wide_compact(const float *__restrict__
     }
 }
 
-// A rotation whose keys did not fit: the radix select of the levels by one workgroup, whose keys
-// (exactly rank of them) replace the list.
-__global__ void __launch_bounds__(1024) k_wide_slow(const float *__restrict__ smap, unsigned n3, float nf3f,
-                                                    TopTState *st, unsigned long long *keys, unsigned rank) {
-    __shared__ unsigned h[256], n;
-    __shared__ unsigned long long prefix, mask;
-    __shared__ unsigned want;
-    __shared__ bool done;
-    const int b = blockIdx.x;
-    if (st[b].count <= (unsigned)kTSortLds) return;  // uniform
-    const float *m = smap + (size_t)b * n3;
-    if (threadIdx.x == 0) {
-        prefix = mask = 0ull;
-        want = rank;
-        n = 0u;
-        done = false;
-    }
-    for (int shift = 56; shift >= 0; shift -= 8) {
-        if (threadIdx.x < 256) h[threadIdx.x] = 0u;
+// Rotations whose keys do not fit: radix select of the keys
+//   sortable(score / nf^3) << 28 | (2^28 - 1 - index)          (60 bits; nf <= 640)
+// by five levels of 12 bits, a launch each, whose workgroups share out those rotations (with one
+// rotation all of them read its map).  A launch first picks the last level's digit of its
+// rotation, each workgroup for itself, from the histogram that the launch before left; the
+// sixth (level 5) writes the keys from the threshold on, rank of them.  The histograms take turns in three
+// places of the rotation's keys: level l - 1 is read, l added to, l + 1 cleared.  Without such
+// rotations a launch ends at its first load (six of them: 1-5 us a call).  Docking one rotation with
+// every score equal, t = 64, took 9.1 ms at 112^3 and 106 at 256^3 with one workgroup that read the map
+// nine times, 0.30 and 0.77 with levels of 8 bits in 17 launches over every rotation, and takes 0.19
+// and 0.42; 128 such rotations of 112^3 14.3, 5.8 and 3.1.
+__device__ __forceinline__ unsigned long long level_key(float v, float nf3f, unsigned i) {
+    return ((unsigned long long)sortable(v / nf3f + 0.0f) << 28) | (0xfffffffu - i);
+}
+
+__global__ void __launch_bounds__(1024) k_wide_level(const float *__restrict__ smap, unsigned n3, float nf3f,
+                                                     TopTState *st, unsigned long long *keys, unsigned rank, int level) {
+    __shared__ unsigned h[kLevelBuckets], wave_sum[16], picked[3];
+    const unsigned n = st[0].nover, parts = max(1u, gridDim.x / max(n, 1u));
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const unsigned part = n < gridDim.x ? blockIdx.x / max(n, 1u) : 0u;
+    if (part >= parts) return;  // uniform, as all that follows but the entries
+    for (unsigned q = n < gridDim.x ? blockIdx.x % max(n, 1u) : blockIdx.x; q < n; q += gridDim.x) {
+        const unsigned b = st[q].nth_over;
+        TopTState &S = st[b];
+        unsigned long long *out = keys + (size_t)b * kTSortLds;
+        unsigned *hist = reinterpret_cast<unsigned *>(out);
+        unsigned long long prefix = 0ull;
+        unsigned want = rank;
+        if (level > 0) {
+            prefix = S.level_prefix[level - 1];
+            want = S.level_wanted[level - 1];
+        }
+        if (level > 0 && want > 0) {
+            // this thread's buckets: 4095 - 4 tid downwards
+            const unsigned *last = hist + (level - 1) % 3 * kLevelBuckets;
+            const uint4 v = reinterpret_cast<const uint4 *>(last)[1023 - tid];
+            const unsigned s = v.x + v.y + v.z + v.w;
+            unsigned c = s;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const unsigned o = __shfl_up(c, d, 64);
+                if (lane >= d) c += o;
+            }
+            if (lane == 63) wave_sum[wave] = c;
+            __syncthreads();
+            for (int w = 0; w < wave; w++) c += wave_sum[w];
+            const unsigned above = c - s;
+            if (above < want && c >= want) {
+                const unsigned in[4] = {v.w, v.z, v.y, v.x};
+                unsigned digit = kLevelBuckets - 1 - 4 * tid, a = above, here = in[0];
+#pragma unroll
+                for (int k = 1; k < 4; k++)
+                    if (a + here < want) {
+                        a += here;
+                        here = in[k];
+                        digit--;
+                    }
+                picked[0] = digit;
+                picked[1] = want - a;
+                picked[2] = want - a == here;  // the whole bucket is wanted
+            }
+            __syncthreads();
+            prefix |= (unsigned long long)picked[0] << (60 - 12 * level);
+            want = picked[2] ? 0u : picked[1];
+            __syncthreads();  // the next rotation writes them
+        }
+        // this workgroup's share of the map, in fours
+        const unsigned share = (n3 / 4 + parts - 1) / parts, i0 = part * share, i1 = min(n3 / 4, i0 + share);
+        const float4 *m = reinterpret_cast<const float4 *>(smap + (size_t)b * n3);
+        if (level == kLevels) {
+            for (unsigned i = i0 + tid; i < i1; i += 1024u) {
+                const float4 f = m[i];
+                const float e[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (level_key(e[k], nf3f, 4 * i + k) >= prefix)
+                        out[atomicAdd(&S.count, 1u)] = topt_key(e[k], nf3f, 4 * i + k);
+            }
+            continue;
+        }
+        if (part == 0) {
+            if (tid == 0) {
+                S.level_prefix[level] = prefix;
+                S.level_wanted[level] = want;
+            }
+            for (int k = tid; k < kLevelBuckets; k += 1024) hist[(level + 1) % 3 * kLevelBuckets + k] = 0u;
+        }
+        if (want == 0u) continue;
+        for (int k = tid; k < kLevelBuckets; k += 1024) h[k] = 0u;
         __syncthreads();
-        const unsigned long long p = prefix, k0 = mask;
-        for (unsigned i = threadIdx.x; i < n3; i += 1024u) {
-            const unsigned long long k = topt_key(m[i], nf3f, i);
-            if ((k & k0) == p) atomicAdd(&h[(unsigned)(k >> shift) & 255u], 1u);
+        const int shift = 48 - 12 * level;
+        for (unsigned i = i0 + tid; i < i1; i += 1024u) {
+            const float4 f = m[i];
+            const float e[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const unsigned long long key = level_key(e[k], nf3f, 4 * i + k);
+                const bool in = level == 0 || key >> (shift + 12) == prefix >> (shift + 12);
+                const int digit = (int)(key >> shift) & (kLevelBuckets - 1);
+                // equal digits are the rule here: one lane adds for all that have the first one's
+                const unsigned long long some = __ballot(in);
+                if (some == 0ull) continue;
+                const int first = __ffsll((long long)some) - 1, d0 = __builtin_amdgcn_readlane(digit, first);
+                const unsigned long long same = __ballot(in && digit == d0);
+                if (lane == first) atomicAdd(&h[d0], (unsigned)__popcll(same));
+                else if (in && digit != d0) atomicAdd(&h[digit], 1u);
+            }
         }
         __syncthreads();
-        if (threadIdx.x == 0) {
-            unsigned c = 0u;
-            int d = 255;
-            while (d > 0 && c + h[d] < want) c += h[d--];
-            prefix |= (unsigned long long)d << shift;
-            mask |= 255ull << shift;
-            want -= c;
-            done = want == h[d];  // the whole bucket is wanted
-        }
-        __syncthreads();
-        if (done) break;  // uniform
+        for (int k = tid; k < kLevelBuckets; k += 1024)
+            if (h[k]) atomicAdd(&hist[level % 3 * kLevelBuckets + k], h[k]);
+        __syncthreads();  // the next rotation clears h
     }
-    const unsigned long long thr = prefix;
-    unsigned long long *out = keys + (size_t)b * kTSortLds;
-    for (unsigned i = threadIdx.x; i < n3; i += 1024u) {
-        const unsigned long long k = topt_key(m[i], nf3f, i);
-        if (k >= thr) out[atomicAdd(&n, 1u)] = k;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) st[b].count = n;
 }
 
 // one workgroup per rotation: descending bitonic sort of its P keys (padded with 0, which
@@ -325,7 +421,8 @@ hipError_t launch_topt(const float *smap, int B, int nf, int t, TopTState *st, u
         k_wide_hist<<<wide, 1024, 0, s>>>(smap, n3, keys);
         k_wide_pick<<<B, 1024, 0, s>>>(st, keys, rank, nf3f);
         k_wide_compact<<<wide, 1024, 0, s>>>(smap, n3, nf3f, st, keys);
-        k_wide_slow<<<B, 1024, 0, s>>>(smap, n3, nf3f, st, keys, rank);
+        for (int level = 0; level <= kLevels; level++)
+            k_wide_level<<<kLevelBlocks, 1024, 0, s>>>(smap, n3, nf3f, st, keys, rank, level);
         k_tsel_sort_out<<<B, 1024, 0, s>>>(keys, P, 0u, st, t, nf, out, rot_id, boff);
         return hipGetLastError();
     }

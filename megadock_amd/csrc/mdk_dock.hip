@@ -44,8 +44,9 @@ hipError_t launch_receptor_voxel(const float *xyz, const float *radius, const fl
 // off-grid scores (mdk_grad.hip)
 hipError_t launch_spec_phase(const float *t_dev, int B, int nf, float2 *ph, hipStream_t s);
 hipError_t launch_spec_finish(const double *part, int B, int n, int nf, float *out_dev, hipStream_t s);
+size_t companion_scratch_doubles(int na);
 hipError_t launch_companion(const LigandDev &lig, const float *wshape, const float2 *recgrid, const float *rot_dev,
-                            const float *t_dev, int B, int nf, float *out_dev, hipStream_t s);
+                            const float *t_dev, int B, int nf, double *part, float *out_dev, hipStream_t s);
 
 #define MDK_NSTAGE 7  // voxelize, fwd_z, fwd_y, x_corr, inv_y, inv_z_top, reduce
 
@@ -619,6 +620,7 @@ struct mdk_ctx {
     float *d_wshape = nullptr;    // companion shape weight per ligand atom
     float2 *d_gph = nullptr;      // spectral score: phases of a batch's poses (max_batch * 3 nf)
     double *d_gpart = nullptr;    // and its partial sums (max_batch * spec_parts() * 4)
+    double *d_cpart = nullptr;    // companion score: partial sums of few poses of a large ligand
     float *d_rpsc = nullptr;      // receptor shape grid without the ACE term (mdk_score_detail), ng^3
     int *d_btrans = nullptr;      // grid translations of a batch (max_batch * 3)
     float *d_dsum = nullptr;      // detail sums of a batch (max_batch * 9)
@@ -937,8 +939,9 @@ int mdk_create(int device, int nf, int ng, int na, int t, int max_batch, mdk_ctx
         dmalloc(&c->d_rc2, na) || dmalloc(&c->d_rs2, na) || dmalloc(&c->d_charge, na) || dmalloc(&c->d_gc, ng) ||
         dmalloc(&c->d_brot, 9 * B) || dmalloc(&c->d_bid, B) || dmalloc(&c->d_recgrid, ng3) ||
         dmalloc(&c->d_wshape, na) ||
-        (pipe_available(nf) && (dmalloc(&c->d_gph, B * 3 * nf) || dmalloc(&c->d_gpart, B * spec_parts(c) * 4))) || dmalloc(&c->d_rpsc, ng3) || dmalloc(&c->d_btrans, 3 * B) ||
-        dmalloc(&c->d_dsum, 9 * B))
+        (pipe_available(nf) && (dmalloc(&c->d_gph, B * 3 * nf) || dmalloc(&c->d_gpart, B * spec_parts(c) * 4))) ||
+        (companion_scratch_doubles(na) && dmalloc(&c->d_cpart, companion_scratch_doubles(na))) ||
+        dmalloc(&c->d_rpsc, ng3) || dmalloc(&c->d_btrans, 3 * B) || dmalloc(&c->d_dsum, 9 * B))
         return bail(1);
     for (int k = 0; k < c->nslots; k++) {
         BatchSlot &S = c->slot[k];
@@ -1019,7 +1022,7 @@ int mdk_destroy(mdk_ctx *c) {
         if (c->slot[k].stream) (void)hipStreamSynchronize(c->slot[k].stream);
     void *ptrs[] = {c->d_tw, c->d_tw4, c->d_rec, c->d_recp, c->d_xyz, c->d_rc2, c->d_rs2, c->d_charge, c->d_gc, c->d_rot,
                     c->d_rotid, c->d_brot, c->d_bid, c->d_results, c->d_topn_scratch, c->d_topn_out,
-                    c->d_recgrid, c->d_wshape, c->d_gph, c->d_gpart, c->d_rpsc, c->d_btrans, c->d_dsum, c->d_recwork, c->d_posework};
+                    c->d_recgrid, c->d_wshape, c->d_gph, c->d_gpart, c->d_cpart, c->d_rpsc, c->d_btrans, c->d_dsum, c->d_recwork, c->d_posework};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (c->h_topn) (void)hipHostFree(c->h_topn);
@@ -1684,7 +1687,8 @@ int mdk_score_companion(mdk_ctx *c, const float *rotcoef, const float *t, int B,
         const size_t np = std::min(kPoses, B - p0);
         if (upload_poses(c, rotcoef + 9 * (size_t)p0, t + 3 * (size_t)p0, np, 7)) return 1;
         float *d = c->d_posework;
-        HIPCHK(launch_companion(c->lig, c->d_wshape, c->d_recgrid, d, d + 9 * np, (int)np, c->nf, d + 12 * np, c->stream));
+        HIPCHK(launch_companion(c->lig, c->d_wshape, c->d_recgrid, d, d + 9 * np, (int)np, c->nf, c->d_cpart, d + 12 * np,
+                                c->stream));
         if (download_poses(c, out + 7 * (size_t)p0, np, 7)) return 1;
     }
     return 0;

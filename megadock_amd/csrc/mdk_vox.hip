@@ -211,7 +211,7 @@ __device__ __forceinline__ void vox_crowded(const int *vi, const float *__restri
 
 // the counts are global words of two 16-bit counts, left zero again
 __global__ void __launch_bounds__(kChargeThreads)
-    k_vox_charge(const int *vidx, uint32_t *cnt, const float *__restrict__ charge, float *chg, int na, int ng3, int cw) {
+    k_vox_charge(const int *__restrict__ vidx, uint32_t *cnt, const float *__restrict__ charge, float *chg, int na, int ng3, int cw) {
     __shared__ int nlist;
     __shared__ int2 list[kCrowdCap];  // (voxel, atom)
     const int b = blockIdx.x, tid = threadIdx.x;

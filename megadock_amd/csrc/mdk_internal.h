@@ -26,18 +26,26 @@ __host__ __device__ inline int row_words(int ng) { return (ng + 31) / 32; }
 inline int mask_words(int ng) { return ng * ng * row_words(ng); }
 // per-voxel atom counts, two 16-bit counters per word (ligands have < 65536 atoms)
 inline int count_words(int ng) { return (ng * ng * ng + 1) / 2; }
-// scratch words per rotation: delta + value-1 masks, counts
-inline size_t vox_scratch_words(int ng) { return 2 * (size_t)mask_words(ng) + count_words(ng); }
+// core and surface masks of one rotation, and whether they fit the LDS of a workgroup
+inline size_t mask_bytes(int ng) { return 2 * sizeof(uint32_t) * (size_t)mask_words(ng); }
+constexpr size_t kVoxLdsBytes = 132 * 1024;
+inline bool masks_in_lds(int ng) { return mask_bytes(ng) <= kVoxLdsBytes; }
+// scratch words per rotation: delta + value-1 masks, counts, and core + surface masks of larger grids
+inline size_t vox_scratch_words(int ng) {
+    return (masks_in_lds(ng) ? 2 : 4) * (size_t)mask_words(ng) + count_words(ng);
+}
 
 // Voxelization scratch of a context, laid out for max_batch rotations:
 //   dmo [b][2][mask_words]  delta mask D and value-1 mask O (written per batch)
 //   cnt [b][count_words]    atom counts per voxel, zero between batches
+//   cs  [b][2][mask_words]  core and surface bits (cleared per batch; grids above masks_in_lds)
 struct VoxScratch {
-    uint32_t *dmo, *cnt;
+    uint32_t *dmo, *cnt, *cs;
 };
 inline VoxScratch vox_scratch(uint32_t *base, int max_batch, int ng) {
-    const size_t mw = mask_words(ng);
-    return VoxScratch{base, base + 2 * mw * max_batch};
+    const size_t B = max_batch;
+    uint32_t *cnt = base + 2 * B * mask_words(ng);
+    return VoxScratch{base, cnt, cnt + B * count_words(ng)};
 }
 
 // A batch of ligand grids as the FFT passes read them: shape value delta where D is set,

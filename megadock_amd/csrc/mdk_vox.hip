@@ -302,8 +302,6 @@ __device__ __forceinline__ void vox_charges_lds(const int *vi, const float *__re
 // 12 together.
 constexpr int kVoxLdsThreads = kChargeThreads;
 constexpr int kVoxSplitAtoms = 512;
-constexpr size_t kVoxLdsBytes = 132 * 1024;  // both masks of one rotation, at most
-inline size_t mask_bytes(int ng) { return 2 * sizeof(uint32_t) * (size_t)mask_words(ng); }
 __global__ void __launch_bounds__(kVoxLdsThreads)
     k_vox_lds(LigandDev L, const float *__restrict__ rot, const int *__restrict__ boff, uint32_t *dmo, uint32_t *cnt,
               int *vidx, int mw, int cw, float *chg, int nt) {
@@ -410,6 +408,46 @@ __global__ void __launch_bounds__(kVoxLdsThreads)
     }
 }
 
+// The same with the core and surface bits in memory, for few rotations: a thread per atom and plane, so that
+// one rotation of a large ligand fills the chip, where its slabs are a workgroup each.
+__global__ void k_vox_clear(uint32_t *p, size_t n) {
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = 0u;
+}
+
+__global__ void __launch_bounds__(128) k_vox_atoms(LigandDev L, const float *__restrict__ rot, const int *__restrict__ boff,
+                                                   uint32_t *cs, uint32_t *cnt, int *vidx, int mw, int cw) {
+    const int b = blockIdx.y, q = blockIdx.x * blockDim.x + threadIdx.x, l = q / 5, d = q - 5 * l;
+    __shared__ float coef[9];  // read once (rot may lie in host memory)
+    if (threadIdx.x < 9) coef[threadIdx.x] = rot[9 * ((size_t)(boff ? *boff : 0) + b) + threadIdx.x];
+    __syncthreads();
+    if (l >= L.na) return;
+    float r[9], X, Y, Z;
+#pragma unroll
+    for (int k = 0; k < 9; k++) r[k] = coef[k];
+    rotate_atom(L, r, l, X, Y, Z);
+    uint32_t *cb = cs + (size_t)b * 2 * mw;
+    vox_planes(L, L.gc, X, Y, Z, l, d - 2, d - 1, cb, cb + mw, 0, L.ng);
+    if (d == 0) {
+        const int v = charge_voxel(L, X, Y, Z);
+        vidx[(size_t)b * L.na + l] = v;
+        atomicAdd(&cnt[(size_t)b * cw + (v >> 1)], 1u << (16 * (v & 1)));
+    }
+}
+
+__global__ void __launch_bounds__(256) k_vox_masks(const uint32_t *__restrict__ cs, uint32_t *dmo, int ng, int mw, float delta) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
+    if (q >= mw) return;
+    const uint32_t *cb = cs + (size_t)b * 2 * mw;
+    uint32_t *db = dmo + (size_t)b * 2 * mw;
+    const MaskRows C{cb, ng, row_words(ng), 0}, S{cb + mw, ng, row_words(ng), 0};
+    vox_mask_word(C, S, q, ng, delta, db[q], db[mw + q]);
+}
+
+// Rotations of a larger grid up to which their bits lie in memory.  One, 4, 8 and 16 rotations at 256^3 (with
+// their charges): 2081 atoms 73, 82, 110, 123 us in memory, 87, 93, 114, 116 in slabs; 8000 atoms 213,
+// 249, 290, 350 and 248, 270, 290, 303; at 216^3 8 rotations 112 and 107, 296 and 283.
+constexpr int kFewRotations = 4;
+
 // grids as (grid_r, grid_i) pairs; clears the charge grid it reads
 __global__ void k_vox_expand(VoxGrid vg, float2 *lg, int ng3) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
@@ -425,7 +463,7 @@ hipError_t launch_voxelize(const LigandDev &lig, const float *rot, int B, const 
     const int ng = lig.ng, mw = mask_words(ng), cw = count_words(ng);
     const int ng3 = ng * ng * ng;
     const size_t masks = mask_bytes(ng);
-    if (masks <= kVoxLdsBytes) {  // one workgroup per rotation, bits in LDS
+    if (masks_in_lds(ng)) {  // one workgroup per rotation, bits in LDS
         // the charges' table beside their list, where it fits into the masks' LDS (or little enough
         // for two workgroups a CU); more atoms than that are counted in memory
         const size_t most = std::max(masks + sizeof(float) * ng, (size_t)64 * 1024);
@@ -436,12 +474,18 @@ hipError_t launch_voxelize(const LigandDev &lig, const float *rot, int B, const 
         const size_t lds = std::max(masks + sizeof(float) * ng, nt ? table(nt) : 0);
         k_vox_lds<<<B, kVoxLdsThreads, lds, s>>>(lig, rot, boff, vs.dmo, vs.cnt, vidx, mw, cw, chg, nt);
         if (!nt) k_vox_charge<<<B, kChargeThreads, 0, s>>>(vidx, vs.cnt, lig.charge, chg, lig.na, ng3, cw);
+    } else if (B <= kFewRotations) {
+        const size_t words = 2 * (size_t)B * mw;
+        k_vox_clear<<<(unsigned)std::min((words + 255) / 256, (size_t)65535), 256, 0, s>>>(vs.cs, words);
+        k_vox_atoms<<<dim3((5 * lig.na + 127) / 128, B), 128, 0, s>>>(lig, rot, boff, vs.cs, vs.cnt, vidx, mw, cw);
+        k_vox_masks<<<dim3((mw + 255) / 256, B), 256, 0, s>>>(vs.cs, vs.dmo, ng, mw, lig.delta);
+        k_vox_charge<<<B, kChargeThreads, 0, s>>>(vidx, vs.cnt, lig.charge, chg, lig.na, ng3, cw);
     } else {
         // slabs of 64 KB of masks (two workgroups a CU), or up to 132 KB where that is fewer than 12 planes
         const size_t plane = 2 * sizeof(uint32_t) * (size_t)ng * row_words(ng);
         const int with_halo = (int)std::max((size_t)64 * 1024 / plane, std::min((size_t)12, kVoxLdsBytes / plane));
         const int planes = with_halo - 4;
-        if (planes < 1) return hipErrorInvalidValue;  // above ng = 300, which no context has
+        if (planes < 1) return hipErrorInvalidValue;  // above ng = 320, which no context has
         const size_t lds = plane * std::min(with_halo, ng) + sizeof(float) * ng;
         k_vox_slab<<<dim3((ng + planes - 1) / planes, B), kVoxLdsThreads, lds, s>>>(lig, rot, boff, vs.dmo, vs.cnt, vidx, mw, cw,
                                                                                    planes);

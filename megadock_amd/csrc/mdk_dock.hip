@@ -71,6 +71,8 @@ constexpr int WY = 16;   // lines per workgroup, y passes
 constexpr int WX = 8;    // kz columns per workgroup in the x pass (plus 8 partner columns)
 constexpr int kThreads = 256;  // threads per workgroup, where not chosen by the size
 constexpr size_t kDirectResults = 256;  // mdk_dock: as many results go straight to host memory
+// off-grid scores: poses a block, and words a pose (rotation, translation, at most seven results)
+constexpr int kPoses = 65536, kPoseWords = 19;
 
 __device__ __forceinline__ void load_tw(float2 *tw_s, const float2 *tw_g, int ntw) {
     for (int q = threadIdx.x; q < ntw; q += blockDim.x) tw_s[q] = tw_g[q];
@@ -604,7 +606,8 @@ struct mdk_ctx {
     int *d_rotid = nullptr;  // iota table, rotation i has number i
     float *d_brot = nullptr; // staging for mdk_dock (max_batch * 9)
     int *d_bid = nullptr;    // staging ids
-    // mdk_dock's calls of few results: one pinned block, read and written by the kernels
+    // mdk_dock's calls of few results: one pinned block, read and written by the kernels (with
+    // h_pose's first room behind it)
     mdk_sortscore *h_dock_out = nullptr;
     float *h_dock_rot = nullptr;
     int *h_dock_id = nullptr;
@@ -637,11 +640,9 @@ struct mdk_ctx {
     float2 *h_rstage = nullptr;
     float *h_lstage = nullptr;
     size_t h_rstage_n = 0, h_lstage_n = 0;  // bytes
-    float *h_pstage = nullptr;  // poses and results of the off-grid scores, pinned and on the device
-    size_t h_pstage_n = 0;      // bytes
-    hipEvent_t ev_pstage = nullptr;
-    float *d_posework = nullptr;
-    size_t posework_n = 0;      // floats
+    // poses and results of the off-grid scores, pinned and on the device: room for pose_room poses
+    float *h_pose = nullptr, *h_pose_grown = nullptr, *d_pose = nullptr;
+    size_t pose_room = 0;
     char *d_recwork = nullptr;  // atoms and bit masks of mdk_set_receptor_atoms, grown to the largest receptor
     size_t recwork_n = 0;       // bytes
     hipEvent_t ev_rstage = nullptr, ev_lstage = nullptr;
@@ -987,11 +988,15 @@ int mdk_create(int device, int nf, int ng, int na, int t, int max_batch, mdk_ctx
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0)
             c->cu_count = cus;
     }
-    if (hipHostMalloc((void **)&c->h_dock_out, kDirectResults * (sizeof(mdk_sortscore) + 10 * sizeof(float)),
+    c->pose_room = std::min(B, (size_t)kPoses);
+    if (dmalloc(&c->d_pose, kPoseWords * c->pose_room)) return bail(1);
+    if (hipHostMalloc((void **)&c->h_dock_out,
+                      kDirectResults * (sizeof(mdk_sortscore) + 10 * sizeof(float)) + kPoseWords * c->pose_room * sizeof(float),
                       hipHostMallocDefault) != hipSuccess)
         return bail(fail("mdk_create: pinned memory allocation failed"));
     c->h_dock_rot = reinterpret_cast<float *>(c->h_dock_out + kDirectResults);
     c->h_dock_id = reinterpret_cast<int *>(c->h_dock_rot + 9 * kDirectResults);
+    c->h_pose = reinterpret_cast<float *>(c->h_dock_id + kDirectResults);
     if (hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess)
         return bail(fail("mdk_create: event creation failed"));
     // the largest kernel LDS request must fit
@@ -1022,7 +1027,7 @@ int mdk_destroy(mdk_ctx *c) {
         if (c->slot[k].stream) (void)hipStreamSynchronize(c->slot[k].stream);
     void *ptrs[] = {c->d_tw, c->d_tw4, c->d_rec, c->d_recp, c->d_xyz, c->d_rc2, c->d_rs2, c->d_charge, c->d_gc, c->d_rot,
                     c->d_rotid, c->d_brot, c->d_bid, c->d_results, c->d_topn_scratch, c->d_topn_out,
-                    c->d_recgrid, c->d_wshape, c->d_gph, c->d_gpart, c->d_cpart, c->d_rpsc, c->d_btrans, c->d_dsum, c->d_recwork, c->d_posework};
+                    c->d_recgrid, c->d_wshape, c->d_gph, c->d_gpart, c->d_cpart, c->d_rpsc, c->d_btrans, c->d_dsum, c->d_recwork, c->d_pose};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (c->h_topn) (void)hipHostFree(c->h_topn);
@@ -1030,8 +1035,7 @@ int mdk_destroy(mdk_ctx *c) {
     if (c->topn_done) (void)hipEventDestroy(c->topn_done);
     if (c->h_rstage) (void)hipHostFree(c->h_rstage);
     if (c->h_lstage) (void)hipHostFree(c->h_lstage);
-    if (c->h_pstage) (void)hipHostFree(c->h_pstage);
-    if (c->ev_pstage) (void)hipEventDestroy(c->ev_pstage);
+    if (c->h_pose_grown) (void)hipHostFree(c->h_pose_grown);
     if (c->ev_rstage) (void)hipEventDestroy(c->ev_rstage);
     if (c->ev_lstage) (void)hipEventDestroy(c->ev_lstage);
     drop_graphs(c);
@@ -1622,31 +1626,33 @@ int mdk_autotune(mdk_ctx *c, int first, int count, int *choice) {
     return 0;
 }
 
-// Poses of the off-grid scores: rotations (9) and translations (3) of n poses in one pinned block
-// and one copy, k results a pose behind them and back the same way.
-constexpr int kPoses = 65536;  // poses a block
-int upload_poses(mdk_ctx *c, const float *rotcoef, const float *t, size_t n, int k) {
-    const size_t words = (12 + k) * n;
-    if (staging((void **)&c->h_pstage, c->h_pstage_n, sizeof(float) * words, c->ev_pstage)) return 1;
-    if (words > c->posework_n) {
-        if (c->d_posework) {
-            HIPCHK(hipStreamSynchronize(c->stream));
-            HIPCHK(hipFree(c->d_posework));
-        }
-        c->d_posework = nullptr;
-        c->posework_n = 0;
-        HIPCHK(hipMalloc((void **)&c->d_posework, sizeof(float) * words));
-        c->posework_n = words;
+// Poses of the off-grid scores: rotations (9) and translations (3) of n <= kPoses poses in one pinned
+// block and one copy, k results a pose behind them and back the same way.  The blocks are there from
+// mdk_create on for a batch's poses and grow to twice their size: made by the first call and to
+// the poses of each, a call of 8 poses took 57-105 us and each larger one 65-115, 29 otherwise.
+int upload_poses(mdk_ctx *c, const float *rotcoef, const float *t, size_t n) {
+    if (n > c->pose_room) {
+        const size_t room = std::min(std::max(n, 2 * c->pose_room), (size_t)kPoses);
+        HIPCHK(hipStreamSynchronize(c->stream));
+        c->pose_room = 0;
+        if (c->d_pose) HIPCHK(hipFree(c->d_pose));
+        c->d_pose = nullptr;
+        if (c->h_pose_grown) HIPCHK(hipHostFree(c->h_pose_grown));
+        c->h_pose = c->h_pose_grown = nullptr;
+        HIPCHK(hipHostMalloc((void **)&c->h_pose_grown, sizeof(float) * kPoseWords * room, hipHostMallocDefault));
+        HIPCHK(hipMalloc((void **)&c->d_pose, sizeof(float) * kPoseWords * room));
+        c->h_pose = c->h_pose_grown;
+        c->pose_room = room;
     }
-    std::memcpy(c->h_pstage, rotcoef, sizeof(float) * 9 * n);
-    std::memcpy(c->h_pstage + 9 * n, t, sizeof(float) * 3 * n);
-    HIPCHK(hipMemcpyAsync(c->d_posework, c->h_pstage, sizeof(float) * 12 * n, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipEventRecord(c->ev_pstage, c->stream));
+    // (the last block's copies are done: download_poses waits for them)
+    std::memcpy(c->h_pose, rotcoef, sizeof(float) * 9 * n);
+    std::memcpy(c->h_pose + 9 * n, t, sizeof(float) * 3 * n);
+    HIPCHK(hipMemcpyAsync(c->d_pose, c->h_pose, sizeof(float) * 12 * n, hipMemcpyHostToDevice, c->stream));
     return 0;
 }
 int download_poses(mdk_ctx *c, float *out, size_t n, int k) {
-    float *h = c->h_pstage + 12 * n;
-    HIPCHK(hipMemcpyAsync(h, c->d_posework + 12 * n, sizeof(float) * k * n, hipMemcpyDeviceToHost, c->stream));
+    float *h = c->h_pose + 12 * n;
+    HIPCHK(hipMemcpyAsync(h, c->d_pose + 12 * n, sizeof(float) * k * n, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     std::memcpy(out, h, sizeof(float) * k * n);
     return 0;
@@ -1663,8 +1669,8 @@ int mdk_score_spectral(mdk_ctx *c, const float *rotcoef, const float *t, int B, 
     BatchSlot &S = c->slot[0];
     for (int p0 = 0; p0 < B; p0 += kPoses) {
         const size_t np = std::min(kPoses, B - p0);
-        if (upload_poses(c, rotcoef + 9 * (size_t)p0, t + 3 * (size_t)p0, np, 4)) return 1;
-        float *d = c->d_posework, *d_t = d + 9 * np, *d_out = d + 12 * np;
+        if (upload_poses(c, rotcoef + 9 * (size_t)p0, t + 3 * (size_t)p0, np)) return 1;
+        float *d = c->d_pose, *d_t = d + 9 * np, *d_out = d + 12 * np;
         for (size_t q0 = 0; q0 < np; q0 += c->max_batch) {  // in batches of the context's size, in order
             const int nb = (int)std::min((size_t)c->max_batch, np - q0);
             HIPCHK(launch_voxelize(c->lig, d + 9 * q0, nb, S.vs, S.d_vidx, S.d_chg, c->stream));
@@ -1685,8 +1691,8 @@ int mdk_score_companion(mdk_ctx *c, const float *rotcoef, const float *t, int B,
     HIPCHK(hipSetDevice(c->device));
     for (int p0 = 0; p0 < B; p0 += kPoses) {
         const size_t np = std::min(kPoses, B - p0);
-        if (upload_poses(c, rotcoef + 9 * (size_t)p0, t + 3 * (size_t)p0, np, 7)) return 1;
-        float *d = c->d_posework;
+        if (upload_poses(c, rotcoef + 9 * (size_t)p0, t + 3 * (size_t)p0, np)) return 1;
+        float *d = c->d_pose;
         HIPCHK(launch_companion(c->lig, c->d_wshape, c->d_recgrid, d, d + 9 * np, (int)np, c->nf, c->d_cpart, d + 12 * np,
                                 c->stream));
         if (download_poses(c, out + 7 * (size_t)p0, np, 7)) return 1;

@@ -595,7 +595,7 @@ struct mdk_ctx {
     int inv_variant = 2;      // MDK_INV_VARIANT: fused-inverse variant (tuning)
     int fwd_variant = 0;      // MDK_FWD_VARIANT: 0 fused forward z + y, prefetching (nf = 256: over half planes), 1 separate passes, 2 fused, not prefetching
     float2 *d_rec = nullptr;
-    float2 *d_recp = nullptr;  // d_rec as pairs of columns, for the specialised pipeline (k_rec_pairs)
+    float2 *d_recp = nullptr;  // behind it, d_rec as pairs of columns, for the specialised pipeline (k_rec_pairs)
     bool have_rec = false, have_lig = false;
     // ligand
     float *d_xyz = nullptr, *d_rc2 = nullptr, *d_rs2 = nullptr, *d_charge = nullptr, *d_gc = nullptr;
@@ -935,8 +935,11 @@ int mdk_create(int device, int nf, int ng, int na, int t, int max_batch, mdk_ctx
             return bail(fail("mdk_create: stream creation failed"));
     c->stream = c->slot[0].stream;
     const size_t nf3 = (size_t)nf * nf * nf, ng3 = (size_t)ng * ng * ng, B = max_batch;
-    if (pipe_available(nf) && dmalloc(&c->d_recp, (size_t)nf * nf * 2 * c->Hp)) return bail(1);
-    if (dmalloc(&c->d_tw, tw.size()) || dmalloc(&c->d_rec, nf3) || dmalloc(&c->d_xyz, 3 * (size_t)na) ||
+    // one allocation for the receptor's two forms (another of this size takes 12 us)
+    const size_t rec_n = (nf3 + 31) / 32 * 32, pairs = pipe_available(nf) ? (size_t)nf * nf * 2 * c->Hp : 0;
+    if (dmalloc(&c->d_rec, rec_n + pairs)) return bail(1);
+    if (pairs) c->d_recp = c->d_rec + rec_n;
+    if (dmalloc(&c->d_tw, tw.size()) || dmalloc(&c->d_xyz, 3 * (size_t)na) ||
         dmalloc(&c->d_rc2, na) || dmalloc(&c->d_rs2, na) || dmalloc(&c->d_charge, na) || dmalloc(&c->d_gc, ng) ||
         dmalloc(&c->d_brot, 9 * B) || dmalloc(&c->d_bid, B) || dmalloc(&c->d_recgrid, ng3) ||
         dmalloc(&c->d_wshape, na) ||
@@ -1025,7 +1028,7 @@ int mdk_destroy(mdk_ctx *c) {
     (void)hipSetDevice(c->device);
     for (int k = 0; k < mdk_ctx::kMaxSlots; k++)
         if (c->slot[k].stream) (void)hipStreamSynchronize(c->slot[k].stream);
-    void *ptrs[] = {c->d_tw, c->d_tw4, c->d_rec, c->d_recp, c->d_xyz, c->d_rc2, c->d_rs2, c->d_charge, c->d_gc, c->d_rot,
+    void *ptrs[] = {c->d_tw, c->d_tw4, c->d_rec, c->d_xyz, c->d_rc2, c->d_rs2, c->d_charge, c->d_gc, c->d_rot,
                     c->d_rotid, c->d_brot, c->d_bid, c->d_results, c->d_topn_scratch, c->d_topn_out,
                     c->d_recgrid, c->d_wshape, c->d_gph, c->d_gpart, c->d_cpart, c->d_rpsc, c->d_btrans, c->d_dsum, c->d_recwork, c->d_pose};
     for (void *p : ptrs)

@@ -32,8 +32,11 @@ struct RecAtoms {
     float gw;
 };
 
-// the voxel holding coordinate p along one axis (src/receptor.cpp:73-83)
-__device__ __forceinline__ int cell_of(float p, float gw, int ng) { return (int)(p / gw + ng / 2); }
+// the voxel holding coordinate p along one axis (src/receptor.cpp:73-83); kept away from the ends of the
+// integers, where an infinite coordinate's box would wrap to a size above 0 far outside the arrays
+__device__ __forceinline__ int cell_of(float p, float gw, int ng) {
+    return min(max((int)(p / gw + ng / 2), -(1 << 24)), 1 << 24);
+}
 
 __device__ __forceinline__ float sq_dist(float p, float g) {
     const float d = p - g;

@@ -237,14 +237,17 @@ __global__ void __launch_bounds__(kChargeThreads)
 }
 
 // The same with the voxels' counts and sums in an LDS table of nt entries (a power of two, three
-// times na where there is room: probes stay under 15; never less than 1.6 times): tab holds
+// times na where there is room, never less than 1.6 times): tab holds
 // (voxel + 1) << 13 | atoms, 0 if free, linear probing.  One workgroup.  The global counts cost an
 // atomic and a read on a line of their own for every atom, the sums another: 20 us of the 52 that
 // a batch of 128 rotations of 2081 atoms took; the table takes 9.
+// The slot is the leading bits of a product.  An atom's probes depend on how the factor takes to the grid's
+// rows and planes: for balls of 50 to 5120 atoms on every grid from 24 to 75 they were 1.33 on average, the
+// longest chain 12 on average and 48 at worst; with 2654435761 1.52, 16 and 131 (grid 75, where one
+// rotation of 5100 atoms took 184 us, 171 with the counts in memory; now 121).
 constexpr int kCountBits = 13, kTableMax = 8192;
-__device__ __forceinline__ uint32_t table_slot(int v, int nt) {  // the product's leading bits
-    return (uint32_t)v * 2654435761u >> (__clz(nt) + 1);
-}
+__device__ __forceinline__ uint32_t table_slot(int v, int nt) { return (uint32_t)v * 0xcc9e2d51u >> (__clz(nt) + 1); }
+
 __device__ __forceinline__ void vox_charges_lds(const int *vi, const float *__restrict__ charge, float *g, int na,
                                                 uint32_t *tab, float *sum, int nt, int2 *list) {
     __shared__ int nlist;

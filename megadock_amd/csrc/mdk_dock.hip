@@ -70,7 +70,11 @@ constexpr int WZ = 16;   // lines per workgroup, z passes
 constexpr int WY = 16;   // lines per workgroup, y passes
 constexpr int WX = 8;    // kz columns per workgroup in the x pass (plus 8 partner columns)
 constexpr int kThreads = 256;  // threads per workgroup, where not chosen by the size
-constexpr size_t kDirectResults = 256;  // mdk_dock: as many results go straight to host memory
+// mdk_dock: as many results go straight to host memory.  The line is the size of the block that a context
+// keeps for it, not where copies become the better way: 64 results at 64^3 take 158 us against 198 with
+// copies, 256 results 298-509 against 329-530, 512 961 against 1011; 1024 (16 a rotation, 80^3) 490 against
+// 600, at 200^3 512 results 5.84 ms against 5.82.
+constexpr size_t kDirectResults = 256;
 // off-grid scores: poses a block, and words a pose (rotation, translation, at most seven results)
 constexpr int kPoses = 65536, kPoseWords = 19;
 
@@ -669,7 +673,8 @@ size_t lds_inv_z(const mdk_ctx *c, int nt, int t) {
 // and 1024 threads take 7.9, 8.3, 16.3 ms at 130 (four workgroups a CU), 8.3, 7.0, 13.0 at 156 and 10.9,
 // 8.0, 10.6 at 260 (two or three), 19.8, 12.9, 10.4 at 324 (one).  At 360 with 256 threads
 // and integer divisions, 16 rotations took 14.8 ms in the x pass, 11.4 in the inverse z, 5.3 in the inverse
-// y, 4.3 and 2.9 in the forward y and z passes; now 6.5, 3.8, 2.1, 1.8 and 0.9.
+// y, 4.3 and 2.9 in the forward y and z passes; now 6.5, 3.8, 2.1, 1.8 and 1.3 (which reads the voxelized
+// batch itself; expanding it was a launch of its own).
 int generic_threads(const mdk_ctx *c) {
     const size_t lds = lds_bytes(c, 16) + 2048;
     return lds > 80 * 1024 || c->nf > 320 ? 1024 : lds > 40 * 1024 || c->nf > 160 ? 512 : 256;
@@ -1667,7 +1672,6 @@ int mdk_score_spectral(mdk_ctx *c, const float *rotcoef, const float *t, int B, 
     if (B < 0) return fail("mdk_score_spectral: negative batch size");
     if (!c->use_pipe)
         return fail("mdk_score_spectral: needs an FFT size with specialised kernels (and MDK_FORCE_GENERIC unset)");
-    if (c->H > 192) return fail("mdk_score_spectral: nf above 382 (three kz per lane in the evaluation)");
     HIPCHK(hipSetDevice(c->device));
     BatchSlot &S = c->slot[0];
     for (int p0 = 0; p0 < B; p0 += kPoses) {

@@ -302,8 +302,11 @@ __device__ __forceinline__ void vox_charges_lds(const int *vi, const float *__re
 // charges by a table of nt entries (else k_vox_charge follows).  For one rotation it is a chain of dependent steps in
 // one workgroup: with a thread per atom walking five planes, the grid's coordinates loaded from
 // memory inside its loops, a ligand of 336 atoms took 21.6 us and its charges a launch of 4.2 us.  Now
-// 12 together.
+// VOX_FIGURE together.
 constexpr int kVoxLdsThreads = kChargeThreads;
+// Atoms up to which an atom's planes go to five threads.  One rotation of 200, 336, 512, 800 and 2081 atoms at 80^3
+// takes 16.0, 21.9, 26.5, 37.0 and 88.5 us with five threads an atom, 18.6, 22.8, 25.4, 33.4 and 76.9
+// with one (with the events that time it); 128 rotations 24.9, 33.0, 38.4, 56.7, 119 and 26.6, 34.4, 38.0, 54.3, 107.
 constexpr int kVoxSplitAtoms = 512;
 __global__ void __launch_bounds__(kVoxLdsThreads)
     k_vox_lds(LigandDev L, const float *__restrict__ rot, const int *__restrict__ boff, uint32_t *dmo, uint32_t *cnt,
@@ -484,7 +487,9 @@ hipError_t launch_voxelize(const LigandDev &lig, const float *rot, int B, const 
         k_vox_masks<<<dim3((mw + 255) / 256, B), 256, 0, s>>>(vs.cs, vs.dmo, ng, mw, lig.delta);
         k_vox_charge<<<B, kChargeThreads, 0, s>>>(vidx, vs.cnt, lig.charge, chg, lig.na, ng3, cw);
     } else {
-        // slabs of 64 KB of masks (two workgroups a CU), or up to 132 KB where that is fewer than 12 planes
+        // Slabs of 64 KB of masks (two workgroups a CU), or up to 132 KB where that is fewer than 12 planes.
+        // Always 132 KB: 3-12% more time for 8 and 32 rotations at 160^3 to 320^3, 5% less for 64 at 216^3 and
+        // 256^3.  Always 64 KB: within 4% of this either way, above 137 planes (where they differ) as well.
         const size_t plane = 2 * sizeof(uint32_t) * (size_t)ng * row_words(ng);
         const int with_halo = (int)std::max((size_t)64 * 1024 / plane, std::min((size_t)12, kVoxLdsBytes / plane));
         const int planes = with_halo - 4;

@@ -237,10 +237,11 @@ __global__ void __launch_bounds__(1024) k_wide_compact(const float *__restrict__
 // rotation, each workgroup for itself, from the histogram that the launch before left; the
 // sixth (level 5) writes the keys from the threshold on, rank of them.  The histograms take turns in three
 // places of the rotation's keys: level l - 1 is read, l added to, l + 1 cleared.  Without such
-// rotations a launch ends at its first load (six of them: 1-5 us a call).  Docking one rotation with
-// every score equal, t = 64, took 9.1 ms at 112^3 and 106 at 256^3 with one workgroup that read the map
-// nine times, 0.30 and 0.77 with levels of 8 bits in 17 launches over every rotation, and takes 0.19
-// and 0.42; 128 such rotations of 112^3 14.3, 5.8 and 3.1.
+// rotations a launch ends at its first load: six of them take 10-14 us of a call of one rotation, under 1%
+// of a search (112^3, 1024 rotations on two streams: 11.77 ms without, 11.86 with).  Docking one rotation
+// with every score equal, t = 64, took 9.1 ms at 112^3 and 106 at 256^3 with one workgroup that read the
+// map nine times, 0.30 and 0.77 with levels of 8 bits in 17 launches over every rotation, and takes 0.19
+// and 0.41; 128 such rotations of 112^3 14.3, 5.8 and 3.1 (with 256 threads a workgroup 4.2, in twice as many 3.4).
 __device__ __forceinline__ unsigned long long level_key(float v, float nf3f, unsigned i) {
     return ((unsigned long long)sortable(v / nf3f + 0.0f) << 28) | (0xfffffffu - i);
 }

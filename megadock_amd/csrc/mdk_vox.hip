@@ -302,7 +302,7 @@ __device__ __forceinline__ void vox_charges_lds(const int *vi, const float *__re
 // charges by a table of nt entries (else k_vox_charge follows).  For one rotation it is a chain of dependent steps in
 // one workgroup: with a thread per atom walking five planes, the grid's coordinates loaded from
 // memory inside its loops, a ligand of 336 atoms took 21.6 us and its charges a launch of 4.2 us.  Now
-// VOX_FIGURE together.
+// 14 together.
 constexpr int kVoxLdsThreads = kChargeThreads;
 // Atoms up to which an atom's planes go to five threads.  One rotation of 200, 336, 512, 800 and 2081 atoms at 80^3
 // takes 16.0, 21.9, 26.5, 37.0 and 88.5 us with five threads an atom, 18.6, 22.8, 25.4, 33.4 and 76.9

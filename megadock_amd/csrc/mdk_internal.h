@@ -86,11 +86,10 @@ struct TopTState {
     unsigned done;                    // the threshold is prefix (its lower bits zero)
     unsigned hist[256];
     // t up to kWideT: whether this rotation's list does not fit; the rotations of the batch where it
-    // does not (how many in state 0, the k-th in state k); their prefix and wanted entries before
-    // the histogram of a level (wanted 0: the threshold is the prefix)
+    // does not (how many in state 0, the k-th in state k); the least quotients of the two histograms
+    // that follow there, the entries wanted from the second on, and how many above the t-th are listed
     unsigned over, nover, nth_over;
-    unsigned long long level_prefix[5];
-    unsigned level_wanted[5];
+    unsigned base, fine_base, fine_want, above;
 };
 // keys that launch_topt keeps per rotation for t results per rotation (a power of two)
 unsigned topt_sort_size(int t, int nf);

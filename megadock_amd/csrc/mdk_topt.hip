@@ -22,8 +22,9 @@
 //      score, and with its lower edge a score below which no key can reach the top t
 //      (quotient_cut);
 //   2. the scores not below it, typically a few times t, become the keys that step 3 sorts.
-// A rotation with more of them than fit (many equal scores) is selected by levels of 12 bits
-// (k_wide_level), all workgroups sharing those rotations.
+// A rotation with more of them than fit (many equal scores) has its t-th score found in two
+// further histograms (k_wide_compact, k_wide_value), and of the entries that equal it the first
+// ones are taken (k_wide_ties), all workgroups sharing those rotations.
 #include <hip/hip_runtime.h>
 
 #include "mdk_internal.h"
@@ -37,10 +38,15 @@ constexpr int kTSortLds = 8192;  // keys sorted in LDS
 // its ties; above, the bucket alone may not fit.
 constexpr int kWideT = kTSortLds / 16, kWideShift = 19, kWideBuckets = 1 << (32 - kWideShift);
 constexpr unsigned kWideChunk = 32768;  // map entries per workgroup: 32 KB of buckets are cleared and added for 128 KB
-constexpr int kLevels = 5, kLevelBuckets = 4096, kLevelBlocks = 512;  // two workgroups a CU
-static_assert(3 * kLevelBuckets * sizeof(unsigned) <= kTSortLds * sizeof(unsigned long long) &&
-                  kWideT * sizeof(unsigned long long) <= kLevelBuckets * sizeof(unsigned),
-              "the levels' histograms lie where the keys go, the last one picked clear of the keys written");
+// Rotations whose list does not fit: histograms of 2^10 quotients a bucket, at the start of the
+// rotation's keys, and of single ones, behind the kTieKeys keys that are kept.  A wide bucket is 2^19
+// neighbouring scores of one binade, and a division leaves at most twice as many units of the last place
+// between them, so its quotients fall into buckets 0 .. 1024; the last bucket takes what lies above.
+constexpr int kCoarseShift = 10, kCoarse = 2048, kFine = 1 << kCoarseShift;
+constexpr int kTieThreads = 512, kTieBlocks = 512;
+constexpr unsigned kTieKeys = kTSortLds - kFine * sizeof(unsigned) / sizeof(unsigned long long);
+static_assert(kCoarse * sizeof(unsigned) <= kTieKeys * sizeof(unsigned long long) && kTieKeys >= 2 * kWideT,
+              "the histograms lie where the keys go; the second clear of the keys written");
 static_assert(kWideBuckets * sizeof(unsigned) <= kTSortLds * sizeof(unsigned long long),
               "the histogram lies where the keys go");
 
@@ -54,6 +60,7 @@ __device__ __forceinline__ unsigned long long topt_key(float v, float nf3f, unsi
 }
 
 __device__ __forceinline__ unsigned sortable_score(float v) { return sortable(v + 0.0f); }  // -0 as +0
+__device__ __forceinline__ unsigned sortable_quotient(float v, float nf3f) { return sortable(v / nf3f + 0.0f); }  // as topt_key
 
 __device__ __forceinline__ float key_float(unsigned long long k) {
     const unsigned u = (unsigned)(k >> 32);
@@ -157,7 +164,7 @@ __global__ void __launch_bounds__(1024) k_wide_hist(const float *__restrict__ sm
 
 // one workgroup per rotation: the score below which nothing reaches the top `rank` (in st.prefix, as
 // sortable bits), and whether the entries of the buckets down to that score's fit the list; if not,
-// the rotation's first level histogram is cleared
+// st.base is the least quotient of the bucket, as sortable bits, and the rotation's histograms are cleared
 __global__ void __launch_bounds__(1024) k_wide_pick(TopTState *st, unsigned long long *keys, unsigned rank, float nf3f) {
     constexpr int PER = kWideBuckets / 1024;
     __shared__ unsigned cum[1024], cut_bits;
@@ -188,6 +195,7 @@ __global__ void __launch_bounds__(1024) k_wide_pick(TopTState *st, unsigned long
         const float cut = quotient_cut(key_float(edge), nf3f);
         over = cut != cut;  // a bucket of what is not a number
         cut_bits = sortable_score(cut);
+        st[blockIdx.x].base = sortable_quotient(key_float(edge), nf3f);
     }
     __syncthreads();
     const int last = (int)(cut_bits >> kWideShift);
@@ -204,14 +212,31 @@ __global__ void __launch_bounds__(1024) k_wide_pick(TopTState *st, unsigned long
     }
     __syncthreads();
     if (over)
-        for (int q = threadIdx.x; q < kLevelBuckets; q += 1024) h[q] = 0u;
+        for (int q = threadIdx.x; q < kCoarse; q += 1024) {
+            h[q] = 0u;
+            if (q < kFine) h[2 * kTieKeys + q] = 0u;
+        }
 }
 
-// grid (chunks, B): the keys of the scores not below the cut, of rotations where they fit
+// Adds one to h[bucket] for the lanes that are `in`.  Equal buckets are the rule here: one lane adds
+// for all that have the first one's.
+__device__ __forceinline__ void add_bucket(unsigned *h, bool in, int bucket) {
+    const unsigned long long some = __ballot(in);
+    if (some == 0ull) return;
+    const int first = __ffsll((long long)some) - 1, b0 = __builtin_amdgcn_readlane(bucket, first);
+    const unsigned long long same = __ballot(in && bucket == b0);
+    if ((int)(threadIdx.x & 63) == first)
+        atomicAdd(&h[b0], (unsigned)__popcll(same));
+    else if (in && bucket != b0)
+        atomicAdd(&h[bucket], 1u);
+}
+
+// grid (chunks, B): the keys of the scores not below the cut, of rotations where they fit; of the others,
+// the quotients from st.base on by kCoarseShift bits
 __global__ void __launch_bounds__(1024) k_wide_compact(const float *__restrict__ smap, unsigned n3, float nf3f,
                                                        TopTState *st, unsigned long long *keys) {
+    __shared__ unsigned h[kCoarse];
     TopTState &s = st[blockIdx.y];
-    if (s.over) return;  // uniform
     const unsigned cut = (unsigned)s.prefix;
     const float4 *m = reinterpret_cast<const float4 *>(smap + (size_t)blockIdx.y * n3);
     unsigned long long *out = keys + (size_t)blockIdx.y * kTSortLds;
@@ -219,6 +244,25 @@ __global__ void __launch_bounds__(1024) k_wide_compact(const float *__restrict__
         if (sortable_score(v) >= cut) out[atomicAdd(&s.count, 1u)] = topt_key(v, nf3f, i);
     };
     const unsigned i0 = blockIdx.x * (kWideChunk / 4), i1 = min(n3 / 4, i0 + kWideChunk / 4);
+    if (s.over) {  // uniform
+        const unsigned base = s.base;
+        for (int q = threadIdx.x; q < kCoarse; q += 1024) h[q] = 0u;
+        __syncthreads();
+        for (unsigned i = i0 + threadIdx.x; i < i1; i += 1024u) {
+            const float4 v = m[i];
+            const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const unsigned q = sortable_quotient(e[k], nf3f);
+                add_bucket(h, q >= base, (int)min((q - base) >> kCoarseShift, (unsigned)kCoarse - 1u));
+            }
+        }
+        __syncthreads();
+        unsigned *g = reinterpret_cast<unsigned *>(out);
+        for (int q = threadIdx.x; q < kCoarse; q += 1024)
+            if (h[q]) atomicAdd(&g[q], h[q]);
+        return;
+    }
     for (unsigned i = i0 + threadIdx.x; i < i1; i += 1024u) {
         const float4 v = m[i];
         if (sortable_score(v.x) >= cut || sortable_score(v.y) >= cut || sortable_score(v.z) >= cut || sortable_score(v.w) >= cut) {
@@ -230,46 +274,140 @@ __global__ void __launch_bounds__(1024) k_wide_compact(const float *__restrict__
     }
 }
 
-// Rotations whose keys do not fit: radix select of the keys
-//   sortable(score / nf^3) << 28 | (2^28 - 1 - index)          (60 bits; nf <= 640)
-// by five levels of 12 bits, a launch each, whose workgroups share out those rotations (with one
-// rotation all of them read its map).  A launch first picks the last level's digit of its
-// rotation, each workgroup for itself, from the histogram that the launch before left; the
-// sixth (level 5) writes the keys from the threshold on, rank of them.  The histograms take turns in three
-// places of the rotation's keys: level l - 1 is read, l added to, l + 1 cleared.  Without such
-// rotations a launch ends at its first load: six of them take 10-14 us of a call of one rotation, under 1%
-// of a search (112^3, 1024 rotations on two streams: 11.77 ms without, 11.86 with).  Docking one rotation
-// with every score equal, t = 64, took 9.1 ms at 112^3 and 106 at 256^3 with one workgroup that read the
-// map nine times, 0.30 and 0.77 with levels of 8 bits in 17 launches over every rotation, and takes 0.19
-// and 0.41; 128 such rotations of 112^3 14.3, 5.8 and 3.1 (with 256 threads a workgroup 4.2, in twice as many 3.4).
-__device__ __forceinline__ unsigned long long level_key(float v, float nf3f, unsigned i) {
-    return ((unsigned long long)sortable(v / nf3f + 0.0f) << 28) | (0xfffffffu - i);
+// The bucket of the want-th entry from the top of a histogram of PER * kTieThreads buckets, and how many of
+// its entries are wanted; by every workgroup for itself.
+struct Picked {
+    int bucket;
+    unsigned want;
+};
+template <int PER> __device__ __forceinline__ Picked pick_from_top(const unsigned *hist, unsigned want) {
+    __shared__ unsigned wave_sum[kTieThreads / 64];
+    __shared__ Picked picked;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, top = PER * kTieThreads - 1 - PER * tid;
+    unsigned in[PER], s = 0u;
+#pragma unroll
+    for (int k = 0; k < PER; k++) s += in[k] = hist[top - k];
+    unsigned c = s;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const unsigned o = __shfl_up(c, d, 64);
+        if (lane >= d) c += o;
+    }
+    if (lane == 63) wave_sum[wave] = c;
+    if (tid == 0) picked = Picked{0, want};
+    __syncthreads();
+    for (int w = 0; w < wave; w++) c += wave_sum[w];
+    if (c - s < want && c >= want) {
+        int b = top;
+        unsigned a = c - s;
+#pragma unroll
+        for (int k = 0; k + 1 < PER; k++)
+            if (b == top - k && a + in[k] < want) {
+                a += in[k];
+                b--;
+            }
+        picked = Picked{b, want - a};
+    }
+    __syncthreads();
+    const Picked p = picked;
+    __syncthreads();  // the next rotation's
+    return p;
 }
 
-__global__ void __launch_bounds__(1024) k_wide_level(const float *__restrict__ smap, unsigned n3, float nf3f,
-                                                     TopTState *st, unsigned long long *keys, unsigned rank, int level) {
-    __shared__ unsigned h[kLevelBuckets], wave_sum[16], picked[3];
-    const unsigned n = st[0].nover, parts = max(1u, gridDim.x / max(n, 1u));
+// Rotations whose keys do not fit: k_wide_compact has their quotients by 2^10 from the wide bucket's least on,
+// k_wide_value counts the single quotients of the bucket that holds the t-th one, and k_wide_ties takes
+// the entries above that quotient and, of those that equal it, the first ones of each share of the map, as many as are
+// wanted of all: the final sort drops what is too many.  A launch's workgroups share out the rotations (with
+// one, all of them read its map).  Without such rotations the two launches end at their first load, but each
+// still waits until the other stream's kernels leave room for it: a search of 112^3, 1024 rotations, t = 64,
+// takes 12.20 ms with 512 threads a workgroup, 12.33 with 1024 (12.19 with one launch of one workgroup a
+// rotation; five levels of 12 bits in six launches of 1024 threads took 1.6 to 3.4% more than that).  Docking
+// with every score equal takes 0.39 ms a rotation of 112^3 with t = 64, 0.60 and 0.90 of 256^3 with t = 64
+// and 512, 2.58 ms 128 rotations of 112^3 (8.98, 106, 100 and 14.1 ms with one workgroup a rotation).
+struct TieShare {  // this workgroup's part of the rotations q0, q0 + step, ...
+    unsigned n, parts, part, q0;
+};
+__device__ __forceinline__ TieShare tie_share(const TopTState *st) {
+    const unsigned n = st[0].nover;
+    if (n == 0u) return TieShare{0u, 1u, 0u, 0u};
+    if (n >= gridDim.x) return TieShare{n, 1u, 0u, blockIdx.x};
+    const unsigned part = blockIdx.x / n, parts = gridDim.x / n;
+    return TieShare{part < parts ? n : 0u, parts, part, blockIdx.x % n};
+}
+
+__global__ void __launch_bounds__(kTieThreads) k_wide_value(const float *__restrict__ smap, unsigned n3, float nf3f,
+                                                     TopTState *st, unsigned long long *keys, unsigned rank) {
+    __shared__ unsigned h[kFine];
+    const TieShare T = tie_share(st);
+    const int tid = threadIdx.x;
+    for (unsigned q = T.q0; q < T.n; q += gridDim.x) {  // uniform
+        const unsigned b = st[q].nth_over;
+        TopTState &S = st[b];
+        unsigned *hist = reinterpret_cast<unsigned *>(keys + (size_t)b * kTSortLds);
+        const Picked p = pick_from_top<kCoarse / kTieThreads>(hist, rank);
+        const unsigned base = S.base + ((unsigned)p.bucket << kCoarseShift);
+        if (T.part == 0 && tid == 0) {
+            S.fine_base = base;
+            S.fine_want = p.want;
+            S.above = 0u;
+        }
+        for (int k = tid; k < kFine; k += kTieThreads) h[k] = 0u;
+        __syncthreads();
+        const unsigned share = (n3 / 4 + T.parts - 1) / T.parts, i0 = T.part * share, i1 = min(n3 / 4, i0 + share);
+        const float4 *m = reinterpret_cast<const float4 *>(smap + (size_t)b * n3);
+        for (unsigned i = i0 + tid; i < i1; i += (unsigned)kTieThreads) {
+            const float4 f = m[i];
+            const float e[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const unsigned d = sortable_quotient(e[k], nf3f) - base;
+                add_bucket(h, d < (unsigned)kFine, (int)d);
+            }
+        }
+        __syncthreads();
+        for (int k = tid; k < kFine; k += kTieThreads)
+            if (h[k]) atomicAdd(&hist[2 * kTieKeys + k], h[k]);
+        __syncthreads();  // the next rotation clears h
+    }
+}
+
+__global__ void __launch_bounds__(kTieThreads) k_wide_ties(const float *__restrict__ smap, unsigned n3, float nf3f,
+                                                    TopTState *st, unsigned long long *keys, unsigned rank) {
+    __shared__ unsigned wave_sum[kTieThreads / 64];
+    const TieShare T = tie_share(st);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const unsigned part = n < gridDim.x ? blockIdx.x / max(n, 1u) : 0u;
-    if (part >= parts) return;  // uniform, as all that follows but the entries
-    for (unsigned q = n < gridDim.x ? blockIdx.x % max(n, 1u) : blockIdx.x; q < n; q += gridDim.x) {
+    for (unsigned q = T.q0; q < T.n; q += gridDim.x) {  // uniform
         const unsigned b = st[q].nth_over;
         TopTState &S = st[b];
         unsigned long long *out = keys + (size_t)b * kTSortLds;
-        unsigned *hist = reinterpret_cast<unsigned *>(out);
-        unsigned long long prefix = 0ull;
-        unsigned want = rank;
-        if (level > 0) {
-            prefix = S.level_prefix[level - 1];
-            want = S.level_wanted[level - 1];
-        }
-        if (level > 0 && want > 0) {
-            // this thread's buckets: 4095 - 4 tid downwards
-            const unsigned *last = hist + (level - 1) % 3 * kLevelBuckets;
-            const uint4 v = reinterpret_cast<const uint4 *>(last)[1023 - tid];
-            const unsigned s = v.x + v.y + v.z + v.w;
-            unsigned c = s;
+        const Picked p = pick_from_top<kFine / kTieThreads>(reinterpret_cast<const unsigned *>(out) + 2 * kTieKeys, S.fine_want);
+        const unsigned value = S.fine_base + (unsigned)p.bucket, want = p.want, above = rank - want;
+        // above + parts * want <= kTieKeys
+        const unsigned parts = min(T.parts, (kTieKeys - (unsigned)kWideT) / want);
+        if (T.part >= parts) continue;
+        if (T.part == 0 && tid == 0) S.count = above + parts * want;
+        unsigned long long *mine = out + above + T.part * want;
+        const unsigned share = (n3 / 4 + parts - 1) / parts, i0 = T.part * share, i1 = min(n3 / 4, i0 + share);
+        const float4 *m = reinterpret_cast<const float4 *>(smap + (size_t)b * n3);
+        unsigned found = 0u;  // entries of this share that equal the value, in index order
+        for (unsigned r = i0; r < i1; r += (unsigned)kTieThreads) {
+            const unsigned i = r + tid;
+            const bool on = i < i1;
+            const float4 f = on ? m[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+            const float e[4] = {f.x, f.y, f.z, f.w};
+            unsigned equal = 0u;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const unsigned s = sortable_quotient(e[k], nf3f);
+                if (on && s > value) {
+                    const unsigned at = atomicAdd(&S.above, 1u);
+                    if (at < above) out[at] = topt_key(e[k], nf3f, 4 * i + k);
+                }
+                equal |= (unsigned)(on && s == value) << k;
+            }
+            if (found >= want || !__syncthreads_or((int)equal)) continue;  // uniform
+            unsigned c = __popc(equal);
+            const unsigned n = c;
 #pragma unroll
             for (int d = 1; d < 64; d <<= 1) {
                 const unsigned o = __shfl_up(c, d, 64);
@@ -277,73 +415,21 @@ __global__ void __launch_bounds__(1024) k_wide_level(const float *__restrict__ s
             }
             if (lane == 63) wave_sum[wave] = c;
             __syncthreads();
-            for (int w = 0; w < wave; w++) c += wave_sum[w];
-            const unsigned above = c - s;
-            if (above < want && c >= want) {
-                const unsigned in[4] = {v.w, v.z, v.y, v.x};
-                unsigned digit = kLevelBuckets - 1 - 4 * tid, a = above, here = in[0];
+            unsigned at = found + c - n, all = 0u;
+            for (int w = 0; w < kTieThreads / 64; w++) {
+                if (w < wave) at += wave_sum[w];
+                all += wave_sum[w];
+            }
 #pragma unroll
-                for (int k = 1; k < 4; k++)
-                    if (a + here < want) {
-                        a += here;
-                        here = in[k];
-                        digit--;
-                    }
-                picked[0] = digit;
-                picked[1] = want - a;
-                picked[2] = want - a == here;  // the whole bucket is wanted
-            }
-            __syncthreads();
-            prefix |= (unsigned long long)picked[0] << (60 - 12 * level);
-            want = picked[2] ? 0u : picked[1];
-            __syncthreads();  // the next rotation writes them
+            for (int k = 0; k < 4; k++)
+                if (equal >> k & 1u) {
+                    if (at < want) mine[at] = topt_key(e[k], nf3f, 4 * i + k);
+                    at++;
+                }
+            found += all;
+            __syncthreads();  // the next round writes wave_sum
         }
-        // this workgroup's share of the map, in fours
-        const unsigned share = (n3 / 4 + parts - 1) / parts, i0 = part * share, i1 = min(n3 / 4, i0 + share);
-        const float4 *m = reinterpret_cast<const float4 *>(smap + (size_t)b * n3);
-        if (level == kLevels) {
-            for (unsigned i = i0 + tid; i < i1; i += 1024u) {
-                const float4 f = m[i];
-                const float e[4] = {f.x, f.y, f.z, f.w};
-#pragma unroll
-                for (int k = 0; k < 4; k++)
-                    if (level_key(e[k], nf3f, 4 * i + k) >= prefix)
-                        out[atomicAdd(&S.count, 1u)] = topt_key(e[k], nf3f, 4 * i + k);
-            }
-            continue;
-        }
-        if (part == 0) {
-            if (tid == 0) {
-                S.level_prefix[level] = prefix;
-                S.level_wanted[level] = want;
-            }
-            for (int k = tid; k < kLevelBuckets; k += 1024) hist[(level + 1) % 3 * kLevelBuckets + k] = 0u;
-        }
-        if (want == 0u) continue;
-        for (int k = tid; k < kLevelBuckets; k += 1024) h[k] = 0u;
-        __syncthreads();
-        const int shift = 48 - 12 * level;
-        for (unsigned i = i0 + tid; i < i1; i += 1024u) {
-            const float4 f = m[i];
-            const float e[4] = {f.x, f.y, f.z, f.w};
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const unsigned long long key = level_key(e[k], nf3f, 4 * i + k);
-                const bool in = level == 0 || key >> (shift + 12) == prefix >> (shift + 12);
-                const int digit = (int)(key >> shift) & (kLevelBuckets - 1);
-                // equal digits are the rule here: one lane adds for all that have the first one's
-                const unsigned long long some = __ballot(in);
-                if (some == 0ull) continue;
-                const int first = __ffsll((long long)some) - 1, d0 = __builtin_amdgcn_readlane(digit, first);
-                const unsigned long long same = __ballot(in && digit == d0);
-                if (lane == first) atomicAdd(&h[d0], (unsigned)__popcll(same));
-                else if (in && digit != d0) atomicAdd(&h[digit], 1u);
-            }
-        }
-        __syncthreads();
-        for (int k = tid; k < kLevelBuckets; k += 1024)
-            if (h[k]) atomicAdd(&hist[level % 3 * kLevelBuckets + k], h[k]);
-        __syncthreads();  // the next rotation clears h
+        for (unsigned k = found + tid; k < want; k += (unsigned)kTieThreads) mine[k] = 0ull;  // sorts last
     }
 }
 
@@ -422,8 +508,8 @@ hipError_t launch_topt(const float *smap, int B, int nf, int t, TopTState *st, u
         k_wide_hist<<<wide, 1024, 0, s>>>(smap, n3, keys);
         k_wide_pick<<<B, 1024, 0, s>>>(st, keys, rank, nf3f);
         k_wide_compact<<<wide, 1024, 0, s>>>(smap, n3, nf3f, st, keys);
-        for (int level = 0; level <= kLevels; level++)
-            k_wide_level<<<kLevelBlocks, 1024, 0, s>>>(smap, n3, nf3f, st, keys, rank, level);
+        k_wide_value<<<kTieBlocks, kTieThreads, 0, s>>>(smap, n3, nf3f, st, keys, rank);
+        k_wide_ties<<<kTieBlocks, kTieThreads, 0, s>>>(smap, n3, nf3f, st, keys, rank);
         k_tsel_sort_out<<<B, 1024, 0, s>>>(keys, P, 0u, st, t, nf, out, rot_id, boff);
         return hipGetLastError();
     }

@@ -55,6 +55,27 @@ def test_few_values(lig, nf, t, values):
     c.close()
 
 
+@pytest.mark.parametrize("nf,t", [(22, 17), (64, 33), (64, 512), (112, 64), (144, 512)])
+@pytest.mark.parametrize("kind", ["close", "along_z", "along_x"])
+def test_one_wide_bucket(lig, nf, t, kind):
+    """Scores that differ but lie within 6% of each other, and equal ones that lie apart in the map."""
+    rng = np.random.default_rng(nf + t)
+    re, im = np.zeros((nf, nf, nf), np.float32), np.zeros((nf, nf, nf), np.float32)
+    if kind == "close":
+        re[0, 0, 0] = 1e5
+        re[:3, :3, 1:4], im[:3, :3, 1:4] = rng.normal(size=(2, 3, 3, 3)).astype(np.float32)
+    else:
+        re[(0, 0, nf // 2) if kind == "along_z" else (nf // 2, 0, 0)] = 1.0
+    c = _ctx(lig, nf, t, 2)
+    c.set_receptor_spectrum(re, im)
+    rot = M.rotation_coefs(M.rotation_set(24)[[3, 11]])
+    got = c.dock(rot, np.arange(2, dtype=np.int32)).reshape(2, t)
+    for b in range(2):
+        print("nf=%d t=%d %s rotation %d" % (nf, t, kind, b), flush=True)
+        _check(got[b], c.score_map(rot[b]), nf, t)
+    c.close()
+
+
 def test_beside_other_maps(golden_dir, lig):
     """A ligand off its centre: rotations that carry it out of the grid give maps of zeros."""
     nf, t = 64, 40
@@ -90,7 +111,7 @@ def test_more_tied_maps_than_workgroups(lig):
 
 
 def test_time_of_a_tied_map(golden_dir, lig):
-    """One tied map takes no more than ten times another (it is read six times more; one workgroup
+    """One tied map takes no more than ten times another (it is read twice more; one workgroup
     took seventy times as long)."""
     nf, t = 112, 64
     rec = M.Protein(os.path.join(golden_dir, "synth_r120.pdb"))

@@ -114,15 +114,13 @@ __global__ void __launch_bounds__(256) k_spec_finish(const double *__restrict__ 
     }
 }
 
-// Sums of a pose by parts of its atoms, out[b][7] = (s, ds/dt'(3), ds/dw(3)): one workgroup a pose goes
-// through the parts (one launch a call: with eight workgroups a pose, their partial sums and a
-// second kernel, in batches of the context's size, 2000 poses of 2081 atoms took 16 times two
-// copies in, two kernels (13 and 4 us) and a copy out); with `split`, few poses of a large ligand,
-// a workgroup takes one part and k_companion_finish adds them in the same order, so that a pose's
-// result does not depend on how many there are.
+// Sums of a pose, out[b][7] = (s, ds/dt'(3), ds/dw(3)), one workgroup a pose and one launch a call (with
+// eight workgroups a pose, their partial sums and a second kernel, in batches of the context's size, 2000
+// poses of 2081 atoms took 16 times two copies in, two kernels (13 and 4 us) and a copy out).  The atoms
+// of a large ligand go to a workgroup by parts, and k_companion_finish adds these in their order.
 __global__ void __launch_bounds__(256) k_companion(LigandDev L, const float *__restrict__ wshape,
                                                    const float2 *__restrict__ rg, const float *__restrict__ rot,
-                                                   const float *__restrict__ tq, int nf, int parts, bool split,
+                                                   const float *__restrict__ tq, int nf, int parts,
                                                    double *__restrict__ part, float *__restrict__ out) {
     const int b = blockIdx.x, tid = threadIdx.x;
     float r[9];
@@ -134,39 +132,35 @@ __global__ void __launch_bounds__(256) k_companion(LigandDev L, const float *__r
     }
     const int ng = L.ng, len = ((L.na + parts - 1) / parts + 255) / 256 * 256;
     const float gw = L.gw, h = 0.5f * ng - 0.5f;
-    double sum[7] = {0, 0, 0, 0, 0, 0, 0};
-    for (int p = split ? blockIdx.y : 0; p < parts; p += split ? parts : 1) {
-        double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-        for (int a = p * len + tid; a < min(L.na, (p + 1) * len); a += 256) {
-            const float x = L.xyz[3 * a] - L.cx, y = L.xyz[3 * a + 1] - L.cy, z = L.xyz[3 * a + 2] - L.cz;
-            const float X = r[0] * x + r[1] * y + r[2] * z;
-            const float Y = r[3] * x + r[4] * y + r[5] * z;
-            const float Z = r[6] * x + r[7] * y + r[8] * z;
-            const float Px = X - gw * t3[0], Py = Y - gw * t3[1], Pz = Z - gw * t3[2];
-            float2 val, dx, dy, dz;
-            trilinear(rg, ng, Px / gw + h, Py / gw + h, Pz / gw + h, val, dx, dy, dz);
-            const float ws = wshape[a], q = L.charge[a];
-            const float s = ws * val.x + q * val.y;
-            // g = ds/dP (per Angstrom)
-            const float gx = (ws * dx.x + q * dx.y) / gw, gy = (ws * dy.x + q * dy.y) / gw, gz = (ws * dz.x + q * dz.y) / gw;
-            acc[0] += s;
-            acc[1] += -gw * gx;
-            acc[2] += -gw * gy;
-            acc[3] += -gw * gz;
-            acc[4] += Y * gz - Z * gy;
-            acc[5] += Z * gx - X * gz;
-            acc[6] += X * gy - Y * gx;
-        }
-        block_sum<7, 256>(acc);
-        for (int a = 0; a < 7; a++) sum[a] += acc[a];
-        __syncthreads();  // the next part's sums
+    const int p = blockIdx.y;
+    double acc[7] = {0, 0, 0, 0, 0, 0, 0};
+    for (int a = p * len + tid; a < min(L.na, (p + 1) * len); a += 256) {
+        const float x = L.xyz[3 * a] - L.cx, y = L.xyz[3 * a + 1] - L.cy, z = L.xyz[3 * a + 2] - L.cz;
+        const float X = r[0] * x + r[1] * y + r[2] * z;
+        const float Y = r[3] * x + r[4] * y + r[5] * z;
+        const float Z = r[6] * x + r[7] * y + r[8] * z;
+        const float Px = X - gw * t3[0], Py = Y - gw * t3[1], Pz = Z - gw * t3[2];
+        float2 val, dx, dy, dz;
+        trilinear(rg, ng, Px / gw + h, Py / gw + h, Pz / gw + h, val, dx, dy, dz);
+        const float ws = wshape[a], q = L.charge[a];
+        const float s = ws * val.x + q * val.y;
+        // g = ds/dP (per Angstrom)
+        const float gx = (ws * dx.x + q * dx.y) / gw, gy = (ws * dy.x + q * dy.y) / gw, gz = (ws * dz.x + q * dz.y) / gw;
+        acc[0] += s;
+        acc[1] += -gw * gx;
+        acc[2] += -gw * gy;
+        acc[3] += -gw * gz;
+        acc[4] += Y * gz - Z * gy;
+        acc[5] += Z * gx - X * gz;
+        acc[6] += X * gy - Y * gx;
     }
+    block_sum<7, 256>(acc);
     if (tid == 0)
         for (int a = 0; a < 7; a++) {
-            if (split)
-                part[((size_t)b * parts + blockIdx.y) * 7 + a] = sum[a];
+            if (parts > 1)
+                part[((size_t)b * parts + p) * 7 + a] = acc[a];
             else
-                out[7 * (size_t)b + a] = (float)sum[a];
+                out[7 * (size_t)b + a] = (float)acc[a];
         }
 }
 
@@ -182,10 +176,11 @@ __global__ void k_companion_finish(const double *__restrict__ part, float *__res
 // one pose takes 28, 38, 48, 73 and 197 us with one workgroup and 336, 2081, 4000, 8000 and 30000
 // atoms, and 34, 36 and 43 us with the last three in parts.
 int companion_parts(int na) { return na < 2560 ? 1 : std::min(16, (na + 1023) / 1024); }
-// Poses up to which the parts go side by side, as many as there are compute units: 64 poses of 4000, 8000 and
-// 30000 atoms 49, 74, 204 -> 36, 43, 81 us, 256 poses 55, 87, 239 -> 52, 80, 211; 512 poses 80, 131, 382
-// with one workgroup each, 82, 133, 388 in parts.
-constexpr int kSplitPoses = 256;
+// Partial sums of one launch, and so poses times parts.  With side by side only as many poses as there are compute
+// units and one workgroup going through all parts above, 300 poses of 4000, 8000 and 30000 atoms (the last
+// at 256^3) took 65, 102 and 625 us, now 56, 86 and 418, 1000 poses 131, 223 and 1356 (131, 220, 1310); 10000 of
+// 2600 atoms 671, now 658.
+constexpr int kParts = 65536;
 
 }  // namespace
 
@@ -199,17 +194,17 @@ hipError_t launch_spec_finish(const double *part, int B, int n, int nf, float *o
     return hipGetLastError();
 }
 
-size_t companion_scratch_doubles(int na) {
-    const int parts = companion_parts(na);
-    return parts > 1 ? (size_t)kSplitPoses * parts * 7 : 0;
-}
+size_t companion_scratch_doubles(int na) { return companion_parts(na) > 1 ? (size_t)kParts * 7 : 0; }
 
 hipError_t launch_companion(const LigandDev &lig, const float *wshape, const float2 *recgrid, const float *rot_dev,
                             const float *t_dev, int B, int nf, double *part, float *out_dev, hipStream_t s) {
-    const int parts = companion_parts(lig.na);
-    const bool split = parts > 1 && B <= kSplitPoses;
-    k_companion<<<dim3(B, split ? parts : 1), 256, 0, s>>>(lig, wshape, recgrid, rot_dev, t_dev, nf, parts, split, part,
-                                                           out_dev);
-    if (split) k_companion_finish<<<(7 * B + 255) / 256, 256, 0, s>>>(part, out_dev, 7 * B, parts);
+    const int parts = companion_parts(lig.na), most = parts > 1 ? kParts / parts : B;
+    for (int b0 = 0; b0 < B; b0 += most) {
+        const int n = std::min(most, B - b0);
+        float *o = out_dev + 7 * (size_t)b0;
+        k_companion<<<dim3(n, parts), 256, 0, s>>>(lig, wshape, recgrid, rot_dev + 9 * (size_t)b0, t_dev + 3 * (size_t)b0, nf,
+                                                   parts, part, o);
+        if (parts > 1) k_companion_finish<<<(7 * n + 255) / 256, 256, 0, s>>>(part, o, 7 * n, parts);
+    }
     return hipGetLastError();
 }

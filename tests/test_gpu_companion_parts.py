@@ -1,6 +1,6 @@
-"""GPU: the companion score sums a large ligand in parts, one workgroup after another or, for few
-poses, side by side: both give the same bits, the values of the float64 companion, and one pose of
-a large ligand takes little more time than one of a small ligand."""
+"""GPU: the companion score sums a large ligand in parts, a workgroup each: a pose's bits do not depend
+on how many poses there are, its values are the float64 companion's, and one pose of a large
+ligand takes little more time than one of a small ligand."""
 import time
 
 import numpy as np
@@ -49,6 +49,15 @@ def test_few_poses_and_many(na):
         assert np.array_equal(c.score_companion(rot[:n], t[:n]).view(np.uint32), many[:n].view(np.uint32))
     c.close()
     assert np.isfinite(many).all()
+
+
+def test_more_poses_than_a_launch_takes():
+    c = _ctx(17000)  # 16 parts, 4096 poses
+    rot, t = _poses(8200)
+    many = c.score_companion(rot, t)
+    for a, b in ((4090, 4100), (8190, 8200), (4096, 8200)):
+        assert np.array_equal(c.score_companion(rot[a:b], t[a:b]).view(np.uint32), many[a:b].view(np.uint32))
+    c.close()
 
 
 @pytest.mark.parametrize("na", [2560, 5000])

@@ -964,9 +964,11 @@ int mdk_create(int device, int nf, int ng, int na, int t, int max_batch, mdk_ctx
                              dmalloc(&S.d_tkeys, B * topt_sort_size(t, nf))))
             return bail(1);
         S.vs = vox_scratch(S.d_bits, B, ng);
-        // the atom counts and the charge grids start, and are kept between batches, all-zero
+        // the atom counts, the charge grids and the select's histograms (among its keys, launch_topt) start,
+        // and are kept between batches, all-zero
         if (hipMemsetAsync(S.d_bits, 0, sizeof(uint32_t) * B * vox_scratch_words(ng), S.stream) != hipSuccess ||
             hipMemsetAsync(S.d_chg, 0, sizeof(float) * B * ng3, S.stream) != hipSuccess ||
+            (S.d_tkeys && hipMemsetAsync(S.d_tkeys, 0, sizeof(unsigned long long) * B * topt_sort_size(t, nf), S.stream) != hipSuccess) ||
             hipStreamSynchronize(S.stream) != hipSuccess)
             return bail(fail("mdk_create: scratch initialisation failed"));
     }

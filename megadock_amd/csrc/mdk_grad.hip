@@ -176,10 +176,10 @@ __global__ void k_companion_finish(const double *__restrict__ part, float *__res
 // one pose takes 28, 38, 48, 73 and 197 us with one workgroup and 336, 2081, 4000, 8000 and 30000
 // atoms, and 34, 36 and 43 us with the last three in parts.
 int companion_parts(int na) { return na < 2560 ? 1 : std::min(16, (na + 1023) / 1024); }
-// Partial sums of one launch, and so poses times parts.  With side by side only as many poses as there are compute
-// units and one workgroup going through all parts above, 300 poses of 4000, 8000 and 30000 atoms (the last
-// at 256^3) took 65, 102 and 625 us, now 56, 86 and 418, 1000 poses 131, 223 and 1356 (131, 220, 1310); 10000 of
-// 2600 atoms 671, now 658.
+// Partial sums of one launch, and so poses times parts.  With one workgroup going through all parts of a pose
+// instead, 300 poses of 4000, 8000 and 30000 atoms (the last at 256^3) take 65, 102 and 625 us in
+// place of 56, 86 and 418, 1000 poses 131, 223 and 1356 in place of 131, 220 and 1310, 10000 poses of 2600
+// atoms 671 in place of 658.
 constexpr int kParts = 65536;
 
 }  // namespace

@@ -95,7 +95,7 @@ struct TopTState {
 unsigned topt_sort_size(int t, int nf);
 // Top-t (t > MDK_MAXT) of B score maps smap[b][nf^3] (unnormalised real scores) into
 // out[(b0 + b) * t + q] as SortScore with rotation number rot_id[b0 + b], where b0 = *boff
-// (0 without boff); st: B states, keys: B * topt_sort_size(t, nf) words.
+// (0 without boff); st: B states, keys: B * topt_sort_size(t, nf) words, zero before the first call.
 hipError_t launch_topt(const float *smap, int B, int nf, int t, TopTState *st, unsigned long long *keys,
                        mdk_sortscore *out, const int *rot_id, const int *boff, hipStream_t s);
 

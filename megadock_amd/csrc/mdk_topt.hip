@@ -135,17 +135,14 @@ __global__ void __launch_bounds__(256) k_tsel_compact(const float *__restrict__ 
     }
 }
 
-// ---- wide select; a rotation's histogram lies at the start of its keys
-__global__ void __launch_bounds__(1024) k_wide_init(TopTState *st, unsigned long long *keys) {
-    unsigned *h = reinterpret_cast<unsigned *>(keys + (size_t)blockIdx.x * kTSortLds);
-    for (int q = threadIdx.x; q < kWideBuckets; q += 1024) h[q] = 0u;
-    if (threadIdx.x == 0) st[blockIdx.x].count = st[blockIdx.x].nover = 0u;
-}
-
+// ---- wide select; a rotation's histogram lies at the start of its keys and is zero between batches
+// (k_tsel_sort_out clears it: a launch of its own for that cost 2000 rotations of 64^3, t = 20, 0.1 of 5.1 ms)
 // grid (chunks, B); n3 is a multiple of 8 (nf is even)
-__global__ void __launch_bounds__(1024) k_wide_hist(const float *__restrict__ smap, unsigned n3, unsigned long long *keys) {
+__global__ void __launch_bounds__(1024) k_wide_hist(const float *__restrict__ smap, unsigned n3, TopTState *st,
+                                                    unsigned long long *keys) {
     __shared__ unsigned h[kWideBuckets];
     for (int q = threadIdx.x; q < kWideBuckets; q += 1024) h[q] = 0u;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) st[0].nover = 0u;
     __syncthreads();
     const float4 *m = reinterpret_cast<const float4 *>(smap + (size_t)blockIdx.y * n3);
     const unsigned i0 = blockIdx.x * (kWideChunk / 4), i1 = min(n3 / 4, i0 + kWideChunk / 4);
@@ -207,6 +204,7 @@ __global__ void __launch_bounds__(1024) k_wide_pick(TopTState *st, unsigned long
         TopTState &S = st[blockIdx.x];
         over = over || c > (unsigned)kTSortLds;
         S.prefix = cut_bits;
+        S.count = 0u;
         S.over = over;
         if (over) st[atomicAdd(&st[0].nover, 1u)].nth_over = blockIdx.x;
     }
@@ -434,7 +432,7 @@ __global__ void __launch_bounds__(kTieThreads) k_wide_ties(const float *__restri
 }
 
 // one workgroup per rotation: descending bitonic sort of its P keys (padded with 0, which
-// sorts last; P = 0: of its count rounded up to a power of two, at most kTSortLds), then the
+// sorts last; P = 0, wide select: of its count rounded up to a power of two, at most kTSortLds), then the
 // rotation's t results; a rotation's keys lie `stride` apart
 __global__ void __launch_bounds__(1024) k_tsel_sort_out(unsigned long long *keys, unsigned stride, unsigned P,
                                                         const TopTState *st, int t, int nf, mdk_sortscore *__restrict__ out,
@@ -443,12 +441,15 @@ __global__ void __launch_bounds__(1024) k_tsel_sort_out(unsigned long long *keys
     const int b = blockIdx.x;
     const unsigned n = st[b].count;
     unsigned long long *g = keys + (size_t)b * stride;
-    if (P == 0u)
+    const bool wide = P == 0u;
+    if (wide)
         for (P = 1u; P < n;) P <<= 1;
     const bool lds = P <= (unsigned)kTSortLds;
     unsigned long long *s = lds ? sl : g;
     for (unsigned i = threadIdx.x; i < P; i += 1024u) s[i] = i < n ? g[i] : 0ull;
     __syncthreads();
+    if (wide)  // the next batch's histogram
+        for (unsigned i = threadIdx.x; i < kWideBuckets / 2; i += 1024u) g[i] = 0ull;
     for (unsigned k = 2; k <= P; k <<= 1)
         for (unsigned j = k >> 1; j > 0; j >>= 1) {
             for (unsigned i = threadIdx.x; i < P; i += 1024u) {
@@ -504,8 +505,7 @@ hipError_t launch_topt(const float *smap, int B, int nf, int t, TopTState *st, u
     const unsigned P = topt_sort_size(t, nf);
     if (rank <= (unsigned)kWideT) {
         const dim3 wide((n3 + kWideChunk - 1) / kWideChunk, B);
-        k_wide_init<<<B, 1024, 0, s>>>(st, keys);
-        k_wide_hist<<<wide, 1024, 0, s>>>(smap, n3, keys);
+        k_wide_hist<<<wide, 1024, 0, s>>>(smap, n3, st, keys);
         k_wide_pick<<<B, 1024, 0, s>>>(st, keys, rank, nf3f);
         k_wide_compact<<<wide, 1024, 0, s>>>(smap, n3, nf3f, st, keys);
         k_wide_value<<<kTieBlocks, kTieThreads, 0, s>>>(smap, n3, nf3f, st, keys, rank);

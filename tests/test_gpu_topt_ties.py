@@ -97,6 +97,26 @@ def test_beside_other_maps(golden_dir, lig):
     assert 0 < tied < 15
 
 
+def test_batches_one_after_another(golden_dir, lig):
+    """A context docks tied maps, others and tied ones again, as many rotations or fewer each time."""
+    nf, t = 64, 40
+    rec = M.Protein(os.path.join(golden_dir, "synth_r120.pdb"))
+    grids, zero = M.receptor_grids(rec, nf // 2), (np.zeros((nf // 2) ** 3, np.float32),) * 2
+    rot = M.rotation_coefs(M.rotation_set(24)[:6])
+    c, want = _ctx(lig, nf, t, 6), {}
+    for tied in (False, True):
+        fresh = _ctx(lig, nf, t, 6)
+        fresh.set_receptor(*(zero if tied else grids))
+        want[tied] = fresh.dock(rot, np.arange(6, dtype=np.int32)).reshape(6, t)
+        fresh.close()
+    for tied, n in ((True, 6), (False, 6), (True, 2), (False, 4), (False, 6), (True, 6), (False, 1), (False, 6)):
+        print("tied=%d rotations=%d" % (tied, n), flush=True)
+        c.set_receptor(*(zero if tied else grids))
+        got = c.dock(rot[:n], np.arange(n, dtype=np.int32)).reshape(n, t)
+        assert np.array_equal(got, want[tied][:n])
+    c.close()
+
+
 def test_more_tied_maps_than_workgroups(lig):
     nf, t, n = 22, 20, 700
     c = _ctx(lig, nf, t, n)

@@ -32,11 +32,8 @@ struct RecAtoms {
     float gw;
 };
 
-// the voxel holding coordinate p along one axis (src/receptor.cpp:73-83); kept away from the ends of the
-// integers, where an infinite coordinate's box would wrap to a size above 0 far outside the arrays
-__device__ __forceinline__ int cell_of(float p, float gw, int ng) {
-    return min(max((int)(p / gw + ng / 2), -(1 << 24)), 1 << 24);
-}
+// the voxel holding coordinate p along one axis (src/receptor.cpp:73-83)
+__device__ __forceinline__ int cell_of(float p, float gw, int ng) { return (int)(p / gw + ng / 2); }
 
 __device__ __forceinline__ float sq_dist(float p, float g) {
     const float d = p - g;
@@ -62,7 +59,9 @@ __global__ void __launch_bounds__(128) k_rec_core(RecAtoms A, uint32_t *core, in
     int lo[3], n[3];
     const float p[3] = {x, y, z};
     for (int a = 0; a < 3; a++) {
-        const int c = cell_of(p[a], A.gw, ng);
+        // kept away from the ends of the integers, where an infinite coordinate's box would wrap to a size
+        // above 0 far outside the arrays
+        const int c = min(max(cell_of(p[a], A.gw, ng), -(1 << 24)), 1 << 24);
         lo[a] = max(c - range, 0);
         n[a] = max(min(c + range + 1, ng) - lo[a], 0);
     }
@@ -211,11 +210,13 @@ struct TileAtom {
     int lo[3], hi[3];
 };
 
+// (An infinite coordinate's box wraps to lo far above the grid or hi below it, so it meets no tile; a clamp
+// here, for every atom in every tile, cost the sums 8 of 479 us.)
 __device__ __forceinline__ void atom_box(const float *p, float gw, int ng, int range, int *lo, int *hi) {
     for (int a = 0; a < 3; a++) {
-        const int c = cell_of(p[a], gw, ng);
-        lo[a] = max(c - range, 0);
-        hi[a] = min(c + range + 1, ng);
+        const unsigned c = (unsigned)cell_of(p[a], gw, ng);
+        lo[a] = max((int)(c - (unsigned)range), 0);
+        hi[a] = min((int)(c + (unsigned)range + 1u), ng);
     }
 }
 
